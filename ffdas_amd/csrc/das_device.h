@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <type_traits>
 
@@ -104,14 +105,20 @@ __device__ __forceinline__ Radius radius_precise(const SplitPt &y, const SplitPt
     const float dcx = y.cx - p.cx, dcy = y.cy - p.cy, dcz = y.cz - p.cz;   // exact integers
     const float dfx = y.fx - p.fx, dfy = y.fy - p.fy, dfz = y.fz - p.fz;   // |.| <= 1
     R.dx = dcx + dfx; R.dy = dcy + dfy; R.dz = dcz + dfz;
-    const float lim = 32767.0f;
-    const bool big = __builtin_fabsf(dcx) > lim || __builtin_fabsf(dcy) > lim ||
-                     __builtin_fabsf(dcz) > lim;
-    // integer part of |d|^2, exact in 32 bits for |dc| <= 32767
-    const int ix = (int)__builtin_fminf(__builtin_fmaxf(dcx, -lim), lim);
-    const int iy = (int)__builtin_fminf(__builtin_fmaxf(dcy, -lim), lim);
-    const int iz = (int)__builtin_fminf(__builtin_fmaxf(dcz, -lim), lim);
-    const uint32_t I = (uint32_t)(ix * ix) + (uint32_t)(iy * iy) + (uint32_t)(iz * iz);
+    if (__builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(dcx), __builtin_fabsf(dcy)),
+                        __builtin_fabsf(dcz)) > 32767.0f) {
+        // far outside any imaging geometry: plain FP32
+        const float q = __builtin_fmaf(R.dx, R.dx, __builtin_fmaf(R.dy, R.dy, R.dz * R.dz));
+        R.rinv = __builtin_amdgcn_rsqf(q);
+        R.rh = q * R.rinv;
+        R.rl = 0.0f;
+        return R;
+    }
+    // integer part of |d|^2, exact in 32 bits; 24-bit multiplications, which run at the full
+    // rate (a 32-bit one takes four times as long)
+    const int ix = (int)dcx, iy = (int)dcy, iz = (int)dcz;
+    const uint32_t I = (uint32_t)__mul24(ix, ix) + (uint32_t)__mul24(iy, iy) +
+                       (uint32_t)__mul24(iz, iz);
     // remainder 2*dc*df + df^2 per axis
     const float F = __builtin_fmaf(dfx, __builtin_fmaf(2.0f, dcx, dfx),
                     __builtin_fmaf(dfy, __builtin_fmaf(2.0f, dcy, dfy),
@@ -126,17 +133,8 @@ __device__ __forceinline__ Radius radius_precise(const SplitPt &y, const SplitPt
     const float pl = __builtin_fmaf(r0, r0, -ph);
     float res = (Ih - ph);                         // exact (Sterbenz)
     res = (res - pl) + (Il + F);
-    float rl = res * (0.5f * R.rinv);
-    if (r2u < kRadiusSqMin || big) rl = 0.0f;
-    if (big) {  // far outside any imaging geometry: plain FP32
-        const float q = __builtin_fmaf(R.dx, R.dx, __builtin_fmaf(R.dy, R.dy, R.dz * R.dz));
-        R.rinv = __builtin_amdgcn_rsqf(q);
-        R.rh = q * R.rinv;
-        R.rl = 0.0f;
-        return R;
-    }
     R.rh = r0;
-    R.rl = rl;
+    R.rl = r2u < kRadiusSqMin ? 0.0f : res * (0.5f * R.rinv);
     return R;
 }
 
@@ -177,6 +175,36 @@ __device__ __forceinline__ Tap make_tap(float ofs, const Radius &R, float scale)
     }
     tp.k = (int)tp.kf;
     return tp;
+}
+
+// ---------------------------------------------------------------------------------------
+// delays in 32.32 fixed point
+// ---------------------------------------------------------------------------------------
+// tau = scale * ofs + scale * r is a sum of one term per (voxel, slot) and one per (voxel,
+// channel).  With both terms in 32.32 fixed point the sum of a tap is one 64-bit integer
+// addition whose high word is floor(tau) and whose low word is the fraction, where the
+// floating-point form needs about fifteen operations (TwoSum, scale, two floors) for each
+// tap.  The terms carry the compensated pairs to within 2^-31 of a sample, below the FP32
+// rounding of the fraction that follows either way.
+constexpr float kFixedLimit = 4194304.0f;      // |term| < 2^22: its low part fits 31 bits
+constexpr int kFixedNone = 0x40000000;         // high word of a term that selects no sample
+
+// h + l (|h| < 2^22, |l| <= ulp(h)) as 32.32 fixed point.
+__device__ __forceinline__ int64_t to_fixed(float h, float l) {
+#pragma clang fp contract(off)
+    const float f = __builtin_floorf(h);
+    const uint32_t lo = (uint32_t)((h - f) * 4294967296.0f);           // saturates at 2^32 - 1
+    const int li = (int)__builtin_rintf(l * 4294967296.0f);
+    return (((int64_t)(int)f << 32) | lo) + (int64_t)li;
+}
+
+// scale * (h + l) as a float pair; exact for scale == 1.
+__device__ __forceinline__ void scale_pair(float scale, float &h, float &l) {
+#pragma clang fp contract(off)
+    const float sh = scale * h;
+    const float sl = __builtin_fmaf(scale, h, -sh);
+    l = __builtin_fmaf(scale, l, sl);
+    h = sh;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -243,6 +271,16 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
     return (b & 7) * (full >> 3) + (b >> 3);
 }
 
+// The same in chunks of q tiles: each XCD still works on neighbouring tiles, but regions whose
+// tiles cost less (channels outside their cones are passed over) are shared out over all of
+// them.  The chunk an XCD takes moves on by one each round of 8, so that a period in the grid
+// does not give one XCD the cheap tiles every time.  A bijection on the complete rounds.
+__device__ __forceinline__ int xcd_chunk(int b, int nb, int q) {
+    const int round = b / (8 * q), i = b - round * 8 * q;
+    if ((round + 1) * 8 * q > nb) return b;
+    return round * 8 * q + ((i + round) & 7) * q + (i >> 3);
+}
+
 __device__ __forceinline__ int voxel_of(const Tiling &tl, int tile, int lane, bool &valid) {
     const int ntiles = tl.nta * tl.nth * tl.ntw;
     valid = tile < ntiles;
@@ -283,5 +321,52 @@ struct Geo {
     float wavenum;
 };
 
+// ---------------------------------------------------------------------------------------
+// pieces the kernel files share
+// ---------------------------------------------------------------------------------------
+template <bool ACC64> using AccT = typename std::conditional<ACC64, double, float>::type;
+
+__device__ __forceinline__ float fmaA(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fmaA(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// Raw buffer resources over the rows of a channel.
+constexpr int kBufWord3 = 0x00020000;          // raw buffer, 32-bit data format
+constexpr uint32_t kNoRows = 0x80000000u;      // beyond every channel block
+
+template <bool ACC64, bool CPLX, int FT>
+__device__ __forceinline__ void store_out(const AccT<ACC64> (&acc)[FT][CPLX ? 2 : 1], void *outv,
+                                          int64_t os_b, int n, int b0, int B, double beta_re,
+                                          double beta_im) {
+    using A = AccT<ACC64>;
+    constexpr int CW = CPLX ? 2 : 1;
+    A *out = static_cast<A *>(outv);
+    const bool zero_beta = beta_re == 0.0 && beta_im == 0.0;
+#pragma unroll
+    for (int f = 0; f < FT; f++) {
+        const int b = b0 + f;
+        if (b >= B) break;
+        A *o = out + ((int64_t)b * os_b + n) * CW;
+        if constexpr (!CPLX) {
+            o[0] = zero_beta ? acc[f][0] : (A)beta_re * o[0] + acc[f][0];
+        } else {
+            if (zero_beta) {
+                o[0] = acc[f][0];
+                o[1] = acc[f][1];
+            } else {
+                const A orr = o[0], oi = o[1];
+                o[0] = (A)beta_re * orr - (A)beta_im * oi + acc[f][0];
+                o[1] = (A)beta_re * oi + (A)beta_im * orr + acc[f][1];
+            }
+        }
+    }
+}
+
 }  // namespace dev
+
+// The forward for few frames in the natural layout (das_few.hip).
+bool few_frames_ok(const DasProblem &p, const XView &xv);
+hipError_t launch_forward_few(hipStream_t st, const dev::Geo &g, const dev::Tiling &tl,
+                              const DasProblem &p, const XView &xv, void *out, double beta_re,
+                              double beta_im);
+
 }  // namespace ffdas

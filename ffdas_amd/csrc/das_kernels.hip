@@ -26,11 +26,6 @@
 namespace ffdas {
 namespace dev {
 
-template <bool ACC64> using AccT = typename std::conditional<ACC64, double, float>::type;
-
-__device__ __forceinline__ float fmaA(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-__device__ __forceinline__ double fmaA(double a, double b, double c) { return __builtin_fma(a, b, c); }
-
 template <class D> __device__ __forceinline__ D convert_to(float v);
 template <> __device__ __forceinline__ float convert_to<float>(float v) { return v; }
 template <> __device__ __forceinline__ _Float16 convert_to<_Float16>(float v) { return (_Float16)v; }
@@ -96,9 +91,6 @@ struct NaturalRows {
 // (below 2^31 bytes, which the host checks): the group step is a scalar offset, and a tap
 // that reads nothing takes an offset past the block, for which the hardware returns zeros,
 // so the loads of a group of taps need no branch and no select of addresses.
-constexpr int kBufWord3 = 0x00020000;          // raw buffer, 32-bit data format
-constexpr uint32_t kNoRows = 0x80000000u;      // beyond every channel block
-
 template <int FT, int CW, int ESZ, bool PL>
 constexpr int fi_group() { return PL ? 8 / (CW * ESZ) : FT; }
 
@@ -365,34 +357,6 @@ __device__ __forceinline__ void das_fwd_body_fi(const Geo &g, const FrameInnerRo
                         }
                     }
                 }
-            }
-        }
-    }
-}
-
-template <bool ACC64, bool CPLX, int FT>
-__device__ __forceinline__ void store_out(const AccT<ACC64> (&acc)[FT][CPLX ? 2 : 1], void *outv,
-                                          int64_t os_b, int n, int b0, int B, double beta_re,
-                                          double beta_im) {
-    using A = AccT<ACC64>;
-    constexpr int CW = CPLX ? 2 : 1;
-    A *out = static_cast<A *>(outv);
-    const bool zero_beta = beta_re == 0.0 && beta_im == 0.0;
-#pragma unroll
-    for (int f = 0; f < FT; f++) {
-        const int b = b0 + f;
-        if (b >= B) break;
-        A *o = out + ((int64_t)b * os_b + n) * CW;
-        if constexpr (!CPLX) {
-            o[0] = zero_beta ? acc[f][0] : (A)beta_re * o[0] + acc[f][0];
-        } else {
-            if (zero_beta) {
-                o[0] = acc[f][0];
-                o[1] = acc[f][1];
-            } else {
-                const A orr = o[0], oi = o[1];
-                o[0] = (A)beta_re * orr - (A)beta_im * oi + acc[f][0];
-                o[1] = (A)beta_re * oi + (A)beta_im * orr + acc[f][1];
             }
         }
     }
@@ -2516,6 +2480,9 @@ ffdas_error_t launch_forward(ffdas_context &h, const DasProblem &p, const DasGeo
         }
         return hip_status(e, FFDAS_ERROR_CUDA_LAUNCH_FAILED);
     }
+if (few_frames_ok(p, xv))
+        return hip_status(launch_forward_few(st, g, tl, p, xv, out, beta_re, beta_im),
+                          FFDAS_ERROR_CUDA_LAUNCH_FAILED);
     if (!p.cplx) {
         switch (p.k_storage) {
             case Storage::F16: e = launch_fwd_t<Storage::F16, false, false>(st, g, tl, xv, out, os_b, beta_re, beta_im); break;
