@@ -1,11 +1,10 @@
 // Frequency-domain Green's function summation (ffdas_greens):
 //   out[b, t, f] = sum_s x[b, s, f] e^{i k_f r_ts} / r_ts,   r_ts = |dst_t - src_s|.
-// Fewer than 5 events (greens_kernel): one lane per target, its position and per-source
-// distance in registers; the source position and the x values of a (source, frequency
-// chunk, event chunk) are the same for the whole wave, so they come through the scalar unit;
-// each thread keeps FPT frequencies x BT events of complex sums on the VALU.  5 or more
-// events (greens_mfma_kernel): the sums on the MFMA, see there.  FP32 throughout (the input
-// may be stored as FP16).
+// One event (greens_kernel): one lane per target, its position and per-source distance in
+// registers; the source position and the x values of a (source, frequency chunk) are the same
+// for the whole wave, so they come through the scalar unit; each thread keeps FPT complex sums
+// on the VALU.  More events (greens_mfma_kernel): the sums on the MFMA, see there.  FP32
+// throughout (the input may be stored as FP16).
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 
@@ -25,17 +24,16 @@ __device__ __forceinline__ float2 load_x<float2>(const float2 *p) { return *p; }
 template <>
 __device__ __forceinline__ float2 load_x<__half2>(const __half2 *p) { return __half22float2(*p); }
 
-template <typename XT, int BT>
+template <typename XT>
 __global__ __launch_bounds__(256) void greens_kernel(const float *__restrict__ src,
                                                      const float *__restrict__ wav,
                                                      const XT *__restrict__ x,
                                                      const float *__restrict__ dst,
                                                      float2 *__restrict__ out, int nsrc, int nfreq,
-                                                     int ndst, int B) {
+                                                     int ndst) {
     const int t = blockIdx.x * 256 + threadIdx.x;
     const int f0 = blockIdx.y * kGreensFPT;
-    const int b0 = blockIdx.z * BT;
-    const int nf = min(kGreensFPT, nfreq - f0), nb = min(BT, B - b0);
+    const int nf = min(kGreensFPT, nfreq - f0);
     const bool valid = t < ndst;
     float px = 0, py = 0, pz = 0;
     if (valid) {
@@ -46,11 +44,9 @@ __global__ __launch_bounds__(256) void greens_kernel(const float *__restrict__ s
     float k[kGreensFPT];
 #pragma unroll
     for (int f = 0; f < kGreensFPT; f++) k[f] = f < nf ? wav[f0 + f] : 0.0f;
-    float ar[kGreensFPT][BT], ai[kGreensFPT][BT];
+    float ar[kGreensFPT], ai[kGreensFPT];
 #pragma unroll
-    for (int f = 0; f < kGreensFPT; f++)
-#pragma unroll
-        for (int b = 0; b < BT; b++) ar[f][b] = ai[f][b] = 0.0f;
+    for (int f = 0; f < kGreensFPT; f++) ar[f] = ai[f] = 0.0f;
 
     for (int s = 0; s < nsrc; s++) {
         // r = rsq * rsqrt(rsq), as the reference (greens_kernels.cuh:59-61)
@@ -58,58 +54,79 @@ __global__ __launch_bounds__(256) void greens_kernel(const float *__restrict__ s
         const float rsq = dx * dx + dy * dy + dz * dz;
         const float rinv = rsqrtf(rsq);
         const float r = rsq * rinv;
-        const XT *xs = x + ((int64_t)b0 * nsrc + s) * nfreq + f0;
+        const XT *xs = x + (int64_t)s * nfreq + f0;
 #pragma unroll
         for (int f = 0; f < kGreensFPT; f++) {
             if (f < nf) {
                 float sn, cs;
                 __sincosf(k[f] * r, &sn, &cs);
                 const float gr = cs * rinv, gi = sn * rinv;
-#pragma unroll
-                for (int b = 0; b < BT; b++) {
-                    if (b < nb) {
-                        const float2 v = load_x<XT>(xs + (int64_t)b * nsrc * nfreq + f);
-                        ar[f][b] += gr * v.x - gi * v.y;
-                        ai[f][b] += gr * v.y + gi * v.x;
-                    }
-                }
+                const float2 v = load_x<XT>(xs + f);
+                ar[f] += gr * v.x - gi * v.y;
+                ai[f] += gr * v.y + gi * v.x;
             }
         }
     }
     if (!valid) return;
+    float2 *o = out + (int64_t)t * nfreq + f0;
 #pragma unroll
-    for (int b = 0; b < BT; b++) {
-        if (b >= nb) break;
-        float2 *o = out + ((int64_t)(b0 + b) * ndst + t) * nfreq + f0;
-#pragma unroll
-        for (int f = 0; f < kGreensFPT; f++)
-            if (f < nf) o[f] = float2{ar[f][b], ai[f][b]};
-    }
+    for (int f = 0; f < kGreensFPT; f++)
+        if (f < nf) o[f] = float2{ar[f], ai[f]};
 }
 
-// Many events: the multiply-adds on the MFMA.  Per wave a 16-target x 16-event tile of
-// kGreensFPW frequencies; per step of 4 sources, lane (jl, g) = (lane % 16, lane / 16)
-// generates the Green's function of target t0 + jl and source s0 + g (the A operand of
-// v_mfma_f32_16x16x4f32) and loads x of event b0 + jl, source s0 + g (the B operand); the
-// complex product is four real MFMAs (A_r B_r - A_i B_i, A_r B_i + A_i B_r).  Output register
-// v of lane (jl, g) holds target t0 + 4 g + v, event b0 + jl.  One sincos per (target,
-// source, frequency) is all the VALU does per term.
+// More events: the multiply-adds on the MFMA, as a real product.  A wave has a tile of 16
+// targets x 8 events x 8 frequencies (NT = 2: two such tiles, 16 events); the 16 columns of a
+// tile are the real parts of its events, then the imaginary parts.  Per step of 4 sources, lane
+// (jl, g) = (lane % 16, lane / 16) generates the Green's function of target t0 + jl and source
+// s0 + g (the A operand of v_mfma_f32_16x16x4f32); column (b, re) sums gr xr - gi xi and column
+// (b, im) gr xi + gi xr, so a tile takes two MFMAs a step into one accumulator.  Output register
+// v of lane (jl, g) holds target t0 + 4 g + v.
+//
+// The workgroup's four waves (64 targets) read the same x, which is staged in LDS for 8 sources
+// at a time, two buffers in turn, as the B operands themselves: X1 = (xr | xi) for the real
+// part of the Green's function and X2 = (-xi | xr) for its imaginary part, four frequencies of a
+// column contiguous (one 16-byte read, consecutive lanes on consecutive banks).
+//
+// Bound by the MFMA pipe (64 cycles a step and frequency) and by one sincos per (target,
+// source, frequency) on the VALU beside it (about 56 cycles).  128 sources to 256 x 128 targets,
+// 512 frequencies, 8 events: 3.24 ms with 16 complex columns a tile (half of them idle, four
+// MFMAs a step), 2.02 ms with the real columns and x read from memory by every wave (the vector
+// L1 at its access rate), 1.81 ms with x staged, 1.60 ms with the MFMAs of a step in one run,
+// 1.51 ms at five waves per SIMD (91 TFLOP/s of the sums' multiply-adds).
 constexpr int kGreensFPW = 8;
-
+constexpr int kGreensSrc = 8;                                         // sources staged at a time
 typedef float GV4 __attribute__((ext_vector_type(4)));
+typedef float GV4p __attribute__((ext_vector_type(4), aligned(8)));   // two packed float2
 
-template <typename XT>
-__global__ __launch_bounds__(256) void greens_mfma_kernel(const float *__restrict__ src,
+// the two values of x from p; complex values lie on 8-byte (FP16: 4-byte) boundaries
+__device__ __forceinline__ void load_two(const float2 *p, float2 (&v)[2]) {
+    const GV4p q = *reinterpret_cast<const GV4p *>(p);
+    v[0] = float2{q[0], q[1]};
+    v[1] = float2{q[2], q[3]};
+}
+__device__ __forceinline__ void load_two(const __half2 *p, float2 (&v)[2]) {
+    v[0] = __half22float2(p[0]);
+    v[1] = __half22float2(p[1]);
+}
+
+template <typename XT, int NT>
+__global__ __launch_bounds__(256, NT == 1 ? 5 : 3) void greens_mfma_kernel(const float *__restrict__ src,
                                                           const float *__restrict__ wav,
                                                           const XT *__restrict__ x,
                                                           const float *__restrict__ dst,
                                                           float2 *__restrict__ out, int nsrc,
                                                           int nfreq, int ndst, int B) {
+    constexpr int FPW = kGreensFPW, SC = kGreensSrc;
+    // [buffer][operand][source][half of the frequencies][tile, column]
+    __shared__ GV4 xs[2][2][SC][2][16 * NT];
+    __shared__ GV4 sp[2][SC];                // source positions
     const int lane = threadIdx.x & 63, jl = lane & 15, g = lane >> 4;
     const int t0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 16;
-    const int f0 = blockIdx.y * kGreensFPW;
-    const int b0 = blockIdx.z * 16;
-    const int nf = min(kGreensFPW, nfreq - f0);
+    const int f0 = blockIdx.y * FPW;
+    const int b0 = blockIdx.z * (8 * NT);
+    const int nf = min(FPW, nfreq - f0);
+    const bool whole = nf == FPW;            // uniform
+    const bool im = jl >= 8;                 // this lane's column is an imaginary part
     const int ta = t0 + jl;                  // this lane's target in the A operand
     const bool tok = ta < ndst;
     float px = 0, py = 0, pz = 0;
@@ -118,84 +135,166 @@ __global__ __launch_bounds__(256) void greens_mfma_kernel(const float *__restric
         py = dst[3 * (int64_t)ta + 1];
         pz = dst[3 * (int64_t)ta + 2];
     }
-    const int be = b0 + jl;                  // this lane's event in the B operand
-    const bool bok = be < B;
-    float k[kGreensFPW];
+    int be[NT];                              // this lane's event in each tile
 #pragma unroll
-    for (int f = 0; f < kGreensFPW; f++) k[f] = f < nf ? wav[f0 + f] : 0.0f;
-    GV4 cr[kGreensFPW], ci[kGreensFPW];
+    for (int n = 0; n < NT; n++) be[n] = b0 + 8 * n + (jl & 7);
+    float k[FPW];
 #pragma unroll
-    for (int f = 0; f < kGreensFPW; f++) {
-        cr[f] = GV4{0.0f, 0.0f, 0.0f, 0.0f};
-        ci[f] = GV4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
-    for (int s0 = 0; s0 < nsrc; s0 += 4) {
-        const int s = s0 + g;
-        const bool sok = s < nsrc;
-        const bool aok = tok && sok;
-        float rinv = 0.0f, r = 0.0f;
-        if (aok) {
-            const float dx = px - src[3 * s], dy = py - src[3 * s + 1], dz = pz - src[3 * s + 2];
+    for (int f = 0; f < FPW; f++) k[f] = f < nf ? wav[f0 + f] : 0.0f;
+    GV4 c[NT][FPW];
+#pragma unroll
+    for (int n = 0; n < NT; n++)
+#pragma unroll
+        for (int f = 0; f < FPW; f++) c[n][f] = GV4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    // staging: a thread takes frequencies 2 p, 2 p + 1 of event e, source sl (NT of them)
+    const int p = threadIdx.x & 3, e = (threadIdx.x >> 2) & 7, sl = threadIdx.x >> 5;
+    float2 v[NT][2];
+    GV4 pos{0.0f, 0.0f, 0.0f, 0.0f};
+    auto fetch = [&](int s0) {
+        const int s = s0 + sl;
+#pragma unroll
+        for (int n = 0; n < NT; n++) {
+            const int b = b0 + 8 * n + e;
+            const XT *xp = x + ((int64_t)b * nsrc + s) * nfreq + f0 + 2 * p;
+            if (whole && b < B && s < nsrc) {
+                load_two(xp, v[n]);
+            } else {
+#pragma unroll
+                for (int f = 0; f < 2; f++)
+                    v[n][f] = b < B && s < nsrc && 2 * p + f < nf ? load_x<XT>(xp + f)
+                                                                  : float2{0.0f, 0.0f};
+            }
+        }
+        if (threadIdx.x < SC && nsrc > 0) {
+            const int q = min(s0 + (int)threadIdx.x, nsrc - 1);
+            pos = GV4{src[3 * q], src[3 * q + 1], src[3 * q + 2], 0.0f};
+        }
+    };
+    auto put = [&](GV4 &at, float a, float b) {
+        reinterpret_cast<float2 *>(&at)[p & 1] = float2{a, b};
+    };
+    auto stage = [&](int buf) {
+#pragma unroll
+        for (int n = 0; n < NT; n++) {
+            GV4 *o1 = xs[buf][0][sl][p >> 1] + 16 * n + e, *o2 = xs[buf][1][sl][p >> 1] + 16 * n + e;
+            put(o1[0], v[n][0].x, v[n][1].x);
+            put(o1[8], v[n][0].y, v[n][1].y);
+            put(o2[0], -v[n][0].y, -v[n][1].y);
+            put(o2[8], v[n][0].x, v[n][1].x);
+        }
+        if (threadIdx.x < SC) sp[buf][threadIdx.x] = pos;
+    };
+    fetch(0);
+    stage(0);
+    __syncthreads();
+    for (int s0 = 0, buf = 0; s0 < nsrc; s0 += SC, buf ^= 1) {
+        const bool more = s0 + SC < nsrc;     // uniform
+        if (more) fetch(s0 + SC);
+#pragma unroll
+        for (int q = 0; q < SC; q += 4) {     // sources past the last: zero x and zero g
+            const GV4 ps = sp[buf][q + g];
+            const float dx = px - ps[0], dy = py - ps[1], dz = pz - ps[2];
             const float rsq = dx * dx + dy * dy + dz * dz;
-            rinv = rsqrtf(rsq);
-            r = rsq * rinv;
-        }
-        const XT *xs = x + ((int64_t)(bok ? be : 0) * nsrc + (sok ? s : 0)) * nfreq + f0;
-        const bool xok = bok && sok;
+            const bool ok = tok && s0 + q + g < nsrc;
+            const float ri = rsqrtf(rsq);
+            const float rinv = ok ? ri : 0.0f, r = ok ? rsq * ri : 0.0f;
+            GV4 x1[NT][2], x2[NT][2];
 #pragma unroll
-        for (int f = 0; f < kGreensFPW; f++) {
-            float sn, cs;
-            __sincosf(k[f] * r, &sn, &cs);
-            const float ar = aok ? cs * rinv : 0.0f, ai = aok ? sn * rinv : 0.0f;
-            const float2 v = (xok && f < nf) ? load_x<XT>(xs + f) : float2{0.0f, 0.0f};
-            cr[f] = __builtin_amdgcn_mfma_f32_16x16x4f32(ar, v.x, cr[f], 0, 0, 0);
-            cr[f] = __builtin_amdgcn_mfma_f32_16x16x4f32(-ai, v.y, cr[f], 0, 0, 0);
-            ci[f] = __builtin_amdgcn_mfma_f32_16x16x4f32(ar, v.y, ci[f], 0, 0, 0);
-            ci[f] = __builtin_amdgcn_mfma_f32_16x16x4f32(ai, v.x, ci[f], 0, 0, 0);
+            for (int n = 0; n < NT; n++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    x1[n][h] = xs[buf][0][q + g][h][16 * n + jl];
+                    x2[n][h] = xs[buf][1][q + g][h][16 * n + jl];
+                }
+            // all sincos of the step, then all its MFMAs: one wave's run of MFMAs leaves the
+            // VALU to the others (term by term both pipes wait: 1.81 ms against 1.60)
+            float ar[FPW], ai[FPW];
+#pragma unroll
+            for (int f = 0; f < FPW; f++) {
+                float sn, cs;
+                __sincosf(k[f] * r, &sn, &cs);
+                ar[f] = cs * rinv;
+                ai[f] = sn * rinv;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int n = 0; n < NT; n++)
+#pragma unroll
+                for (int f = 0; f < FPW; f++)
+                    c[n][f] = __builtin_amdgcn_mfma_f32_16x16x4f32(ar[f], x1[n][f / 4][f & 3],
+                                                                   c[n][f], 0, 0, 0);
+#pragma unroll
+            for (int n = 0; n < NT; n++)
+#pragma unroll
+                for (int f = 0; f < FPW; f++)
+                    c[n][f] = __builtin_amdgcn_mfma_f32_16x16x4f32(ai[f], x2[n][f / 4][f & 3],
+                                                                   c[n][f], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
+        // the other buffer was last read before the previous barrier
+        if (more) stage(buf ^ 1);
+        __syncthreads();
     }
-    if (!bok) return;
+
+    // Lanes jl and jl ^ 8 hold the real and imaginary parts of an event: the first takes the
+    // lower half of the frequencies, the second the upper half, and each gets the other's part
+    // of its half (a rotation by 8 within the row of 16 lanes), so that each lane writes one
+    // contiguous run of complex values.
+    constexpr int H = FPW / 2;
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
-        const int t = t0 + 4 * g + v;
-        if (t >= ndst) continue;
-        float2 *o = out + ((int64_t)be * ndst + t) * nfreq + f0;
+    for (int n = 0; n < NT; n++) {
 #pragma unroll
-        for (int f = 0; f < kGreensFPW; f++)
-            if (f < nf) o[f] = float2{cr[f][v], ci[f][v]};
+        for (int v = 0; v < 4; v++) {
+            float2 o[H];
+#pragma unroll
+            for (int f = 0; f < H; f++) {
+                const float give = im ? c[n][f][v] : c[n][f + H][v];
+                const float got = __int_as_float(__builtin_amdgcn_update_dpp(
+                    0, __float_as_int(give), 0x128, 0xf, 0xf, false));      // row_ror:8
+                o[f] = im ? float2{got, c[n][f + H][v]} : float2{c[n][f][v], got};
+            }
+            const int t = t0 + 4 * g + v;
+            if (t >= ndst || be[n] >= B) continue;
+            const int fo = im ? H : 0;
+            float2 *po = out + ((int64_t)be[n] * ndst + t) * nfreq + f0 + fo;
+            if (whole) {
+#pragma unroll
+                for (int f = 0; f < H; f += 2)
+                    *reinterpret_cast<GV4p *>(po + f) = GV4p{o[f].x, o[f].y, o[f + 1].x, o[f + 1].y};
+            } else {
+#pragma unroll
+                for (int f = 0; f < H; f++)
+                    if (fo + f < nf) po[f] = o[f];
+            }
+        }
     }
 }
 
 template <typename XT>
 ffdas_error_t launch(hipStream_t st, const float *src, const float *wav, const void *x,
                      const float *dst, void *out, int nsrc, int nfreq, int ndst, int B) {
-    // each (target, source, frequency) sincos once where it pays (measured): the MFMA tile
-    // from 5 events (one 16-event tile instead of two VALU passes), the 4-event VALU kernel
-    // for 2-4, the 1-event one for 1
-    if (B >= 5) {
-        const dim3 g((unsigned)((ndst + 63) / 64), (unsigned)((nfreq + kGreensFPW - 1) / kGreensFPW),
-                     (unsigned)((B + 15) / 16));
+    if (B == 1) {
+        // one column pair of the 8-event tile would be in use: for the geometry above 0.84 ms
+        // on the VALU and 1.5 ms on the MFMA, which 2 events take too (on the VALU 1.79)
+        const dim3 grid((unsigned)((ndst + 255) / 256),
+                        (unsigned)((nfreq + kGreensFPT - 1) / kGreensFPT), 1);
         ProfScope ps(st, "greens");
-        hipLaunchKernelGGL((greens_mfma_kernel<XT>), g, dim3(256), 0, st, src, wav,
+        hipLaunchKernelGGL((greens_kernel<XT>), grid, dim3(256), 0, st, src, wav,
                            static_cast<const XT *>(x), dst, static_cast<float2 *>(out), nsrc,
-                           nfreq, ndst, B);
+                           nfreq, ndst);
         return hip_status(hipGetLastError(), FFDAS_ERROR_CUDA_LAUNCH_FAILED);
     }
-    const dim3 grid((unsigned)((ndst + 255) / 256), (unsigned)((nfreq + kGreensFPT - 1) / kGreensFPT),
-                    1);
+    const int events = B <= 8 ? 8 : 16;
+    const dim3 g((unsigned)((ndst + 63) / 64), (unsigned)((nfreq + kGreensFPW - 1) / kGreensFPW),
+                 (unsigned)((B + events - 1) / events));
     ProfScope ps(st, "greens");
-    if (B >= 2) {
-        const dim3 g(grid.x, grid.y, (unsigned)((B + 3) / 4));
-        hipLaunchKernelGGL((greens_kernel<XT, 4>), g, dim3(256), 0, st, src, wav,
-                           static_cast<const XT *>(x), dst, static_cast<float2 *>(out), nsrc,
-                           nfreq, ndst, B);
-    } else {
-        const dim3 g(grid.x, grid.y, (unsigned)B);
-        hipLaunchKernelGGL((greens_kernel<XT, 1>), g, dim3(256), 0, st, src, wav,
-                           static_cast<const XT *>(x), dst, static_cast<float2 *>(out), nsrc,
-                           nfreq, ndst, B);
-    }
-    return hip_status(hipGetLastError(), FFDAS_ERROR_CUDA_LAUNCH_FAILED);
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, g, dim3(256), 0, st, src, wav, static_cast<const XT *>(x), dst,
+                           static_cast<float2 *>(out), nsrc, nfreq, ndst, B);
+        return hip_status(hipGetLastError(), FFDAS_ERROR_CUDA_LAUNCH_FAILED);
+    };
+    return events == 8 ? go(greens_mfma_kernel<XT, 1>) : go(greens_mfma_kernel<XT, 2>);
 }
 
 bool packed(const ffdas_tensor_desc &d) {
