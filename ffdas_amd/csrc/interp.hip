@@ -1,19 +1,18 @@
 // Interpolation from a structured grid with arbitrary vertex positions to scattered points
 // (ffdas_create_interpolation_plan / _preprocess / ffdas_interpolation / _destroy).
 //
-// Plan (once per grid): the grid's bounding box (per-block partial min/max, finished on the
-// host), 128 bins per axis over it, every tetrahedron counted into each bin of its quantised
-// bounding box (atomics), a device scan of the counts, and a fill of the per-bin lists.  The
-// list order inside a bin is whatever the atomics give: the query takes the lowest passing
-// tetrahedron id of the whole bin, which is the reference's answer (its lists are sorted by
-// id and it returns the first that passes) without sorting anything.
-// Query (once per point set): per point, its bin and the FP32 barycentric test of each
-// candidate, computed without contraction in the reference's operation order; the result is
-// four vertex ids and weights (linear) or one vertex id (nearest).
+// Plan (once per grid): the vertices as 16-byte vectors, the grid's bounding box and the scale of
+// the 128 bins per axis over it (one pass over the vertices, finished on the device).
+// Query (once per point set): the points are ordered by bin, and every grid cell tests the points
+// in the bins of its quantised bounding box; per point, the lowest tetrahedron id whose FP32
+// barycentric test passes (computed without contraction in the reference's operation order) and
+// whose own quantised box holds the point's bin, which is the first of the reference's sorted
+// list of that bin.  The lookup of a point is that tetrahedron's key and three weights (linear)
+// or one vertex id (nearest).
 // Evaluation (per call, the per-frame part): x is first copied frame-inner (the frames of a
-// chunk, 16 for 4-byte data and 8 otherwise, contiguous per vertex), so one thread per query
-// point fetches each of its vertices' chunk with one vector load; its lookup is read once per
-// chunk; out is packed.
+// chunk, up to 16 for 4-byte data and 8 otherwise, contiguous per vertex; one frame is read as it
+// is), so one thread per query point fetches each of its vertices' chunk with one vector load;
+// its lookup is read once per chunk; out is packed.
 #include <hip/hip_runtime.h>
 
 #include <cstring>   // before rocPRIM, whose iterators use memset
@@ -25,6 +24,7 @@
 #include <climits>
 #include <cmath>
 #include <cstdlib>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -34,17 +34,19 @@ struct ffdas_interpolation_plan {
     int device = 0;
     int64_t nx = 0, ny = 0, nz = 0;
     int mode = FFDAS_INTERP_LINEAR;
-    float *verts = nullptr;            // 3 * nx * ny * nz
-    float4 *verts4 = nullptr;          // the same, one 16-byte vector per vertex (location)
+    float4 *verts = nullptr;           // nx * ny * nz, one 16-byte vector per vertex
     float bmin[3] = {0, 0, 0}, scale[3] = {0, 0, 0};
     int64_t ntet = 0;
+    long long list_total = 0;          // entries of the bin lists
+    // per-bin lists of tetrahedra, built when the point-by-point location first needs them
+    std::mutex list_mutex;
     long long *bin_start = nullptr;    // kBins^3 + 1
     int *bin_list = nullptr;
     // preprocessed query points
     bool pre = false;
     int64_t pre_n = 0;
-    int *pre_idx = nullptr;            // nearest: n ids; linear: 4 n ids
-    float *pre_w = nullptr;            // linear: 4 n weights
+    int *pre_idx = nullptr;            // n vertex ids (nearest) or tetrahedron keys (linear)
+    float *pre_w = nullptr;            // linear: 3 n weights
 };
 
 namespace ffdas {
@@ -56,45 +58,45 @@ constexpr int64_t kBins3 = (int64_t)kBins * kBins * kBins;
 // the six tetrahedra of a cell as corner codes (bit 0: +x, bit 1: +y, bit 2: +z), in the
 // reference's order (src/interpolation/spatial_hash_kernels.cuh:183-190): the split fixes
 // which vertices a point is interpolated from
-__constant__ unsigned char kTet[6][4] = {{0, 1, 2, 4}, {1, 3, 2, 7}, {1, 2, 4, 7},
-                                         {2, 4, 6, 7}, {1, 4, 5, 7}, {4, 6, 5, 7}};
+constexpr int kTet[6][4] = {{0, 1, 2, 4}, {1, 3, 2, 7}, {1, 2, 4, 7},
+                            {2, 4, 6, 7}, {1, 4, 5, 7}, {4, 6, 5, 7}};
 
-__device__ __forceinline__ int4 tet_vertices(long long tid, int nx, int ny) {
-    const long long cell = tid / 6;
-    const int t = (int)(tid - cell * 6);
-    const long long cx = cell % (nx - 1), cy = (cell / (nx - 1)) % (ny - 1),
-                    cz = cell / ((long long)(nx - 1) * (ny - 1));
-    const long long base = cx + cy * nx + cz * (long long)ny * nx;
-    int v[4];
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-        const int code = kTet[t][c];
-        v[c] = (int)(base + (code & 1) + ((code >> 1) & 1) * nx + ((code >> 2) & 1) * (long long)ny * nx);
-    }
-    return int4{v[0], v[1], v[2], v[3]};
+constexpr unsigned tet_codes(int t) {
+    return kTet[t][0] | kTet[t][1] << 3 | kTet[t][2] << 6 | kTet[t][3] << 9;
 }
 
-// A tetrahedron in the bin lists: key = base vertex * 8 + t, base = cx + cy nx + cz ny nx of
-// its cell.  Keys order exactly as the ids cell * 6 + t do (cells in (cz, cy, cx) order, then
-// t), so the lowest passing id is the lowest passing key, and the vertices follow from the
-// key without divisions.
+// the corner codes of tetrahedron t, three bits each, without a table in memory
+__device__ __forceinline__ unsigned corner_codes(int t) {
+    constexpr uint64_t first = (uint64_t)tet_codes(0) | (uint64_t)tet_codes(1) << 12 |
+                               (uint64_t)tet_codes(2) << 24 | (uint64_t)tet_codes(3) << 36 |
+                               (uint64_t)tet_codes(4) << 48;
+    return t == 5 ? tet_codes(5) : (unsigned)(first >> (12 * t)) & 0xfffu;
+}
+
+// Vertex id of corner `code` of the cell at base vertex `base`.
+__device__ __forceinline__ int corner(int base, int code, int nx, int ny) {
+    return base + (code & 1) + ((code >> 1) & 1) * nx + ((code >> 2) & 1) * ny * nx;
+}
+
+// A tetrahedron: key = base vertex * 8 + t, base = cx + cy nx + cz ny nx of its cell.  Keys
+// order exactly as the ids cell * 6 + t do (cells in (cz, cy, cx) order, then t), so the lowest
+// passing id is the lowest passing key, and the vertices follow from the key without divisions.
+__device__ __forceinline__ int cell_base(unsigned cell, int nx, int ny) {
+    const unsigned row = cell / (unsigned)(nx - 1), cx = cell - row * (unsigned)(nx - 1);
+    const unsigned cz = row / (unsigned)(ny - 1), cy = row - cz * (unsigned)(ny - 1);
+    return (int)(cx + (cy + cz * (unsigned)ny) * (unsigned)nx);
+}
+
 __device__ __forceinline__ int tet_key(long long tid, int nx, int ny) {
-    const long long cell = tid / 6;
-    const int t = (int)(tid - cell * 6);
-    const long long cx = cell % (nx - 1), cy = (cell / (nx - 1)) % (ny - 1),
-                    cz = cell / ((long long)(nx - 1) * (ny - 1));
-    return (int)((cx + cy * nx + cz * (long long)ny * nx) * 8 + t);
+    const unsigned cell = (unsigned)(tid / 6);
+    return cell_base(cell, nx, ny) * 8 + (int)(tid - (long long)cell * 6);
 }
 
 __device__ __forceinline__ int4 key_vertices(int key, int nx, int ny) {
-    const int base = key >> 3, t = key & 7;
-    int v[4];
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-        const int code = kTet[t][c];
-        v[c] = base + (code & 1) + ((code >> 1) & 1) * nx + ((code >> 2) & 1) * ny * nx;
-    }
-    return int4{v[0], v[1], v[2], v[3]};
+    const int base = key >> 3;
+    const unsigned c = corner_codes(key & 7);
+    return int4{corner(base, c & 7, nx, ny), corner(base, (c >> 3) & 7, nx, ny),
+                corner(base, (c >> 6) & 7, nx, ny), corner(base, c >> 9, nx, ny)};
 }
 
 struct Box {
@@ -120,15 +122,24 @@ __device__ __forceinline__ bool quantize(const Box &b, float x, float y, float z
     return true;
 }
 
-__global__ __launch_bounds__(256) void interp_bbox_kernel(const float *__restrict__ v, int64_t n,
-                                                          float *__restrict__ part) {
+// What the plan needs on the host: the box and the number of entries the bin lists would have.
+struct PlanHead {
+    Box box;
+    unsigned long long total;
+};
+
+// The vertices into 16-byte vectors, and the minima and maxima of each block's part.
+__global__ __launch_bounds__(256) void interp_verts_kernel(const float *__restrict__ v, int64_t n,
+                                                           float4 *__restrict__ v4,
+                                                           float *__restrict__ part) {
     float mn[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, mx[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        const float p[3] = {v[3 * i], v[3 * i + 1], v[3 * i + 2]};
+        v4[i] = float4{p[0], p[1], p[2], 0.f};
 #pragma unroll
         for (int a = 0; a < 3; a++) {
-            const float x = v[3 * i + a];
-            mn[a] = fminf(mn[a], x);
-            mx[a] = fmaxf(mx[a], x);
+            mn[a] = fminf(mn[a], p[a]);
+            mx[a] = fmaxf(mx[a], p[a]);
         }
     }
     __shared__ float red[6][4];
@@ -156,61 +167,126 @@ __global__ __launch_bounds__(256) void interp_bbox_kernel(const float *__restric
     }
 }
 
+// The box and the bins' scale, in FP32 as the reference (spatial_hash.cu:51-55), from the
+// partial minima and maxima; one wave.
+__global__ __launch_bounds__(64) void interp_box_kernel(const float *__restrict__ part, int blocks,
+                                                        PlanHead *__restrict__ head) {
+#pragma clang fp contract(off)
+    for (int a = 0; a < 3; a++) {
+        float mn = FLT_MAX, mx = -FLT_MAX;
+        for (int k = threadIdx.x; k < blocks; k += 64) {
+            mn = fminf(mn, part[k * 6 + a]);
+            mx = fmaxf(mx, part[k * 6 + 3 + a]);
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+            mn = fminf(mn, __shfl_xor(mn, o));
+            mx = fmaxf(mx, __shfl_xor(mx, o));
+        }
+        if (threadIdx.x == 0) {
+            head->box.mn[a] = mn;
+            head->box.sc[a] = (float)(kBins - 1) / (mx - mn);
+        }
+    }
+    if (threadIdx.x == 0) head->total = 0;
+}
+
 __global__ void interp_zero_kernel(long long *p, int64_t n) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
          i += (int64_t)gridDim.x * blockDim.x)
         p[i] = 0;
 }
 
+// A vertex lies inside the box: (p - min) * scale is in [0, 127] up to rounding.
+__device__ __forceinline__ int vertex_bin(float x, float mn, float sc) {
+    return (int)fminf(rintf(fmaxf((x - mn) * sc, 0.0f)), (float)(kBins - 1));
+}
+
 // quantised bounding box of tetrahedron tid, clamped to the bins
-__device__ __forceinline__ void tet_bins(const Box &b, const float *__restrict__ v, long long tid,
+__device__ __forceinline__ void tet_bins(const Box &b, const float4 *__restrict__ v, int key,
                                          int nx, int ny, int lo[3], int hi[3]) {
-    const int4 id = tet_vertices(tid, nx, ny);
+    const int4 id = key_vertices(key, nx, ny);
     const int ids[4] = {id.x, id.y, id.z, id.w};
     lo[0] = lo[1] = lo[2] = kBins - 1;
     hi[0] = hi[1] = hi[2] = 0;
 #pragma unroll
     for (int c = 0; c < 4; c++) {
-        const float *p = v + 3 * (int64_t)ids[c];
+        const float4 q = v[ids[c]];
+        const float p[3] = {q.x, q.y, q.z};
 #pragma unroll
         for (int a = 0; a < 3; a++) {
-            // vertices lie inside the box: (p - min) * scale is in [0, 127] up to rounding
-            const float q = rintf(fmaxf((p[a] - b.mn[a]) * b.sc[a], 0.0f));
-            const int k = (int)fminf(q, (float)(kBins - 1));
+            const int k = vertex_bin(p[a], b.mn[a], b.sc[a]);
             lo[a] = min(lo[a], k);
             hi[a] = max(hi[a], k);
         }
     }
 }
 
-__global__ __launch_bounds__(256) void interp_count_kernel(Box b, const float *__restrict__ v,
+// head->total += the bins of every tetrahedron's box
+__global__ __launch_bounds__(256) void interp_total_kernel(const float4 *__restrict__ v,
+                                                           int64_t ncell, int nx, int ny,
+                                                           PlanHead *__restrict__ head) {
+    const Box b = head->box;
+    unsigned long long sum = 0;
+    for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < ncell; c += (int64_t)gridDim.x * 256) {
+        const int base = cell_base((unsigned)c, nx, ny);
+        int bin[8][3];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const float4 q = v[corner(base, k, nx, ny)];
+            bin[k][0] = vertex_bin(q.x, b.mn[0], b.sc[0]);
+            bin[k][1] = vertex_bin(q.y, b.mn[1], b.sc[1]);
+            bin[k][2] = vertex_bin(q.z, b.mn[2], b.sc[2]);
+        }
+#pragma unroll
+        for (int t = 0; t < 6; t++) {
+            unsigned long long n = 1;
+#pragma unroll
+            for (int a = 0; a < 3; a++) {
+                const int b0 = bin[kTet[t][0]][a], b1 = bin[kTet[t][1]][a],
+                          b2 = bin[kTet[t][2]][a], b3 = bin[kTet[t][3]][a];
+                n *= (unsigned)(max(max(b0, b1), max(b2, b3)) - min(min(b0, b1), min(b2, b3)) + 1);
+            }
+            sum += n;
+        }
+    }
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+    __shared__ unsigned long long red[4];
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(&head->total, red[0] + red[1] + red[2] + red[3]);
+}
+
+// The per-bin lists of the point-by-point location: every tetrahedron counted into, then
+// listed in, each bin of its box.
+__global__ __launch_bounds__(256) void interp_count_kernel(Box b, const float4 *__restrict__ v,
                                                            int64_t ntet, int nx, int ny,
                                                            long long *__restrict__ cnt) {
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (t >= ntet) return;
     int lo[3], hi[3];
-    tet_bins(b, v, t, nx, ny, lo, hi);
+    tet_bins(b, v, tet_key(t, nx, ny), nx, ny, lo, hi);
     for (int z = lo[2]; z <= hi[2]; z++)
         for (int y = lo[1]; y <= hi[1]; y++)
             for (int x = lo[0]; x <= hi[0]; x++)
                 atomicAdd((unsigned long long *)cnt + (x + kBins * (y + kBins * z)), 1ull);
 }
 
-__global__ __launch_bounds__(256) void interp_fill_kernel(Box b, const float *__restrict__ v,
+__global__ __launch_bounds__(256) void interp_fill_kernel(Box b, const float4 *__restrict__ v,
                                                           int64_t ntet, int nx, int ny,
                                                           const long long *__restrict__ start,
                                                           long long *__restrict__ cursor,
                                                           int *__restrict__ list) {
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (t >= ntet) return;
+    const int key = tet_key(t, nx, ny);
     int lo[3], hi[3];
-    tet_bins(b, v, t, nx, ny, lo, hi);
+    tet_bins(b, v, key, nx, ny, lo, hi);
     for (int z = lo[2]; z <= hi[2]; z++)
         for (int y = lo[1]; y <= hi[1]; y++)
             for (int x = lo[0]; x <= hi[0]; x++) {
                 const int64_t bin = x + kBins * (y + kBins * z);
                 const long long k = (long long)atomicAdd((unsigned long long *)cursor + bin, 1ull);
-                list[start[bin] + k] = tet_key(t, nx, ny);
+                list[start[bin] + k] = key;
             }
 }
 
@@ -237,7 +313,7 @@ __device__ __forceinline__ void xcd_tile(int &bx, int &by) {
 
 // FP32 barycentric coordinates of p in (v0, v1, v2, v3) and whether all are >= 0, in the
 // reference's operation order (spatial_hash_kernels.cuh:62-90), with no FMA contraction
-__device__ bool barycentric(const float *p, const float *v0, const float *v1, const float *v2,
+__device__ __forceinline__ bool barycentric(const float *p, const float *v0, const float *v1, const float *v2,
                             const float *v3, float w[4]) {
 #pragma clang fp contract(off)
     const float a0 = v1[0] - v0[0], a1 = v1[1] - v0[1], a2 = v1[2] - v0[2];
@@ -269,10 +345,41 @@ __device__ bool barycentric(const float *p, const float *v0, const float *v1, co
     return w[0] >= 0.0f && w[1] >= 0.0f && w[2] >= 0.0f && w[3] >= 0.0f;
 }
 
-// mode 0: idx[i] = vertex of largest weight (the reference's tie order); mode 1: idx[4 i..]
-// and w[4 i..]; -1 where no tetrahedron holds the point
+// "no tetrahedron holds the point" in the lookup of point i
+__device__ __forceinline__ void write_missing(int64_t i, int *idx) { idx[i] = -1; }
+
+// The lookup of point i in tetrahedron `key` with weights w.  Nearest: the vertex of largest
+// weight (the reference's tie order, float4_max_by_key, spatial_hash_kernels.cuh:51-59).
+// Linear: the key and weights 1 to 3; weight 0 is 1 - w1 - w2 - w3, formed again in the same order.
+__device__ __forceinline__ void write_found(int mode, int64_t i, int key, const float w[4], int nx,
+                                            int ny, int *idx, float *wout) {
+    if (mode == FFDAS_INTERP_NEAREST) {
+        const int4 id = key_vertices(key, nx, ny);
+        const int ixy = w[0] > w[1] ? id.x : id.y;
+        const float mxy = ixy == id.x ? w[0] : w[1];
+        const int izw = w[2] > w[3] ? id.z : id.w;
+        const float mzw = izw == id.z ? w[2] : w[3];
+        idx[i] = mxy > mzw ? ixy : izw;
+    } else {
+        idx[i] = key;
+        wout[3 * i] = w[1];
+        wout[3 * i + 1] = w[2];
+        wout[3 * i + 2] = w[3];
+    }
+}
+
+__device__ __forceinline__ bool test_key(const float p[3], int key, const float4 *__restrict__ v,
+                                         int nx, int ny, float w[4]) {
+    const int4 id = key_vertices(key, nx, ny);
+    const float4 a = v[id.x], b = v[id.y], c = v[id.z], d = v[id.w];
+    const float pa[3] = {a.x, a.y, a.z}, pb[3] = {b.x, b.y, b.z}, pc[3] = {c.x, c.y, c.z},
+                pd[3] = {d.x, d.y, d.z};
+    return barycentric(p, pa, pb, pc, pd, w);
+}
+
+// Point by point: every point tests the tetrahedra of its bin's list and keeps the lowest id.
 __global__ __launch_bounds__(256) void interp_locate_kernel(
-    Box b, const float *__restrict__ v, int nx, int ny, int64_t ntet,
+    Box b, const float4 *__restrict__ v, int nx, int ny, int64_t ntet,
     const long long *__restrict__ start, const int *__restrict__ list,
     const float *__restrict__ qp, int64_t n, int mode, int *__restrict__ idx,
     float *__restrict__ wout) {
@@ -281,55 +388,38 @@ __global__ __launch_bounds__(256) void interp_locate_kernel(
     const float p[3] = {qp[3 * i], qp[3 * i + 1], qp[3 * i + 2]};
     int ix, iy, iz;
     int best = INT_MAX;
-    int4 bid{-1, -1, -1, -1};
     float bw[4] = {0, 0, 0, 0};
     if (ntet > 0 && quantize(b, p[0], p[1], p[2], ix, iy, iz)) {
         const int64_t bin = ix + kBins * (iy + kBins * (int64_t)iz);
         for (long long e = start[bin]; e < start[bin + 1]; e++) {
             const int t = list[e];
-            if (t >= best) continue;
-            const int4 id = key_vertices(t, nx, ny);
             float w[4];
-            if (barycentric(p, v + 3 * (int64_t)id.x, v + 3 * (int64_t)id.y, v + 3 * (int64_t)id.z,
-                            v + 3 * (int64_t)id.w, w)) {
+            if (t < best && test_key(p, t, v, nx, ny, w)) {
                 best = t;
-                bid = id;
 #pragma unroll
                 for (int c = 0; c < 4; c++) bw[c] = w[c];
             }
         }
     }
-    if (mode == FFDAS_INTERP_NEAREST) {
-        int r = -1;
-        if (best != INT_MAX) {   // float4_max_by_key (spatial_hash_kernels.cuh:51-59)
-            const int ixy = bw[0] > bw[1] ? bid.x : bid.y;
-            const float mxy = ixy == bid.x ? bw[0] : bw[1];
-            const int izw = bw[2] > bw[3] ? bid.z : bid.w;
-            const float mzw = izw == bid.z ? bw[2] : bw[3];
-            r = mxy > mzw ? ixy : izw;
-        }
-        idx[i] = r;
-    } else {
-        reinterpret_cast<int4 *>(idx)[i] = bid;
-        reinterpret_cast<float4 *>(wout)[i] = float4{bw[0], bw[1], bw[2], bw[3]};
-    }
+    if (best != INT_MAX)
+        write_found(mode, i, best, bw, nx, ny, idx, wout);
+    else
+        write_missing(i, idx);
 }
 
 // ---------------------------------------------------------------------------------------
-// Location by bins: the query points are counted and ordered by bin, and one wave per bin
-// loads the bin's points (one per lane) and candidate tetrahedra (key, vertices and bounding
-// box, one per lane and chunk) once and tests every point of the bin against them, so each
-// candidate's vertices are fetched once per bin rather than once per point, and no load waits
-// inside the per-point loop (the per-point scan re-read about 3.2 KB per point on a 512 x 96 x 96
-// sector with 256^3 query points).  The result is the same: per point, the lowest passing key
-// of its bin.
+// Location by cells.  The query points are counted, scanned and ordered by bin, so that the
+// points of the bins (x0 .. x1, y, z) are one run, and every cell walks the runs of its quantised
+// bounding box (the union of its tetrahedra's boxes: every tetrahedron the reference would list
+// in a point's bin is met).  A point inside the cell's box, widened by 5 % of its extent plus
+// 1e-5 of the coordinates' magnitude per axis (the FP32 weights of a tetrahedron that the 1e-12
+// volume test admits err far less than that), is tested against the six tetrahedra in order; one
+// that passes, and whose own quantised box holds the point's bin, lowers the point's best key
+// by an atomic minimum.  The lookups are written by a last pass over the points.  No lists of
+// tetrahedra are built: their atomics met at the apex of a sector, where thousands of small
+// cells share a bin (512 x 96 x 96 sector: count 7.9 and fill 8.7 ms of a plan, and 7.7 ms to
+// locate 256^3 points in them; now 0.3 ms and 3.6 ms).
 // ---------------------------------------------------------------------------------------
-
-__global__ __launch_bounds__(256) void interp_pad_kernel(const float *__restrict__ v, int64_t n,
-                                                         float4 *__restrict__ v4) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) v4[i] = float4{v[3 * i], v[3 * i + 1], v[3 * i + 2], 0.f};
-}
 
 __global__ void interp_zero_i32_kernel(int *p, int64_t n) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
@@ -337,188 +427,154 @@ __global__ void interp_zero_i32_kernel(int *p, int64_t n) {
         p[i] = 0;
 }
 
-// "no tetrahedron holds the point" in the lookup of point i
-__device__ __forceinline__ void write_missing(int mode, int64_t i, int *idx, float *wout) {
-    if (mode == FFDAS_INTERP_NEAREST) {
-        idx[i] = -1;
-    } else {
-        reinterpret_cast<int4 *>(idx)[i] = int4{-1, -1, -1, -1};
-        reinterpret_cast<float4 *>(wout)[i] = float4{0.f, 0.f, 0.f, 0.f};
-    }
-}
-
-// pbin[i] = the point's bin, or -1 (outside the bins, or no tetrahedra: its lookup is written
-// here); cnt[bin] counts the points of each bin
-__global__ __launch_bounds__(256) void interp_point_bin_kernel(
-    Box b, const float *__restrict__ qp, int64_t n, int64_t ntet, int mode,
-    int *__restrict__ pbin, int *__restrict__ cnt, int *__restrict__ idx,
-    float *__restrict__ wout) {
+// cnt[bin] = the points of each bin; a point outside the bins has its lookup written here
+__global__ __launch_bounds__(256) void interp_point_bin_kernel(Box b, const float *__restrict__ qp,
+                                                               int64_t n, int *__restrict__ cnt,
+                                                               int *__restrict__ idx) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
-    int ix, iy, iz, bin = -1;
-    if (ntet > 0 && quantize(b, qp[3 * i], qp[3 * i + 1], qp[3 * i + 2], ix, iy, iz))
-        bin = ix + kBins * (iy + kBins * iz);
-    pbin[i] = bin;
-    if (bin >= 0)
-        atomicAdd(cnt + bin, 1);
+    int ix, iy, iz;
+    if (quantize(b, qp[3 * i], qp[3 * i + 1], qp[3 * i + 2], ix, iy, iz))
+        atomicAdd(cnt + (ix + kBins * (iy + kBins * iz)), 1);
     else
-        write_missing(mode, i, idx, wout);
+        write_missing(i, idx);
 }
 
-// order[start[bin] ..) = the points of each bin (counting cnt back down to 0)
-__global__ __launch_bounds__(256) void interp_point_order_kernel(const int *__restrict__ pbin,
-                                                                 int64_t n,
-                                                                 const int *__restrict__ start,
-                                                                 int *__restrict__ cnt,
-                                                                 int *__restrict__ order) {
+// pts[start[bin] ..) = the points of each bin (position, id), counting cnt back down to 0;
+// best = none
+__global__ __launch_bounds__(256) void interp_point_order_kernel(
+    Box b, const float *__restrict__ qp, int64_t n, const int *__restrict__ start,
+    int *__restrict__ cnt, float4 *__restrict__ pts, int *__restrict__ best) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
-    const int bin = pbin[i];
-    if (bin < 0) return;
-    order[start[bin] + atomicSub(cnt + bin, 1) - 1] = (int)i;
+    const float x = qp[3 * i], y = qp[3 * i + 1], z = qp[3 * i + 2];
+    int ix, iy, iz;
+    if (!quantize(b, x, y, z, ix, iy, iz)) return;
+    const int bin = ix + kBins * (iy + kBins * iz);
+    const int e = start[bin] + atomicSub(cnt + bin, 1) - 1;
+    pts[e] = float4{x, y, z, __int_as_float((int)i)};
+    best[e] = INT_MAX;
 }
 
-// One wave per bin.  The bin's points come in batches of 64, one per lane (its id and
-// position, loaded once); the bin's candidates in groups of up to two chunks of 64, lane c
-// holding candidate c of each chunk in registers (its key, vertices and bounding box), each
-// group loaded once per batch.  For each point t of the batch (read from lane t), a chunk is tested
-// only if the point lies in the box of one of its candidates, widened by 5 % of its extent plus
-// 1e-5 of the coordinates' magnitude per axis (the FP32 barycentric weights of a tetrahedron
-// that the 1e-12 volume test admits err far less than that, so no candidate the test would
-// pass is skipped); then every lane runs the reference's FP32 test on its candidate.  A chunk's passing lanes come from one ballot, usually none or one, whose keys a scalar
-// loop compares with point t's best so far; point t's best key and the winner's weights are
-// kept in lane t.  Lane t then writes the lookup of point t (mode 0: the vertex of largest
-// weight; mode 1: ids and weights), or "none".
-constexpr int kLocateChunks = 2;
-
-__device__ __forceinline__ float readlane_f(float v, int l) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-}
-
-
-__global__ __launch_bounds__(256) void interp_locate_bin_kernel(
-    const float4 *__restrict__ v4, int nx, int ny, const long long *__restrict__ start,
-    const int *__restrict__ list, const float *__restrict__ qp, const int *__restrict__ pstart,
-    const int *__restrict__ order, int mode, int *__restrict__ idx, float *__restrict__ wout) {
+// 2^(lgr + lgp) lanes per cell: 2^lgr share out the runs of its box, 2^lgp the points of a run.
+// The points inside a cell's box are few and come to the lanes at different times, so they are
+// put on a queue of the wave, and the tests, most of the work, run with a queued point in
+// every lane (one lane testing its own point on the spot: 0.54 ms for the cells of a 256 x 64 x 64
+// sector and 128^3 points, 0.26 ms queued).
+__global__ __launch_bounds__(256) void interp_locate_cells_kernel(
+    Box b, const float4 *__restrict__ v, int64_t ncell, int nx, int ny, int lgr, int lgp,
+    const int *__restrict__ pstart, const float4 *__restrict__ pts, int *__restrict__ best) {
+    __shared__ int2 queue[4][128];           // (base vertex, point) by wave
     const int lane = threadIdx.x & 63;
-    const int64_t bin = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (bin >= kBins3) return;
-    const int ps = pstart[bin], pe = pstart[bin + 1];
-    if (ps == pe) return;
-    const long long cs = start[bin], ce = start[bin + 1];
-    constexpr int G = 64 * kLocateChunks;
-    int key[kLocateChunks];
-    float lo[kLocateChunks][3], hi[kLocateChunks][3], vp[kLocateChunks][4][3];
-    // the group of chunks from g0: key INT_MAX (and an empty box) past the list
-    const auto load = [&](long long g0) {
+    int2 *q = queue[threadIdx.x >> 6];
+    const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t cell = gid >> (lgr + lgp);
+    const int psub = (int)gid & ((1 << lgp) - 1), rsub = (int)(gid >> lgp) & ((1 << lgr) - 1);
+    int base = 0, rows = 0, ny1 = 1;
+    float lo[3], hi[3];
+    int b0[3] = {kBins - 1, kBins - 1, kBins - 1}, b1[3] = {0, 0, 0};
 #pragma unroll
-        for (int c = 0; c < kLocateChunks; ++c) {
-            const long long e = g0 + 64 * c + lane;
-            key[c] = INT_MAX;
+    for (int a = 0; a < 3; a++) {
+        lo[a] = 3.4e38f;
+        hi[a] = -3.4e38f;
+    }
+    if (cell < ncell) {
+        base = cell_base((unsigned)cell, nx, ny);
 #pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                lo[c][a] = 3.4e38f;
-                hi[c][a] = -3.4e38f;
+        for (int k = 0; k < 8; k++) {
+            const float4 u = v[corner(base, k, nx, ny)];
+            const float p[3] = {u.x, u.y, u.z};
+#pragma unroll
+            for (int a = 0; a < 3; a++) {
+                lo[a] = fminf(lo[a], p[a]);
+                hi[a] = fmaxf(hi[a], p[a]);
+                const int q1 = vertex_bin(p[a], b.mn[a], b.sc[a]);
+                b0[a] = min(b0[a], q1);
+                b1[a] = max(b1[a], q1);
             }
-            if (e < ce) {
-                key[c] = list[e];
-                const int4 id = key_vertices(key[c], nx, ny);
-                const int ids[4] = {id.x, id.y, id.z, id.w};
+        }
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const float4 x = v4[ids[q]];
-                    vp[c][q][0] = x.x;
-                    vp[c][q][1] = x.y;
-                    vp[c][q][2] = x.z;
-#pragma unroll
-                    for (int a = 0; a < 3; ++a) {
-                        lo[c][a] = fminf(lo[c][a], vp[c][q][a]);
-                        hi[c][a] = fmaxf(hi[c][a], vp[c][q][a]);
-                    }
-                }
-#pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    const float m = 0.05f * (hi[c][a] - lo[c][a]) +
-                                    1e-5f * (fabsf(lo[c][a]) + fabsf(hi[c][a])) + 1e-30f;
-                    lo[c][a] -= m;
-                    hi[c][a] += m;
-                }
-            }
+        for (int a = 0; a < 3; a++) {
+            const float m = 0.05f * (hi[a] - lo[a]) + 1e-5f * (fabsf(lo[a]) + fabsf(hi[a])) + 1e-30f;
+            lo[a] -= m;
+            hi[a] += m;
+        }
+        ny1 = b1[1] - b0[1] + 1;
+        rows = ny1 * (b1[2] - b0[2] + 1);
+    }
+    // a queued point against the six tetrahedra of its cell
+    auto test = [&](int2 c) {
+        const float4 u = pts[c.y];
+        const float p[3] = {u.x, u.y, u.z};
+        // an outdated best only costs a test: the minimum is taken atomically
+        const int known = best[c.y];
+#pragma unroll 1
+        for (int key = c.x * 8; key < min(c.x * 8 + 6, known); key++) {
+            float w[4];
+            if (!test_key(p, key, v, nx, ny, w)) continue;
+            int tl[3], th[3], ib[3];
+            tet_bins(b, v, key, nx, ny, tl, th);
+            (void)quantize(b, p[0], p[1], p[2], ib[0], ib[1], ib[2]);
+            if (ib[0] < tl[0] || ib[0] > th[0] || ib[1] < tl[1] || ib[1] > th[1] ||
+                ib[2] < tl[2] || ib[2] > th[2])
+                continue;
+            atomicMin(best + c.y, key);
+            break;
         }
     };
-    const bool one_group = ce - cs <= G;
-    if (one_group) load(cs);
-    for (int q0 = ps; q0 < pe; q0 += 64) {
-        const int np = min(64, pe - q0);
-        // point q0 + lane: its id, position, and best key and weights so far
-        int mi = -1, mbest = INT_MAX;
-        float mp[3] = {0.f, 0.f, 0.f}, mw[4] = {0.f, 0.f, 0.f, 0.f};
-        if (lane < np) {
-            mi = order[q0 + lane];
-#pragma unroll
-            for (int a = 0; a < 3; ++a) mp[a] = qp[3 * (int64_t)mi + a];
+    int r = rsub, e = 0, pe = 0, waiting = 0;     // waiting: queued points, uniform
+    for (;;) {
+        // a step takes a point of the run, or goes to the next run
+        bool hit = false;
+        int at = 0;
+        if (e < pe) {
+            const float4 u = pts[e];
+            hit = u.x >= lo[0] && u.x <= hi[0] && u.y >= lo[1] && u.y <= hi[1] &&
+                  u.z >= lo[2] && u.z <= hi[2];
+            at = e;
+            e += 1 << lgp;
+        } else if (r < rows) {
+            const int dz = r / ny1, row = kBins * (b0[1] + r - dz * ny1 + kBins * (b0[2] + dz));
+            e = pstart[row + b0[0]] + psub;
+            pe = pstart[row + b1[0] + 1];
+            r += 1 << lgr;
         }
-        for (long long g0 = cs; g0 < ce; g0 += G) {
-            if (!one_group) load(g0);
-            for (int t = 0; t < np; ++t) {
-                const float p[3] = {readlane_f(mp[0], t), readlane_f(mp[1], t),
-                                    readlane_f(mp[2], t)};
-                int best = __builtin_amdgcn_readlane(mbest, t);
-                int won = -1;   // uniform
-#pragma unroll
-                for (int c = 0; c < kLocateChunks; ++c) {
-                    if (g0 + 64 * c >= ce) break;   // uniform
-                    const bool near = key[c] < best && p[0] >= lo[c][0] && p[0] <= hi[c][0] &&
-                                      p[1] >= lo[c][1] && p[1] <= hi[c][1] &&
-                                      p[2] >= lo[c][2] && p[2] <= hi[c][2];
-                    if (__ballot(near) == 0) continue;   // no candidate of the chunk can pass
-                    float w[4] = {0.f, 0.f, 0.f, 0.f};
-                    bool pass = false;
-                    if (key[c] < best)
-                        pass = barycentric(p, vp[c][0], vp[c][1], vp[c][2], vp[c][3], w);
-                    uint64_t m = __ballot(pass);
-                    int cw = -1;
-                    while (m) {
-                        const int l = __builtin_ctzll(m);
-                        m &= m - 1;
-                        const int k = __builtin_amdgcn_readlane(key[c], l);
-                        if (k < best) {
-                            best = k;
-                            cw = l;
-                        }
-                    }
-                    if (cw >= 0) {
-                        won = cw;
-                        // the winner's weights into lane t
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) {
-                            const float wu = readlane_f(w[u], cw);
-                            mw[u] = lane == t ? wu : mw[u];
-                        }
-                    }
-                }
-                if (won >= 0 && lane == t) mbest = best;
+        const bool live = e < pe || r < rows;
+        const uint64_t hits = __ballot(hit);
+        if (hits) {
+            if (hit)
+                q[waiting + __builtin_amdgcn_mbcnt_hi((unsigned)(hits >> 32),
+                                                      __builtin_amdgcn_mbcnt_lo((unsigned)hits, 0))] =
+                    int2{base, at};
+            waiting += __popcll(hits);
+            if (waiting >= 64) {
+                waiting -= 64;
+                test(q[waiting + lane]);
             }
         }
-        if (lane < np) {
-            if (mbest == INT_MAX) {
-                write_missing(mode, mi, idx, wout);
-            } else {
-                const int4 bid = key_vertices(mbest, nx, ny);
-                if (mode == FFDAS_INTERP_NEAREST) {
-                    // float4_max_by_key (spatial_hash_kernels.cuh:51-59)
-                    const int ixy = mw[0] > mw[1] ? bid.x : bid.y;
-                    const float mxy = ixy == bid.x ? mw[0] : mw[1];
-                    const int izw = mw[2] > mw[3] ? bid.z : bid.w;
-                    const float mzw = izw == bid.z ? mw[2] : mw[3];
-                    idx[mi] = mxy > mzw ? ixy : izw;
-                } else {
-                    reinterpret_cast<int4 *>(idx)[mi] = bid;
-                    reinterpret_cast<float4 *>(wout)[mi] = float4{mw[0], mw[1], mw[2], mw[3]};
-                }
-            }
-        }
+        if (__ballot(live) == 0) break;
     }
+    if (lane < waiting) test(q[lane]);
+}
+
+// The lookups of the ordered points.
+__global__ __launch_bounds__(256) void interp_found_kernel(
+    const float4 *__restrict__ v, int nx, int ny, const int *__restrict__ count,
+    const float4 *__restrict__ pts, const int *__restrict__ best, int mode, int *__restrict__ idx,
+    float *__restrict__ wout) {
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= *count) return;
+    const float4 q = pts[e];
+    const int key = best[e];
+    const int64_t i = __float_as_int(q.w);
+    if (key == INT_MAX) {
+        write_missing(i, idx);
+        return;
+    }
+    const float p[3] = {q.x, q.y, q.z};
+    float w[4];
+    (void)test_key(p, key, v, nx, ny, w);
+    write_found(mode, i, key, w, nx, ny, idx, wout);
 }
 
 // element types: real or complex (two components), FP32 or FP64
@@ -527,40 +583,38 @@ struct El {
     R c[CW];
 };
 
-// Outputs are written once and never read back by the kernel: streamed past the caches so
+// Outputs are written once and never read back by the kernel: streamed past the caches (NT) so
 // they do not evict the vertex blocks that neighbouring query points gather.
-template <typename R, int CW>
+template <bool NT, typename R, int CW>
 __device__ __forceinline__ void put_out(El<R, CW> *p, const El<R, CW> &v) {
+    if constexpr (NT) {
 #pragma unroll
-    for (int c = 0; c < CW; c++) __builtin_nontemporal_store(v.c[c], &p->c[c]);
+        for (int c = 0; c < CW; c++) __builtin_nontemporal_store(v.c[c], &p->c[c]);
+    } else {
+        *p = v;
+    }
 }
 
-constexpr int kFramesPerThread = 8;   // frames per chunk: the smallest, for the extent check
+constexpr int kFramesPerThread = 8;   // frames per chunk of 8-byte elements, for the extent check
 
-// frames per chunk: 16 for 4-byte elements (a 64-byte vector load per vertex), else 8
-template <typename R, int CW>
-constexpr int frames_per_chunk() {
-    return sizeof(R) * CW == 4 ? 16 : 8;
-}
-
-// the frames of one vertex in one chunk, contiguous: one vector load per vertex
-template <typename R, int CW>
-struct alignas(16) Frames {
-    El<R, CW> f[frames_per_chunk<R, CW>()];
+// the frames of one vertex in one chunk, contiguous: one vector load per vertex.  A chunk of one
+// frame is x as it is (element-aligned).
+template <typename R, int CW, int FPC>
+struct alignas(FPC == 1 ? sizeof(R) : (sizeof(R) * CW * FPC < 16 ? sizeof(R) * CW * FPC : 16)) Frames {
+    El<R, CW> f[FPC];
 };
 
 // x [frame][vertex] -> xfi [chunk][vertex][frame in chunk], zero past the last frame; each
 // thread reads its vertex from the chunk's frames (coalesced per frame) and writes the
 // vertex's frames as one contiguous block (coalesced across threads)
-template <typename R, int CW>
+template <typename R, int CW, int FPC>
 __global__ __launch_bounds__(256) void interp_frames_kernel(const El<R, CW> *__restrict__ x,
-                                                            Frames<R, CW> *__restrict__ xfi,
+                                                            Frames<R, CW, FPC> *__restrict__ xfi,
                                                             int64_t npts, int64_t B) {
-    constexpr int FPC = frames_per_chunk<R, CW>();
     const int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (v >= npts) return;
     const int64_t b0 = (int64_t)blockIdx.y * FPC;
-    Frames<R, CW> o;
+    Frames<R, CW, FPC> o;
 #pragma unroll
     for (int f = 0; f < FPC; f++) {
         if (b0 + f < B) {
@@ -573,13 +627,10 @@ __global__ __launch_bounds__(256) void interp_frames_kernel(const El<R, CW> *__r
     xfi[blockIdx.y * npts + v] = o;
 }
 
-template <typename R, int CW>
-__global__ __launch_bounds__(256) void interp_nearest_kernel(const Frames<R, CW> *__restrict__ xfi,
-                                                             El<R, CW> *__restrict__ out,
-                                                             const int *__restrict__ idx, int64_t n,
-                                                             int64_t npts, int64_t B,
-                                                             El<R, CW> fill) {
-    constexpr int FPC = frames_per_chunk<R, CW>();
+template <typename R, int CW, int FPC>
+__global__ __launch_bounds__(256) void interp_nearest_kernel(
+    const Frames<R, CW, FPC> *__restrict__ xfi, El<R, CW> *__restrict__ out,
+    const int *__restrict__ idx, int64_t n, int64_t npts, int64_t B, El<R, CW> fill) {
     int bx, by;
     xcd_tile(bx, by);
     const int64_t i = (int64_t)bx * 256 + threadIdx.x;
@@ -588,64 +639,107 @@ __global__ __launch_bounds__(256) void interp_nearest_kernel(const Frames<R, CW>
     const int64_t b0 = (int64_t)by * FPC;
     const int nf = (int)(B - b0 < FPC ? B - b0 : FPC);
     if (k >= 0) {
-        const Frames<R, CW> v = xfi[by * npts + k];
+        const Frames<R, CW, FPC> v = xfi[by * npts + k];
 #pragma unroll
         for (int f = 0; f < FPC; f++)
-            if (f < nf) put_out(out + (b0 + f) * n + i, v.f[f]);
+            if (f < nf) put_out<true>(out + (b0 + f) * n + i, v.f[f]);
     } else {
 #pragma unroll
         for (int f = 0; f < FPC; f++)
-            if (f < nf) put_out(out + (b0 + f) * n + i, fill);
+            if (f < nf) put_out<true>(out + (b0 + f) * n + i, fill);
     }
 }
 
-template <typename R, int CW>
-__global__ __launch_bounds__(256) void interp_linear_kernel(const Frames<R, CW> *__restrict__ xfi,
-                                                            El<R, CW> *__restrict__ out,
-                                                            const int4 *__restrict__ idx,
-                                                            const float4 *__restrict__ wt, int64_t n,
-                                                            int64_t npts, int64_t B,
-                                                            El<R, CW> fill) {
+// Every output is written once, the frame-inner copy is read about once, and per point a key, and
+// three weights where it is located: bound by HBM and by the vector L1, whose accesses are the
+// vertex blocks.  Two lanes share a point of a 32-byte block or more, each taking half of its
+// vertices' blocks, so that a load instruction touches half as many blocks; a wave covers 64
+// consecutive points in two turns, all their loads in flight together.  The stores of an
+// instruction are then runs of 32 points (128 bytes of 4-byte elements): streamed where those
+// are whole cache lines (NT), through L2, which joins them, where they are not.  16 frames of a
+// 512 x 96 x 96 sector to 256^3 points: 0.558 ms with a lane per point and ids and weights of 32
+// bytes a point, 0.517 ms with keys and three weights, 0.46 ms with two lanes (four: 0.62, their
+// runs are half lines).  To 255^3 points, off the lines, the call takes 0.66 ms through L2 and
+// 1.02 ms streamed.
+template <typename R, int CW, int FPC, bool NT>
+__global__ __launch_bounds__(256) void interp_linear_kernel(
+    const Frames<R, CW, FPC> *__restrict__ xfi, El<R, CW> *__restrict__ out,
+    const int *__restrict__ idx, const float *__restrict__ wt, int nx, int ny, int64_t n,
+    int64_t npts, int64_t B, El<R, CW> fill) {
 #pragma clang fp contract(off)
-    constexpr int FPC = frames_per_chunk<R, CW>();
+    constexpr int BB = FPC * (int)sizeof(El<R, CW>);          // bytes of a vertex's block
+    constexpr int LPP = BB >= 32 ? 2 : 1;
+    constexpr int EPL = FPC / LPP;                            // frames of a lane
+    using Part = Frames<R, CW, EPL>;
     int bx, by;
     xcd_tile(bx, by);
-    const int64_t i = (int64_t)bx * 256 + threadIdx.x;
-    if (i >= n) return;
+    const int lane = threadIdx.x & 63, sub = lane % LPP;
+    const int64_t i0 = (int64_t)bx * 256 + (threadIdx.x & ~63) + lane / LPP;
+    const int64_t b0 = (int64_t)by * FPC + sub * EPL;
+    const int nf = (int)(B - b0 < EPL ? B - b0 : EPL);
+    const Part *xc = reinterpret_cast<const Part *>(xfi + by * npts) + sub;
     // the lookup is read once per frame chunk: streamed, like the outputs
-    typedef int I4 __attribute__((ext_vector_type(4)));
-    typedef float F4 __attribute__((ext_vector_type(4)));
-    const I4 kv = __builtin_nontemporal_load(reinterpret_cast<const I4 *>(idx) + i);
-    const F4 wv = __builtin_nontemporal_load(reinterpret_cast<const F4 *>(wt) + i);
-    const int4 k = make_int4(kv.x, kv.y, kv.z, kv.w);
-    const float4 w = make_float4(wv.x, wv.y, wv.z, wv.w);
-    const int64_t b0 = (int64_t)by * FPC;
-    const int nf = (int)(B - b0 < FPC ? B - b0 : FPC);
-    const Frames<R, CW> *xc = xfi + by * npts;
-    // unlocated points read vertex 0 (always present) and write the fill value: the loads
-    // stay unconditional, so the four blocks live in registers
-    const bool in = k.x >= 0;
-    const Frames<R, CW> v0 = xc[in ? k.x : 0], v1 = xc[in ? k.y : 0], v2 = xc[in ? k.z : 0],
-                        v3 = xc[in ? k.w : 0];
+    int key[LPP];
+    bool any = false;
 #pragma unroll
-    for (int f = 0; f < FPC; f++) {
-        El<R, CW> r;
+    for (int r = 0; r < LPP; r++) {
+        const int64_t i = i0 + r * (64 / LPP);
+        key[r] = i < n ? __builtin_nontemporal_load(idx + i) : -1;
+        any = any || key[r] >= 0;
+    }
+    if (__ballot(any) == 0) {
+#pragma unroll
+        for (int r = 0; r < LPP; r++) {
+            const int64_t i = i0 + r * (64 / LPP);
+#pragma unroll
+            for (int f = 0; f < EPL; f++)
+                if (i < n && f < nf) put_out<NT>(out + (b0 + f) * n + i, fill);
+        }
+        return;
+    }
+    float w[LPP][3];
+    Part v[LPP][4];
+#pragma unroll
+    for (int r = 0; r < LPP; r++) {
+        // points outside read vertex 0 and weights that are not used: the loads stay
+        // unconditional
+        const bool in = key[r] >= 0;
+        typedef float F3 __attribute__((ext_vector_type(3), aligned(4)));
+        const F3 q = __builtin_nontemporal_load(
+            reinterpret_cast<const F3 *>(wt + (in ? 3 * (i0 + r * (64 / LPP)) : 0)));
+        w[r][0] = q.x;
+        w[r][1] = q.y;
+        w[r][2] = q.z;
+        const int4 k = in ? key_vertices(key[r], nx, ny) : int4{0, 0, 0, 0};
+        v[r][0] = xc[(int64_t)k.x * LPP];
+        v[r][1] = xc[(int64_t)k.y * LPP];
+        v[r][2] = xc[(int64_t)k.z * LPP];
+        v[r][3] = xc[(int64_t)k.w * LPP];
+    }
+#pragma unroll
+    for (int r = 0; r < LPP; r++) {
+        const int64_t i = i0 + r * (64 / LPP);
+        const float w0 = 1.0f - w[r][0] - w[r][1] - w[r][2];
         // w0 v0 + w1 v1 + w2 v2 + w3 v3, left to right (interpolation_kernels.cuh:110-115)
 #pragma unroll
-        for (int c = 0; c < CW; c++)
-            r.c[c] = in ? (R)w.x * v0.f[f].c[c] + (R)w.y * v1.f[f].c[c] + (R)w.z * v2.f[f].c[c] +
-                              (R)w.w * v3.f[f].c[c]
-                        : fill.c[c];
-        if (f < nf) put_out(out + (b0 + f) * n + i, r);
+        for (int f = 0; f < EPL; f++) {
+            El<R, CW> o;
+#pragma unroll
+            for (int c = 0; c < CW; c++)
+                o.c[c] = key[r] >= 0 ? (R)w0 * v[r][0].f[f].c[c] + (R)w[r][0] * v[r][1].f[f].c[c] +
+                                           (R)w[r][1] * v[r][2].f[f].c[c] +
+                                           (R)w[r][2] * v[r][3].f[f].c[c]
+                                     : fill.c[c];
+            if (i < n && f < nf) put_out<NT>(out + (b0 + f) * n + i, o);
+        }
     }
 }
 
 void free_plan_device(ffdas_interpolation_plan *p) {
-    for (void *q : {(void *)p->verts, (void *)p->verts4, (void *)p->bin_start, (void *)p->bin_list,
+    for (void *q : {(void *)p->verts, (void *)p->bin_start, (void *)p->bin_list,
                     (void *)p->pre_idx, (void *)p->pre_w})
         if (q) (void)hipFree(q);
     p->verts = nullptr;
-    p->verts4 = nullptr;
     p->bin_start = nullptr;
     p->bin_list = nullptr;
     p->pre_idx = nullptr;
@@ -663,179 +757,232 @@ Box box_of(const ffdas_interpolation_plan &p) {
 
 int grid1(int64_t n) { return (int)std::max<int64_t>(1, (n + 255) / 256); }
 
-// locate n points into idx (and w): device buffers sized by the caller.  By bins (the points
-// counted, scanned and ordered by bin in the handle's workspace, then one wave per bin) when
-// the point ids fit an int and FFDAS_INTERP_LOCATE is not "point"; otherwise one thread per
-// point scanning its bin.
-ffdas_error_t locate(ffdas_context &h, const ffdas_interpolation_plan &p, const float *qp, int64_t n,
-                     int *idx, float *w) {
-    const char *how = std::getenv("FFDAS_INTERP_LOCATE");
-    const bool by_bins = n < INT_MAX && !(how && std::string(how) == "point");
-    if (!by_bins) {
-        ProfScope ps(h.stream, "interp_locate");
-        hipLaunchKernelGGL(interp_locate_kernel, dim3(grid1(n)), dim3(256), 0, h.stream,
-                           box_of(p), p.verts, (int)p.nx, (int)p.ny, p.ntet, p.bin_start,
-                           p.bin_list, qp, n, p.mode, idx, w);
-        return hip_status(hipGetLastError(), FFDAS_ERROR_CUDA_LAUNCH_FAILED);
-    }
+size_t up256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+// The per-bin lists of the point-by-point location, once per plan.
+ffdas_error_t build_lists(ffdas_context &h, ffdas_interpolation_plan &p) {
+    std::lock_guard<std::mutex> lock(p.list_mutex);
+    if (p.bin_list) return FFDAS_SUCCESS;
     hipStream_t st = h.stream;
     const size_t nb = (size_t)kBins3 + 1;
-    size_t scan_bytes = 0;
-    int *no_int = nullptr;
-    if (rocprim::exclusive_scan(nullptr, scan_bytes, no_int, no_int, 0, nb, rocprim::plus<int>(),
-                                st) != hipSuccess)
-        return FFDAS_ERROR_CUDA_LAUNCH_FAILED;
-    const auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    const size_t b_pbin = up((size_t)n * 4), b_cnt = up(nb * 4), b_scan = up(scan_bytes);
-    void *ws = nullptr;
-    FFDAS_TRY(h.workspace(2 * b_pbin + 2 * b_cnt + b_scan, &ws));
-    h.xcopy.valid = false;   // the converted-x record of the delay-and-sum calls
-    char *c = (char *)ws;
-    int *pbin = (int *)c, *order = (int *)(c + b_pbin);
-    int *cnt = (int *)(c + 2 * b_pbin), *pstart = (int *)(c + 2 * b_pbin + b_cnt);
-    void *scan_tmp = c + 2 * b_pbin + 2 * b_cnt;
-    ProfScope ps(st, "interp_locate");
-    hipLaunchKernelGGL(interp_zero_i32_kernel, dim3(1024), dim3(256), 0, st, cnt, (int64_t)nb);
-    hipLaunchKernelGGL(interp_point_bin_kernel, dim3(grid1(n)), dim3(256), 0, st, box_of(p), qp, n,
-                       p.ntet, p.mode, pbin, cnt, idx, w);
-    if (rocprim::exclusive_scan(scan_tmp, scan_bytes, cnt, pstart, 0, nb, rocprim::plus<int>(),
-                                st) != hipSuccess)
-        return FFDAS_ERROR_CUDA_LAUNCH_FAILED;
-    hipLaunchKernelGGL(interp_point_order_kernel, dim3(grid1(n)), dim3(256), 0, st, pbin, n,
-                       pstart, cnt, order);
-    hipLaunchKernelGGL(interp_locate_bin_kernel, dim3((unsigned)((kBins3 + 3) / 4)), dim3(256), 0,
-                       st, p.verts4, (int)p.nx, (int)p.ny, p.bin_start, p.bin_list, qp, pstart,
-                       order, p.mode, idx, w);
-    return hip_status(hipGetLastError(), FFDAS_ERROR_CUDA_LAUNCH_FAILED);
-}
-
-ffdas_error_t alloc_lookup(int mode, int64_t n, int **idx, float **w) {
-    const size_t ni = (size_t)n * (mode == FFDAS_INTERP_NEAREST ? 1 : 4);
-    if (hipMalloc((void **)idx, ni * sizeof(int)) != hipSuccess) return FFDAS_ERROR_ALLOCATION_FAILED;
-    *w = nullptr;
-    if (mode != FFDAS_INTERP_NEAREST &&
-        hipMalloc((void **)w, (size_t)n * 4 * sizeof(float)) != hipSuccess) {
-        (void)hipFree(*idx);
-        *idx = nullptr;
-        return FFDAS_ERROR_ALLOCATION_FAILED;
+    long long *start = nullptr, *cnt = nullptr;
+    int *list = nullptr;
+    void *tmp = nullptr;
+    size_t tmp_bytes = 0;
+    hipError_t e = rocprim::exclusive_scan(nullptr, tmp_bytes, cnt, start, 0ll, nb,
+                                           rocprim::plus<long long>(), st);
+    if (e == hipSuccess) e = hipMalloc((void **)&start, nb * sizeof(long long));
+    if (e == hipSuccess) e = hipMalloc((void **)&cnt, nb * sizeof(long long));
+    if (e == hipSuccess) e = hipMalloc(&tmp, std::max<size_t>(tmp_bytes, 1));
+    if (e == hipSuccess)
+        e = hipMalloc((void **)&list, (size_t)std::max<long long>(p.list_total, 1) * sizeof(int));
+    if (e == hipSuccess) {
+        const Box b = box_of(p);
+        const int zg = (int)std::min<int64_t>(4096, (kBins3 + 1 + 255) / 256);
+        hipLaunchKernelGGL(interp_zero_kernel, dim3(zg), dim3(256), 0, st, cnt, kBins3 + 1);
+        if (p.ntet > 0)
+            hipLaunchKernelGGL(interp_count_kernel, dim3(grid1(p.ntet)), dim3(256), 0, st, b,
+                               p.verts, p.ntet, (int)p.nx, (int)p.ny, cnt);
+        // the sentinel count is 0, so start[kBins3] = total
+        e = rocprim::exclusive_scan(tmp, tmp_bytes, cnt, start, 0ll, nb,
+                                    rocprim::plus<long long>(), st);
+        hipLaunchKernelGGL(interp_zero_kernel, dim3(zg), dim3(256), 0, st, cnt, kBins3 + 1);
+        if (e == hipSuccess && p.ntet > 0)
+            hipLaunchKernelGGL(interp_fill_kernel, dim3(grid1(p.ntet)), dim3(256), 0, st, b,
+                               p.verts, p.ntet, (int)p.nx, (int)p.ny, start, cnt, list);
+        if (e == hipSuccess) e = hipGetLastError();
+        const hipError_t es = hipStreamSynchronize(st);   // cnt and tmp are freed next
+        if (e == hipSuccess) e = es;
     }
+    if (cnt) (void)hipFree(cnt);
+    if (tmp) (void)hipFree(tmp);
+    if (e != hipSuccess) {
+        if (start) (void)hipFree(start);
+        if (list) (void)hipFree(list);
+        return e == hipErrorOutOfMemory ? FFDAS_ERROR_ALLOCATION_FAILED : hip_status(e);
+    }
+    p.bin_start = start;
+    p.bin_list = list;
     return FFDAS_SUCCESS;
 }
 
-template <typename R, int CW>
-ffdas_error_t evaluate(ffdas_context &h, int mode, const void *x, void *out, const int *idx,
-                       const float *w, int64_t n, int64_t B, int64_t npts, const void *fill) {
+// By cells unless the point ids do not fit an int or FFDAS_INTERP_LOCATE is "point".
+bool locate_by_cells(int64_t n) {
+    const char *how = std::getenv("FFDAS_INTERP_LOCATE");
+    return n < INT_MAX && !(how && std::string(how) == "point");
+}
+
+// Scratch of a location by cells, carved from one block.
+struct LocateScratch {
+    size_t pts = 0, best = 0, cnt = 0, start = 0, scan = 0, scan_bytes = 0, total = 0;
+    static ffdas_error_t plan(int64_t n, hipStream_t st, LocateScratch &s) {
+        const size_t nb = (size_t)kBins3 + 1;
+        int *none = nullptr;
+        if (rocprim::exclusive_scan(nullptr, s.scan_bytes, none, none, 0, nb, rocprim::plus<int>(),
+                                    st) != hipSuccess)
+            return FFDAS_ERROR_CUDA_LAUNCH_FAILED;
+        s.pts = 0;
+        s.best = s.pts + up256((size_t)n * sizeof(float4));
+        s.cnt = s.best + up256((size_t)n * sizeof(int));
+        s.start = s.cnt + up256(nb * sizeof(int));
+        s.scan = s.start + up256(nb * sizeof(int));
+        s.total = s.scan + up256(s.scan_bytes);
+        return FFDAS_SUCCESS;
+    }
+};
+
+// Locate n points into idx (and w): device buffers sized by the caller; `scratch` has the bytes
+// of LocateScratch for a location by cells.
+ffdas_error_t locate(ffdas_context &h, ffdas_interpolation_plan &p, const float *qp, int64_t n,
+                     int *idx, float *w, const LocateScratch &ls, void *scratch) {
+    hipStream_t st = h.stream;
+    const int nx = (int)p.nx, ny = (int)p.ny;
+    if (!scratch) {
+        FFDAS_TRY(build_lists(h, p));
+        ProfScope ps(st, "interp_locate");
+        hipLaunchKernelGGL(interp_locate_kernel, dim3(grid1(n)), dim3(256), 0, st, box_of(p),
+                           p.verts, nx, ny, p.ntet, p.bin_start, p.bin_list, qp, n, p.mode, idx, w);
+        return hip_status(hipGetLastError(), FFDAS_ERROR_CUDA_LAUNCH_FAILED);
+    }
+    char *c = static_cast<char *>(scratch);
+    float4 *pts = (float4 *)(c + ls.pts);
+    int *best = (int *)(c + ls.best), *cnt = (int *)(c + ls.cnt), *start = (int *)(c + ls.start);
+    const int64_t ncell = p.ntet / 6;
+    // Lanes per cell, from the points in the box of an average tetrahedron (its bins from the
+    // list total, the points per bin as if evenly spread): one lane for every six points, those
+    // of a run sharing it two points a lane.  Measured by lanes (runs x points): 9 points
+    // (256 x 64 x 64 vertices, 128^3 points) 0.59 ms 1 x 1, 0.55 2 x 1, 0.61 2 x 4; 99 points
+    // (128 x 32 x 32, 180^3) 2.84 ms 1 x 1, 0.98 4 x 4; 414 points (64 x 16 x 20, 180^3) 12.4 ms
+    // 1 x 1, 0.91 8 x 8; 0.2 points (400 x 90 x 90, 40^3) 0.44 ms 1 x 1, 0.53 4 x 1.
+    int lgr = 0, lgp = 0;
+    if (p.ntet > 0) {
+        const double bins = (double)p.list_total / (double)p.ntet, dens = (double)n / (double)kBins3;
+        const auto lg = [](double v) { return v > 1.0 ? (int)(std::log2(v) + 0.5) : 0; };
+        const int all = std::min(lg(bins * dens / 6.0), 6);
+        lgp = std::min(all, lg(std::cbrt(bins) * dens / 2.0));
+        lgr = all - lgp;
+    }
+    ProfScope ps(st, "interp_locate");
+    const Box b = box_of(p);
+    hipLaunchKernelGGL(interp_zero_i32_kernel, dim3(1024), dim3(256), 0, st, cnt, kBins3 + 1);
+    hipLaunchKernelGGL(interp_point_bin_kernel, dim3(grid1(n)), dim3(256), 0, st, b, qp, n, cnt, idx);
+    size_t scan_bytes = ls.scan_bytes;
+    if (rocprim::exclusive_scan(c + ls.scan, scan_bytes, cnt, start, 0, (size_t)kBins3 + 1,
+                                rocprim::plus<int>(), st) != hipSuccess)
+        return FFDAS_ERROR_CUDA_LAUNCH_FAILED;
+    hipLaunchKernelGGL(interp_point_order_kernel, dim3(grid1(n)), dim3(256), 0, st, b, qp, n, start,
+                       cnt, pts, best);
+    if (ncell > 0)
+        hipLaunchKernelGGL(interp_locate_cells_kernel, dim3(grid1(ncell << (lgr + lgp))), dim3(256), 0,
+                           st, b, p.verts, ncell, nx, ny, lgr, lgp, start, pts, best);
+    hipLaunchKernelGGL(interp_found_kernel, dim3(grid1(n)), dim3(256), 0, st, p.verts, nx, ny,
+                       start + kBins3, pts, best, p.mode, idx, w);
+    return hip_status(hipGetLastError(), FFDAS_ERROR_CUDA_LAUNCH_FAILED);
+}
+
+size_t lookup_ids(int64_t n) { return up256((size_t)n * sizeof(int)); }
+size_t lookup_weights(int mode, int64_t n) {
+    return mode == FFDAS_INTERP_NEAREST ? 0 : up256((size_t)n * 3 * sizeof(float));
+}
+
+// Frames per chunk: the smallest power of two that holds all, at most 64 bytes of 4-byte
+// elements and 8 frames of others (the 64-byte block a vertex load takes whole).
+int frames_per_chunk(int64_t B, size_t elem) {
+    const int most = elem == 4 ? 16 : 8;
+    int f = 1;
+    while (f < most && f < B) f *= 2;
+    return f;
+}
+
+// bytes of the frame-inner copy (one frame is read in place)
+size_t frames_bytes(int64_t B, int64_t npts, size_t elem) {
+    const int f = frames_per_chunk(B, elem);
+    return f == 1 ? 0 : (size_t)((B + f - 1) / f) * f * npts * elem;
+}
+
+template <typename R, int CW, int FPC>
+ffdas_error_t evaluate_f(ffdas_context &h, const ffdas_interpolation_plan &p, const void *x,
+                         void *out, const int *idx, const float *w, int64_t n, int64_t B,
+                         const El<R, CW> &f, void *ws) {
     using E = El<R, CW>;
-    using F = Frames<R, CW>;
-    E f;
-    for (int c = 0; c < CW; c++) f.c[c] = static_cast<const R *>(fill)[c];
-    constexpr int FPC = frames_per_chunk<R, CW>();
-    const int64_t chunks = (B + FPC - 1) / FPC;
-    // the frame-inner copy of x lives in the handle's workspace (which then no longer holds
-    // the converted x of an earlier delay-and-sum call)
-    void *ws = nullptr;
-    h.xcopy.valid = false;
-    FFDAS_TRY(h.workspace((size_t)chunks * npts * sizeof(F), &ws));
-    F *xfi = static_cast<F *>(ws);
-    {
+    using F = Frames<R, CW, FPC>;
+    const int64_t npts = p.nx * p.ny * p.nz, chunks = (B + FPC - 1) / FPC;
+    const F *xfi = static_cast<const F *>(x);
+    if (FPC > 1) {
         ProfScope ps(h.stream, "interp_frames");
-        hipLaunchKernelGGL((interp_frames_kernel<R, CW>), dim3(grid1(npts), (unsigned)chunks),
-                           dim3(256), 0, h.stream, static_cast<const E *>(x), xfi, npts, B);
+        hipLaunchKernelGGL((interp_frames_kernel<R, CW, FPC>), dim3(grid1(npts), (unsigned)chunks),
+                           dim3(256), 0, h.stream, static_cast<const E *>(x), static_cast<F *>(ws),
+                           npts, B);
+        xfi = static_cast<const F *>(ws);
     }
     const dim3 grid(grid1(n), (unsigned)chunks);
     ProfScope ps(h.stream, "interp_eval");
-    if (mode == FFDAS_INTERP_NEAREST)
-        hipLaunchKernelGGL((interp_nearest_kernel<R, CW>), grid, dim3(256), 0, h.stream, xfi,
+    if (p.mode == FFDAS_INTERP_NEAREST)
+        hipLaunchKernelGGL((interp_nearest_kernel<R, CW, FPC>), grid, dim3(256), 0, h.stream, xfi,
                            static_cast<E *>(out), idx, n, npts, B, f);
     else
-        hipLaunchKernelGGL((interp_linear_kernel<R, CW>), grid, dim3(256), 0, h.stream, xfi,
-                           static_cast<E *>(out), reinterpret_cast<const int4 *>(idx),
-                           reinterpret_cast<const float4 *>(w), n, npts, B, f);
+    {
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, grid, dim3(256), 0, h.stream, xfi, static_cast<E *>(out), idx,
+                               w, (int)p.nx, (int)p.ny, n, npts, B, f);
+        };
+        if (reinterpret_cast<uintptr_t>(out) % 128 == 0 && n * sizeof(E) % 128 == 0)
+            go(interp_linear_kernel<R, CW, FPC, true>);
+        else
+            go(interp_linear_kernel<R, CW, FPC, false>);
+    }
     return hip_status(hipGetLastError(), FFDAS_ERROR_CUDA_LAUNCH_FAILED);
+}
+
+template <typename R, int CW>
+ffdas_error_t evaluate(ffdas_context &h, const ffdas_interpolation_plan &p, const void *x, void *out,
+                       const int *idx, const float *w, int64_t n, int64_t B, const void *fill,
+                       void *ws) {
+    El<R, CW> f;
+    for (int c = 0; c < CW; c++) f.c[c] = static_cast<const R *>(fill)[c];
+    constexpr size_t elem = sizeof(R) * CW;
+    switch (frames_per_chunk(B, elem)) {
+        case 1: return evaluate_f<R, CW, 1>(h, p, x, out, idx, w, n, B, f, ws);
+        case 2: return evaluate_f<R, CW, 2>(h, p, x, out, idx, w, n, B, f, ws);
+        case 4: return evaluate_f<R, CW, 4>(h, p, x, out, idx, w, n, B, f, ws);
+        case 8: return evaluate_f<R, CW, 8>(h, p, x, out, idx, w, n, B, f, ws);
+        default:
+            if constexpr (elem == 4) return evaluate_f<R, CW, 16>(h, p, x, out, idx, w, n, B, f, ws);
+            return FFDAS_ERROR_INTERNAL;
+    }
 }
 
 ffdas_error_t build_plan(ffdas_context &h, ffdas_interpolation_plan &p, const float *gridpos) {
     const int64_t npts = p.nx * p.ny * p.nz;
     hipStream_t st = h.stream;
-    if (hipMalloc((void **)&p.verts, (size_t)npts * 3 * sizeof(float)) != hipSuccess)
+    if (hipMalloc((void **)&p.verts, (size_t)npts * sizeof(float4)) != hipSuccess)
         return FFDAS_ERROR_ALLOCATION_FAILED;
-    FFDAS_TRY(hip_status(hipMemcpyAsync(p.verts, gridpos, (size_t)npts * 3 * sizeof(float),
-                                        hipMemcpyDeviceToDevice, st),
-                         FFDAS_ERROR_CUDA_MEMCPY_FAILED));
-    if (hipMalloc((void **)&p.verts4, (size_t)npts * sizeof(float4)) != hipSuccess)
-        return FFDAS_ERROR_ALLOCATION_FAILED;
-    hipLaunchKernelGGL(interp_pad_kernel, dim3(grid1(npts)), dim3(256), 0, st, p.verts, npts,
-                       p.verts4);
-    // bounding box: per-block partials, finished on the host
-    const int nblk = (int)std::min<int64_t>(256, std::max<int64_t>(1, (npts + 255) / 256));
-    float *part = nullptr;
-    if (hipMalloc((void **)&part, (size_t)nblk * 6 * sizeof(float)) != hipSuccess)
-        return FFDAS_ERROR_ALLOCATION_FAILED;
-    hipLaunchKernelGGL(interp_bbox_kernel, dim3(nblk), dim3(256), 0, st, p.verts, npts, part);
-    std::vector<float> hp((size_t)nblk * 6);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(hp.data(), part, hp.size() * sizeof(float), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    (void)hipFree(part);
-    FFDAS_TRY(hip_status(e));
-    float mn[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, mx[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
-    for (int k = 0; k < nblk; k++)
-        for (int a = 0; a < 3; a++) {
-            mn[a] = std::min(mn[a], hp[k * 6 + a]);
-            mx[a] = std::max(mx[a], hp[k * 6 + 3 + a]);
-        }
-    for (int a = 0; a < 3; a++) {
-        p.bmin[a] = mn[a];
-        // the reference's scale, in FP32 (spatial_hash.cu:51-55)
-        volatile float ext = mx[a] - mn[a];
-        p.scale[a] = (float)(kBins - 1) / ext;
-    }
+    const int nblk = (int)std::min<int64_t>(1024, std::max<int64_t>(1, (npts + 255) / 256));
+    void *ws = nullptr;
+    const size_t head_bytes = up256(sizeof(PlanHead));
+    FFDAS_TRY(h.workspace(head_bytes + (size_t)nblk * 6 * sizeof(float), &ws));
+    h.xcopy.valid = false;   // the converted-x record of the delay-and-sum calls
+    PlanHead *head = static_cast<PlanHead *>(ws);
+    float *part = reinterpret_cast<float *>(static_cast<char *>(ws) + head_bytes);
+    hipLaunchKernelGGL(interp_verts_kernel, dim3(nblk), dim3(256), 0, st, gridpos, npts, p.verts, part);
+    hipLaunchKernelGGL(interp_box_kernel, dim3(1), dim3(64), 0, st, part, nblk, head);
     p.ntet = 6 * (p.nx - 1) * (p.ny - 1) * (p.nz - 1);
-    if (hipMalloc((void **)&p.bin_start, (size_t)(kBins3 + 1) * sizeof(long long)) != hipSuccess)
-        return FFDAS_ERROR_ALLOCATION_FAILED;
-    long long *cnt = nullptr;
-    if (hipMalloc((void **)&cnt, (size_t)(kBins3 + 1) * sizeof(long long)) != hipSuccess)
-        return FFDAS_ERROR_ALLOCATION_FAILED;
-    const Box b = box_of(p);
-    const int zg = (int)std::min<int64_t>(4096, (kBins3 + 1 + 255) / 256);
-    hipLaunchKernelGGL(interp_zero_kernel, dim3(zg), dim3(256), 0, st, cnt, kBins3 + 1);
     if (p.ntet > 0)
-        hipLaunchKernelGGL(interp_count_kernel, dim3(grid1(p.ntet)), dim3(256), 0, st, b, p.verts,
-                           p.ntet, (int)p.nx, (int)p.ny, cnt);
-    // exclusive scan of the counts (the sentinel count is 0, so start[kBins3] = total)
-    size_t tmp_bytes = 0;
-    e = rocprim::exclusive_scan(nullptr, tmp_bytes, cnt, p.bin_start, 0ll, (size_t)(kBins3 + 1),
-                                rocprim::plus<long long>(), st);
-    void *tmp = nullptr;
-    if (e == hipSuccess) e = hipMalloc(&tmp, tmp_bytes);
-    if (e == hipSuccess)
-        e = rocprim::exclusive_scan(tmp, tmp_bytes, cnt, p.bin_start, 0ll, (size_t)(kBins3 + 1),
-                                    rocprim::plus<long long>(), st);
-    long long total = 0;
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(&total, p.bin_start + kBins3, sizeof(long long), hipMemcpyDeviceToHost, st);
+        hipLaunchKernelGGL(interp_total_kernel, dim3(std::min(grid1(p.ntet / 6), 1024)), dim3(256), 0,
+                           st, p.verts, p.ntet / 6, (int)p.nx, (int)p.ny, head);
+    PlanHead hh{};
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpyAsync(&hh, head, sizeof(hh), hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (tmp) (void)hipFree(tmp);
-    if (e != hipSuccess) {
-        (void)hipFree(cnt);
-        return hip_status(e);
+    FFDAS_TRY(hip_status(e));
+    for (int a = 0; a < 3; a++) {
+        p.bmin[a] = hh.box.mn[a];
+        p.scale[a] = hh.box.sc[a];
     }
-    if (total > INT_MAX || p.ntet > INT_MAX) {
-        (void)hipFree(cnt);
-        return FFDAS_ERROR_DIMS_TOO_LARGE;
-    }
-    if (hipMalloc((void **)&p.bin_list, (size_t)std::max<long long>(total, 1) * sizeof(int)) != hipSuccess) {
-        (void)hipFree(cnt);
-        return FFDAS_ERROR_ALLOCATION_FAILED;
-    }
-    hipLaunchKernelGGL(interp_zero_kernel, dim3(zg), dim3(256), 0, st, cnt, kBins3 + 1);
-    if (p.ntet > 0)
-        hipLaunchKernelGGL(interp_fill_kernel, dim3(grid1(p.ntet)), dim3(256), 0, st, b, p.verts,
-                           p.ntet, (int)p.nx, (int)p.ny, p.bin_start, cnt, p.bin_list);
-    e = hipGetLastError();
-    if (e == hipSuccess) e = hipStreamSynchronize(st);   // cnt is freed next
-    (void)hipFree(cnt);
-    return hip_status(e, FFDAS_ERROR_CUDA_LAUNCH_FAILED);
+    // entries of a point-by-point location's lists
+    if (hh.total > (unsigned long long)INT_MAX || p.ntet > INT_MAX) return FFDAS_ERROR_DIMS_TOO_LARGE;
+    p.list_total = (long long)hh.total;
+    return FFDAS_SUCCESS;
 }
 
 }  // namespace
@@ -903,8 +1050,18 @@ static ffdas_error_t interpolation_preprocess_call(ffdas_handle_t handle,
     }
     plan->pre = false;
     plan->pre_n = 0;
-    FFDAS_TRY(alloc_lookup(plan->mode, num_querypos, &plan->pre_idx, &plan->pre_w));
-    FFDAS_TRY(locate(*handle, *plan, querypos, num_querypos, plan->pre_idx, plan->pre_w));
+    LocateScratch ls;
+    void *scratch = nullptr;
+    if (locate_by_cells(num_querypos)) {
+        FFDAS_TRY(LocateScratch::plan(num_querypos, handle->stream, ls));
+        FFDAS_TRY(handle->workspace(ls.total, &scratch));
+        handle->xcopy.valid = false;   // the converted-x record of the delay-and-sum calls
+    }
+    const size_t wb = lookup_weights(plan->mode, num_querypos);
+    if (hipMalloc((void **)&plan->pre_idx, lookup_ids(num_querypos)) != hipSuccess)
+        return FFDAS_ERROR_ALLOCATION_FAILED;
+    if (wb && hipMalloc((void **)&plan->pre_w, wb) != hipSuccess) return FFDAS_ERROR_ALLOCATION_FAILED;
+    FFDAS_TRY(locate(*handle, *plan, querypos, num_querypos, plan->pre_idx, plan->pre_w, ls, scratch));
     plan->pre = true;
     plan->pre_n = num_querypos;
     return FFDAS_SUCCESS;
@@ -945,35 +1102,46 @@ static ffdas_error_t interpolation_call(ffdas_handle_t handle, ffdas_interpolati
     if ((B + kFramesPerThread - 1) / kFramesPerThread > 65535) return FFDAS_ERROR_DIMS_TOO_LARGE;
     FFDAS_TRY(handle->check_device());
 
+    size_t elem;
+    switch (xd.dtype) {
+        case FFDAS_R_32F: elem = 4; break;
+        case FFDAS_C_32F: case FFDAS_R_64F: elem = 8; break;
+        case FFDAS_C_64F: elem = 16; break;
+        default: return FFDAS_ERROR_UNSUPPORTED_TYPE;
+    }
+    // One block of workspace: the one-shot lookup, then the location's scratch or, after it, the
+    // frame-inner copy of x.  Any converted x of a delay-and-sum call kept there is gone.
+    const bool cells = !use_pre && locate_by_cells(num_querypos);
+    if (!use_pre) {
+        // a location is not captured into a graph (preprocess first)
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(handle->stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone)
+            return FFDAS_ERROR_ALLOCATION_FAILED;
+    }
+    LocateScratch ls;
+    if (cells) FFDAS_TRY(LocateScratch::plan(num_querypos, handle->stream, ls));
+    const size_t ib = use_pre ? 0 : lookup_ids(num_querypos);
+    const size_t wb = use_pre ? 0 : lookup_weights(plan->mode, num_querypos);
+    void *ws = nullptr;
+    handle->xcopy.valid = false;
+    FFDAS_TRY(handle->workspace(ib + wb + std::max(ls.total, frames_bytes(B, bs, elem)), &ws));
+    char *c = static_cast<char *>(ws);
     const int *idx = plan->pre_idx;
     const float *w = plan->pre_w;
-    int *tidx = nullptr;
-    float *tw = nullptr;
+    void *rest = ws ? c + ib + wb : nullptr;
     if (!use_pre) {
-        FFDAS_TRY(alloc_lookup(plan->mode, num_querypos, &tidx, &tw));
-        const ffdas_error_t e = locate(*handle, *plan, querypos, num_querypos, tidx, tw);
-        if (e != FFDAS_SUCCESS) {
-            (void)hipFree(tidx);
-            if (tw) (void)hipFree(tw);
-            return e;
-        }
+        int *tidx = reinterpret_cast<int *>(c);
+        float *tw = wb ? reinterpret_cast<float *>(c + ib) : nullptr;
+        FFDAS_TRY(locate(*handle, *plan, querypos, num_querypos, tidx, tw, ls, cells ? rest : nullptr));
         idx = tidx;
         w = tw;
     }
     ffdas_error_t err;
     switch (xd.dtype) {
-        case FFDAS_R_32F: err = evaluate<float, 1>(*handle, plan->mode, x, out, idx, w, num_querypos, B, bs, fill_value); break;
-        case FFDAS_C_32F: err = evaluate<float, 2>(*handle, plan->mode, x, out, idx, w, num_querypos, B, bs, fill_value); break;
-        case FFDAS_R_64F: err = evaluate<double, 1>(*handle, plan->mode, x, out, idx, w, num_querypos, B, bs, fill_value); break;
-        case FFDAS_C_64F: err = evaluate<double, 2>(*handle, plan->mode, x, out, idx, w, num_querypos, B, bs, fill_value); break;
-        default: err = FFDAS_ERROR_UNSUPPORTED_TYPE;
-    }
-    if (tidx) {
-        // the one-shot lookup is freed once the evaluation that reads it has run
-        const hipError_t e = hipStreamSynchronize(handle->stream);
-        (void)hipFree(tidx);
-        if (tw) (void)hipFree(tw);
-        if (err == FFDAS_SUCCESS) err = hip_status(e, FFDAS_ERROR_CUDA_SYNC_FAILED);
+        case FFDAS_R_32F: err = evaluate<float, 1>(*handle, *plan, x, out, idx, w, num_querypos, B, fill_value, rest); break;
+        case FFDAS_C_32F: err = evaluate<float, 2>(*handle, *plan, x, out, idx, w, num_querypos, B, fill_value, rest); break;
+        case FFDAS_R_64F: err = evaluate<double, 1>(*handle, *plan, x, out, idx, w, num_querypos, B, fill_value, rest); break;
+        default: err = evaluate<double, 2>(*handle, *plan, x, out, idx, w, num_querypos, B, fill_value, rest); break;
     }
     return err;
 }
