@@ -258,8 +258,34 @@ struct Tiling {
     int A, H, W;        // spatial view (outer dims folded into A)
     int ta, th, tw;     // wave tile, ta*th*tw == 64
     int nta, nth, ntw;  // tile counts
-    int xcd;            // 1: blocks regrouped so that each XCD takes a contiguous range
+    int tiles;          // tiles a launch covers (flat: of the orientation with most)
+    int xcd;            // order of the blocks over the XCDs (xcd_order)
+    int flat;           // a volume whose tiles the kernel orients (oriented): the per mille that a
+                        // tile 2 thick costs more, and 4 thick, as p2 + 4096 * p4; 0: fixed tiles
+    int steep;          // oriented: the axis the tiles are thin along (0 A, 1 H, 2 W)
 };
+
+// The tile of a volume whose steep axis has n voxels and the other two u and v: thin along the
+// steep axis, unless the voxels that the tiles cover beyond the grid, and compute for nothing,
+// cost more than the thickness.  Returns t | u << 8 | v << 16 of the tile; *tiles gets their count.
+__host__ __device__ inline int flat_tile(int n, int u, int v, int flat, int64_t *tiles) {
+    const int cand[6] = {1 | 8 << 8 | 8 << 16,  1 | 4 << 8 | 16 << 16, 1 | 16 << 8 | 4 << 16,
+                         2 | 8 << 8 | 4 << 16,  2 | 4 << 8 | 8 << 16,  4 | 4 << 8 | 4 << 16};
+    int best = 0;
+    int64_t cost = 0;
+    for (int c = 0; c < 6; c++) {
+        const int t = cand[c] & 255, tu = (cand[c] >> 8) & 255, tv = cand[c] >> 16;
+        const int64_t count = (int64_t)((n + t - 1) / t) * ((u + tu - 1) / tu) * ((v + tv - 1) / tv);
+        const int extra = c == 0 ? 0 : c < 3 ? 5 : c < 5 ? flat & 4095 : flat >> 12;
+        const int64_t k = count * (1000 + extra);
+        if (c == 0 || k < cost) {
+            best = cand[c];
+            cost = k;
+            *tiles = count;
+        }
+    }
+    return best;
+}
 
 // Workgroups are dispatched to the eight XCDs in turn (linear block id mod 8).  With xcd
 // set, linear id b is read as block (b mod 8) * (nb / 8) + b / 8 of the grid's order, so the
@@ -281,13 +307,29 @@ __device__ __forceinline__ int xcd_chunk(int b, int nb, int q) {
     return round * 8 * q + ((i + round) & 7) * q + (i >> 3);
 }
 
+// The order of Tiling::xcd: 0 the hardware's, 1 contiguous ranges, more: chunks of so many blocks.
+__device__ __forceinline__ int xcd_order(int xcd, int b, int nb) {
+    return xcd == 0 ? b : xcd == 1 ? xcd_block(b, nb) : xcd_chunk(b, nb, xcd);
+}
+
 __device__ __forceinline__ int voxel_of(const Tiling &tl, int tile, int lane, bool &valid) {
     const int ntiles = tl.nta * tl.nth * tl.ntw;
     valid = tile < ntiles;
-    const int iw = tile % tl.ntw;
-    const int rest = tile / tl.ntw;
-    const int ih = rest % tl.nth;
-    const int ia = rest / tl.nth;
+    // tiles in the order (w, h, a); where w or h is the steep axis, it comes last
+    int ia, ih, iw;
+    if (tl.steep == 2) {
+        ih = tile % tl.nth;
+        const int rest = tile / tl.nth;
+        ia = rest % tl.nta;
+        iw = rest / tl.nta;
+    } else {
+        iw = tile % tl.ntw;
+        const int rest = tile / tl.ntw;
+        const int nin = tl.steep == 1 ? tl.nta : tl.nth;
+        const int in = rest % nin, out = rest / nin;
+        ih = tl.steep == 1 ? out : in;
+        ia = tl.steep == 1 ? in : out;
+    }
     const int lw = lane % tl.tw;
     const int lh = (lane / tl.tw) % tl.th;
     const int la = lane / (tl.tw * tl.th);
@@ -359,6 +401,41 @@ __device__ __forceinline__ void store_out(const AccT<ACC64> (&acc)[FT][CPLX ? 2 
             }
         }
     }
+}
+
+// A volume's tiles are thin along the axis whose step changes the receive distance most (depth,
+// first in the (z, y, x) grids of the examples, last in column-major callers'): the lanes of a
+// wave then read the narrowest window of each row.  Taken at the middle of the grid from the
+// middle channel; the sums do not depend on it.
+__device__ __forceinline__ Tiling oriented(Tiling tl, const Geo &g) {
+    tl.steep = 0;
+    if (!tl.flat) return tl;
+    const float *s = g.srcpos + 3 * (g.C / 2);
+    const auto r = [&](int a, int h, int w) {
+        const float *p = g.dstpos + 3 * (int64_t)((a * tl.H + h) * tl.W + w);
+        const float dx = p[0] - s[0], dy = p[1] - s[1], dz = p[2] - s[2];
+        return __builtin_sqrtf(dx * dx + dy * dy + dz * dz);
+    };
+    const int a = (tl.A - 1) / 2, h = (tl.H - 1) / 2, w = (tl.W - 1) / 2;   // each axis has a step
+    const float r0 = r(a, h, w);
+    const float da = __builtin_fabsf(r(a + 1, h, w) - r0), dh = __builtin_fabsf(r(a, h + 1, w) - r0),
+                dw = __builtin_fabsf(r(a, h, w + 1) - r0);
+    tl.steep = __builtin_amdgcn_readfirstlane(dw > da && dw >= dh ? 2 : dh > da ? 1 : 0);
+    int64_t count;
+    if (tl.steep == 0) {
+        const int c = flat_tile(tl.A, tl.H, tl.W, tl.flat, &count);
+        tl.ta = c & 255; tl.th = (c >> 8) & 255; tl.tw = c >> 16;
+    } else if (tl.steep == 1) {
+        const int c = flat_tile(tl.H, tl.A, tl.W, tl.flat, &count);
+        tl.th = c & 255; tl.ta = (c >> 8) & 255; tl.tw = c >> 16;
+    } else {
+        const int c = flat_tile(tl.W, tl.A, tl.H, tl.flat, &count);
+        tl.tw = c & 255; tl.ta = (c >> 8) & 255; tl.th = c >> 16;
+    }
+    tl.nta = (tl.A + tl.ta - 1) / tl.ta;
+    tl.nth = (tl.H + tl.th - 1) / tl.th;
+    tl.ntw = (tl.W + tl.tw - 1) / tl.tw;
+    return tl;
 }
 
 }  // namespace dev

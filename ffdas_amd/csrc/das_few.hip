@@ -76,7 +76,7 @@ __global__ __launch_bounds__(1024) void das_fwd_few_kernel(Geo g, Tiling tl,
         tile = b - chunk * gridDim.x;
     }
     bool valid;
-    int n = voxel_of(tl, tile, lane, valid);
+    int n = voxel_of(oriented(tl, g), tile, lane, valid);
     if (!valid) n = 0;          // computed, never stored: keeps every lane at the barrier
     const SplitPt yp = split_point(g.dstpos[3 * n], g.dstpos[3 * n + 1], g.dstpos[3 * n + 2]);
     const uint32_t last = (uint32_t)(g.S - 1);
@@ -294,7 +294,7 @@ template <Storage ST, bool CPLX, int FT>
 hipError_t launch_few_ft(hipStream_t st, const dev::Geo &g, const dev::Tiling &tl, const XView &xv,
                          void *out, int64_t os_b, double br, double bi) {
     constexpr int TB = tap_group<CPLX, FT>();
-    const int ntiles = tl.nta * tl.nth * tl.ntw;
+    const int ntiles = tl.tiles;
     dim3 grid(ntiles, (g.B + FT - 1) / FT);
     int G = 1;
     while (G < 16 && (int64_t)ntiles * grid.y * G < 8192 && 2 * G <= g.C) G *= 2;
@@ -329,21 +329,10 @@ bool few_frames_ok(const DasProblem &p, const XView &xv) {
     return span < 2147483648.0 - 64.0 && (!p.cplx || reinterpret_cast<uintptr_t>(xv.ptr) % 4 == 0);
 }
 
-hipError_t launch_forward_few(hipStream_t st, const dev::Geo &g, const dev::Tiling &tiling,
+hipError_t launch_forward_few(hipStream_t st, const dev::Geo &g, const dev::Tiling &tl,
                               const DasProblem &p, const XView &xv, void *out, double beta_re,
                               double beta_im) {
     const int64_t os_b = p.os_b;
-    dev::Tiling tl = tiling;
-    if (tl.ta > 1) {
-        // volumes: flat 2 x 8 x 4 tiles.  The delay grows fastest along the first dimension
-        // (depth in the (z, y, x) grids of the examples), so a flat tile reads a narrower
-        // window of each row: 128^3 volume 13.3 ms with 4 x 4 x 4, 11.7 ms with 2 x 8 x 4 and
-        // 1 x 8 x 8, of which the first also suits other orders of the dimensions.
-        tl.ta = 2; tl.th = 8; tl.tw = 4;
-        tl.nta = (tl.A + 1) / 2;
-        tl.nth = (tl.H + 7) / 8;
-        tl.ntw = (tl.W + 3) / 4;
-    }
     switch (p.k_storage) {
         case Storage::F16:
             return p.cplx ? launch_few_t<Storage::F16, true>(st, g, tl, xv, out, os_b, beta_re, beta_im)

@@ -381,22 +381,24 @@ __global__ __launch_bounds__(256) void das_fwd_kernel(Geo g, Tiling tl, const vo
     store_out<ACC64, CPLX, FT>(acc, outv, os_b, n, b0, g.B, beta_re, beta_im);
 }
 
-// frame-inner layout.  A workgroup of G waves shares one voxel tile; wave w sums channels
-// w, w+G, ... and the G partial sums are combined through LDS, so a launch has G times more
-// waves in flight than tiles (latency hiding for the gathers) without repeating any delay
-// arithmetic.
+// frame-inner layout.  G waves share one voxel tile; wave w sums channels w, w+G, ... and the G
+// partial sums are combined through LDS, so a launch has G times more waves in flight than
+// tiles (latency hiding for the gathers) without repeating any delay arithmetic.  A workgroup
+// holds one tile, or for sparse compounding the waves of several neighbouring ones, which
+// read the same rows of a channel at about the same time.
 template <Storage ST, bool ACC64, bool CPLX, bool PRECISE, int FT, int KC, int TB, bool PL>
 __device__ __forceinline__ void fwd_fi_tile(const Geo &g, const Tiling &tl, const void *xv,
                                             void *outv, int64_t os_b, double beta_re,
-                                            double beta_im, int tile, int chunk,
+                                            double beta_im, int block, int chunk, int G,
                                             unsigned char *lds) {
     using A = AccT<ACC64>;
     constexpr int CW = CPLX ? 2 : 1;
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int G = blockDim.x >> 6;
+    const int w0 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int own = w0 / G, wave = w0 - own * G;       // the workgroup's tile, its wave of G
+    const int tile = block * ((int)(blockDim.x >> 6) / G) + own;
     bool valid;
-    int n = voxel_of(tl, tile, lane, valid);
+    int n = voxel_of(oriented(tl, g), tile, lane, valid);
     if (!valid) n = 0;          // computed, never stored: keeps every lane at the barrier
     const FrameInnerRows<ST, FT, CW, PL> xr(xv, chunk, g.C, g.T, g.S);
     A acc[FT][CW];
@@ -409,7 +411,7 @@ __device__ __forceinline__ void fwd_fi_tile(const Geo &g, const Tiling &tl, cons
         return;
     }
     // red[w][i][lane], i = f * CW + c
-    A *red = reinterpret_cast<A *>(lds);
+    A *red = reinterpret_cast<A *>(lds) + own * G * FT * CW * 64;
 #pragma unroll
     for (int f = 0; f < FT; f++)
 #pragma unroll
@@ -442,20 +444,16 @@ __device__ __forceinline__ void fwd_fi_tile(const Geo &g, const Tiling &tl, cons
     }
 }
 
-// grid.x = voxel tile, grid.y = frame chunk
+// grid.x = workgroups of voxel tiles, grid.y = frame chunk
 template <Storage ST, bool ACC64, bool CPLX, bool PRECISE, int FT, int KC, int TB, bool PL>
 __global__ __launch_bounds__(512) void das_fwd_fi_kernel(Geo g, Tiling tl, const void *__restrict__ xv,
                                                          void *__restrict__ outv, int64_t os_b,
-                                                         double beta_re, double beta_im) {
+                                                         double beta_re, double beta_im, int G) {
     extern __shared__ unsigned char fwd_lds[];
-    int tile = blockIdx.x, chunk = blockIdx.y;
-    if (tl.xcd) {
-        const int b = xcd_block(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
-        chunk = b / gridDim.x;
-        tile = b - chunk * gridDim.x;
-    }
+    const int b = xcd_order(tl.xcd, blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+    const int chunk = b / gridDim.x, block = b - chunk * gridDim.x;
     fwd_fi_tile<ST, ACC64, CPLX, PRECISE, FT, KC, TB, PL>(g, tl, xv, outv, os_b, beta_re, beta_im,
-                                                       tile, chunk, fwd_lds);
+                                                       block, chunk, G, fwd_lds);
 }
 
 // Several problems (mixed probes, grids, frame counts, sparse tables) in one launch.  The
@@ -470,26 +468,27 @@ struct BatchItem {
     int64_t os_b;
     double beta_re, beta_im;
     int start;            // first block of the problem
-    int tiles;            // voxel tiles per frame chunk
+    int blocks;           // workgroups per frame chunk
 };
 struct BatchArgs {
     int count;
-    int xcd;              // regroup blocks by XCD (xcd_block)
+    int xcd;              // order of the blocks over the XCDs (xcd_order)
+    int G;                // waves per voxel tile
     BatchItem item[kMaxBatch];
 };
 
 template <Storage ST, bool CPLX, bool PRECISE, int FT, int KC, int TB, bool PL>
 __global__ __launch_bounds__(512) void das_fwd_fi_batched_kernel(BatchArgs args) {
     extern __shared__ unsigned char fwd_lds[];
-    const int b = args.xcd ? xcd_block(blockIdx.x, gridDim.x) : (int)blockIdx.x;
+    const int b = xcd_order(args.xcd, blockIdx.x, gridDim.x);
     int i = 0;
     while (i + 1 < args.count && b >= args.item[i + 1].start) i++;
     const BatchItem &it = args.item[i];
     const int local = b - it.start;
-    const int chunk = local / it.tiles;
+    const int chunk = local / it.blocks;
     fwd_fi_tile<ST, false, CPLX, PRECISE, FT, KC, TB, PL>(it.g, it.tl, it.x, it.out, it.os_b, it.beta_re,
-                                                   it.beta_im, local - chunk * it.tiles, chunk,
-                                                   fwd_lds);
+                                                   it.beta_im, local - chunk * it.blocks, chunk,
+                                                   args.G, fwd_lds);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -714,13 +713,13 @@ __global__ __launch_bounds__(512) void das_bwd_param_fi_kernel(
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int G = blockDim.x >> 6;
     int tile = blockIdx.x, chunk = blockIdx.y;
-    if (tl.xcd) {
-        const int b = xcd_block(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+    {
+        const int b = xcd_order(tl.xcd, blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
         chunk = b / gridDim.x;
         tile = b - chunk * gridDim.x;
     }
     bool valid;
-    int n = voxel_of(tl, tile, lane, valid);
+    int n = voxel_of(oriented(tl, g), tile, lane, valid);
     if (!valid) n = 0;          // computed, never stored: keeps every lane at the barriers
     const FrameInnerRows<ST, FT, CW, PL> xr(xv, chunk, g.C, g.T, g.S);
     float *go = gofs ? gofs + chunk * pstride : nullptr;
@@ -1827,6 +1826,12 @@ int frame_tile_for(int B) {
 // the frame-group planes: 2-D benchmark forward 0.198 -> 0.192 ms, parameter adjoint
 // 0.226 -> 0.223 ms; batched sparse compounding (mixed probes, HBM-bound) 575 -> 534 ms.
 // FFDAS_XCD=0 keeps the hardware's round-robin order.
+// Sparse compounding takes chunks instead (xcd_chunk): what a tile fetches changes over the grid,
+// and with whole eighths the XCDs finished at different times (64^3 voxels of 1024 channels in
+// flat tiles: 18.7 ms in eighths, 14.2 round-robin, 13.0 in chunks of 8).  Images keep the eighths
+// below 512 tiles (8 frames, 9 transmits: 468 tiles 199 us and 211 in chunks, 648 tiles 235 and 221).
+constexpr int kXcdSparse = 8;      // workgroups of a chunk
+
 bool xcd_groups() {
     static const bool on = [] {
         const char *env = std::getenv("FFDAS_XCD");
@@ -1835,9 +1840,15 @@ bool xcd_groups() {
     return on;
 }
 
-dev::Tiling make_tiling(const std::vector<int64_t> &spatial, const DasTune &tune = DasTune()) {
+// flat: the kernel orients a volume's tiles (dev::oriented).  Tiles 1, 2 and 4 voxels thick: one
+// frame of a 128^3 volume 11.7, 11.7 and 13.3 ms; sparse compounding of 64^3 voxels of 1024 channels
+// 12.4, 13.8 and 17.0 ms (with two small probes), the same whichever axis is depth (tiles thin
+// along the wrong one: 29 ms); eight dense frames a few per cent.  Sparse volumes that do not give
+// every CU a tile keep the cubes and the eighths (24^3 voxels 158 us, flat 164, in chunks 172; from
+// there on it is the other way round, 30^3 voxels 312 and 265).
+dev::Tiling make_tiling(const DasProblem &p, bool flat) {
     std::vector<int64_t> d;
-    for (int64_t v : spatial)
+    for (int64_t v : p.spatial)
         if (v > 1) d.push_back(v);
     dev::Tiling t{};
     t.A = 1; t.H = 1; t.W = 1;
@@ -1847,16 +1858,27 @@ dev::Tiling make_tiling(const std::vector<int64_t> &spatial, const DasTune &tune
     if (d.size() >= 3) { t.ta = 4; t.th = 4; t.tw = 4; }
     else if (d.size() == 2) {
         t.ta = 1; t.th = 8; t.tw = 8;
-        if (tune.tile_h > 0 && tune.tile_w > 0 && tune.tile_h * tune.tile_w == 64) {
-            t.th = tune.tile_h;
-            t.tw = tune.tile_w;
+        if (p.tune.tile_h > 0 && p.tune.tile_w > 0 && p.tune.tile_h * p.tune.tile_w == 64) {
+            t.th = p.tune.tile_h;
+            t.tw = p.tune.tile_w;
         }
     }
     else { t.ta = 1; t.th = 1; t.tw = 64; }
     t.nta = (t.A + t.ta - 1) / t.ta;
     t.nth = (t.H + t.th - 1) / t.th;
     t.ntw = (t.W + t.tw - 1) / t.tw;
-    t.xcd = xcd_groups() ? 1 : 0;
+    t.tiles = t.nta * t.nth * t.ntw;
+    if (flat && d.size() >= 3 && !(p.sparse && t.tiles < 256)) {
+        const int p2 = p.sparse ? 110 : 20, p4 = p.sparse ? 370 : p.fi_frames > 0 ? 50 : 130;
+        t.flat = p2 + 4096 * p4;
+        int64_t c[3];
+        dev::flat_tile(t.A, t.H, t.W, t.flat, &c[0]);
+        dev::flat_tile(t.H, t.A, t.W, t.flat, &c[1]);
+        dev::flat_tile(t.W, t.A, t.H, t.flat, &c[2]);
+        t.tiles = (int)std::max({c[0], c[1], c[2]});
+    }
+    const bool chunks = p.sparse && (t.flat || t.tiles >= 512);
+    t.xcd = !xcd_groups() ? 0 : chunks ? kXcdSparse : 1;
     return t;
 }
 
@@ -1888,6 +1910,20 @@ int channel_groups(const dev::Geo &g, int64_t tiles, int want) {
     return G;
 }
 
+// Waves per voxel tile and tiles per workgroup of the frame-inner forward.  Dense problems: one
+// tile a workgroup.  Sparse compounding: four waves of neighbouring tiles, which read a
+// channel's rows at about the same time (the mixed probes above, waves a tile x tiles: 2 x 1 13.6
+// ms, 2 x 2 12.4, 2 x 4 12.8, 8 x 1 12.4, 1 x 8 13.2).
+struct Waves {
+    int G, tiles;
+};
+Waves forward_waves(int C, int64_t tiles, int want, bool sparse) {
+    dev::Geo g{};
+    g.C = C;
+    const int G = channel_groups(g, tiles, want);
+    return {G, sparse ? std::max(1, 4 / G) : 1};
+}
+
 dev::Geo make_geo(const DasGeomArgs &a, const DasProblem &p) {
     dev::Geo g{};
     g.srcpos = a.srcpos; g.srcdir = a.srcdir; g.dstpos = a.dstpos;
@@ -1905,7 +1941,7 @@ template <Storage ST, bool ACC64, bool CPLX, int FT>
 hipError_t launch_fwd_ft(hipStream_t st, const dev::Geo &g, const dev::Tiling &tl, const XView &xv,
                          void *out, int64_t os_b, double br, double bi) {
     constexpr bool PRECISE = true;
-    const int ntiles = tl.nta * tl.nth * tl.ntw;
+    const int ntiles = tl.tiles;
     dim3 grid((ntiles + 3) / 4, (g.B + FT - 1) / FT);
     ProfScope ps(st, "das_fwd");
     dev::das_fwd_kernel<ST, ACC64, CPLX, PRECISE, FT, kKC><<<grid, 256, 0, st>>>(
@@ -1948,7 +1984,7 @@ template <Storage ST, bool ACC64, bool CPLX, int FT>
 hipError_t launch_bwdp_ft(hipStream_t st, const dev::Geo &g, const dev::Tiling &tl,
                           const XView &xv, const void *gout, int64_t gs_b, const ParamOut &po) {
     constexpr bool PRECISE = true;
-    const int ntiles = tl.nta * tl.nth * tl.ntw;
+    const int ntiles = tl.tiles;
     dim3 grid((ntiles + 3) / 4, (g.B + FT - 1) / FT);
     const bool multi = grid.y > 1;
     const int64_t kn = (int64_t)g.K * g.N;
@@ -1987,7 +2023,7 @@ size_t bwdx_lds_bytes(int S, int FS, bool cplx, bool acc64) {
 template <bool ACC64, bool CPLX, bool PRECISE, int FT>
 hipError_t launch_bwdx_plain_ft(hipStream_t st, const dev::Geo &g, const dev::Tiling &tl,
                                 const void *gout, int64_t gs_b, void *gx) {
-    const int ntiles = tl.nta * tl.nth * tl.ntw;
+    const int ntiles = tl.tiles;
     dim3 grid((ntiles + 3) / 4, (g.B + FT - 1) / FT);
     const int64_t gx_t = g.S, gx_c = (int64_t)g.T * g.S, gx_b = (int64_t)g.C * g.T * g.S;
     ProfScope ps(st, "das_bwd_x_plain");
@@ -2166,16 +2202,16 @@ hipError_t launch_fwd_fi_f(hipStream_t st, const dev::Geo &g, const dev::Tiling 
         return hipErrorInvalidValue;
     } else {
         constexpr bool PRECISE = true;
-        const int ntiles = tl.nta * tl.nth * tl.ntw;
-        dim3 grid(ntiles, (g.B + F - 1) / F);
-        const int G = channel_groups(g, (int64_t)grid.x * grid.y, groups);
-        const size_t lds = G > 1 ? (size_t)G * F * (CPLX ? 2 : 1) * 64 * sizeof(float) : 0;
+        const int ntiles = tl.tiles, chunks = (g.B + F - 1) / F;
+        const Waves w = forward_waves(g.C, (int64_t)ntiles * chunks, groups, g.sparse != nullptr);
+        const dim3 grid((ntiles + w.tiles - 1) / w.tiles, chunks);
+        const size_t lds = w.G > 1 ? (size_t)w.G * w.tiles * F * (CPLX ? 2 : 1) * 64 * sizeof(float) : 0;
         auto go = [&](auto kern) {
             if (lds > 0)
                 (void)hipFuncSetAttribute((const void *)kern,
                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
             ProfScope ps(st, "das_fwd_fi");
-            kern<<<grid, 64 * G, lds, st>>>(g, tl, x, out, os_b, br, bi);
+            kern<<<grid, 64 * w.G * w.tiles, lds, st>>>(g, tl, x, out, os_b, br, bi, w.G);
             return hipGetLastError();
         };
         auto by_taps = [&](auto pl) {
@@ -2209,7 +2245,7 @@ hipError_t launch_bwdp_fi_f(hipStream_t st, const dev::Geo &g, const dev::Tiling
         return hipErrorInvalidValue;
     } else {
         constexpr bool PRECISE = true;
-        const int ntiles = tl.nta * tl.nth * tl.ntw;
+        const int ntiles = tl.tiles;
         dim3 grid(ntiles, (g.B + F - 1) / F);
         const int G = channel_groups(g, (int64_t)grid.x * grid.y, groups);
         const size_t lds = G > 1 ? (size_t)G * 2 * kKC * 64 * sizeof(float) : 0;
@@ -2252,44 +2288,46 @@ hipError_t launch_fwd_batched_f(hipStream_t st, const std::vector<BatchMember> &
         for (size_t off = 0; off < ms.size(); off += dev::kMaxBatch) {
             dev::BatchArgs args{};
             const int n = (int)std::min(ms.size() - off, (size_t)dev::kMaxBatch);
-            int64_t start = 0;
+            // the members of one launch share the layout, so all are sparse or none is
+            const bool sparse = ms[off].p.sparse;
+            int64_t tiles = 0;
             int minC = 1 << 30;
-            int want = 0;
+            for (int i = 0; i < n; i++) {
+                const BatchMember &m = ms[off + i];
+                args.item[i].tl = make_tiling(m.p, true);
+                const dev::Tiling &tl = args.item[i].tl;
+                tiles += (int64_t)tl.tiles * ((m.p.B + F - 1) / F);
+                minC = std::min(minC, m.p.C);
+            }
+            const Waves w = forward_waves(minC, tiles, ms[off].p.tune.groups, sparse);
+            int64_t start = 0;
             for (int i = 0; i < n; i++) {
                 const BatchMember &m = ms[off + i];
                 dev::BatchItem &it = args.item[i];
                 it.g = make_geo(m.a, m.p);
-                it.tl = make_tiling(m.p.spatial, m.p.tune);
-                const int tiles = it.tl.nta * it.tl.nth * it.tl.ntw;
-                const int chunks = (m.p.B + F - 1) / F;
                 it.x = m.xfi;
                 it.out = m.out;
                 it.os_b = m.p.os_b;
                 it.beta_re = m.beta_re;
                 it.beta_im = m.beta_im;
                 it.start = (int)start;
-                it.tiles = tiles;
-                start += (int64_t)tiles * chunks;
-                minC = std::min(minC, m.p.C);
-                if (i == 0) want = m.p.tune.groups;
+                it.blocks = (it.tl.tiles + w.tiles - 1) / w.tiles;
+                start += (int64_t)it.blocks * ((m.p.B + F - 1) / F);
+                if (start > 0x7fffffff) return hipErrorInvalidValue;
             }
             args.count = n;
-            args.xcd = xcd_groups() ? 1 : 0;
+            for (int i = 0; i < n; i++) args.xcd = std::max(args.xcd, args.item[i].tl.xcd);
+            args.G = w.G;
             if (start == 0) continue;
-            if (start > 0x7fffffff) return hipErrorInvalidValue;
-            dev::Geo gc{};
-            gc.C = minC;
-            const int G = channel_groups(gc, start, want);
-            const size_t lds = G > 1 ? (size_t)G * F * (CPLX ? 2 : 1) * 64 * sizeof(float) : 0;
+            const size_t lds = w.G > 1 ? (size_t)w.G * w.tiles * F * (CPLX ? 2 : 1) * 64 * sizeof(float) : 0;
             auto go = [&](auto kern) {
                 if (lds > 0)
                     (void)hipFuncSetAttribute((const void *)kern,
                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
                 ProfScope ps(st, "das_fwd_fi_batched");
-                kern<<<(unsigned)start, 64 * G, lds, st>>>(args);
+                kern<<<(unsigned)start, 64 * w.G * w.tiles, lds, st>>>(args);
                 return hipGetLastError();
             };
-            // the members of one launch share the layout (the caller groups them so)
             auto by_taps = [&](auto pl) {
                 constexpr bool PL = decltype(pl)::value;
                 const int tb = tap_group<ST, CPLX>();
@@ -2457,7 +2495,8 @@ ffdas_error_t launch_forward_batched(ffdas_context &h, const std::vector<BatchMe
 ffdas_error_t launch_forward(ffdas_context &h, const DasProblem &p, const DasGeomArgs &a,
                              const XView &xv, void *out, double beta_re, double beta_im) {
     const dev::Geo g = make_geo(a, p);
-    const dev::Tiling tl = make_tiling(p.spatial, p.tune);
+    const bool few = p.fi_frames <= 0 && few_frames_ok(p, xv);
+    const dev::Tiling tl = make_tiling(p, p.fi_frames > 0 || few);
     hipError_t e = hipSuccess;
     hipStream_t st = h.stream;
     const int64_t os_b = p.os_b;
@@ -2579,8 +2618,8 @@ struct ParamLayout {
 size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 ParamLayout param_layout(const DasProblem &p, bool has_o, bool has_w, bool has_s) {
     ParamLayout L;
-    const dev::Tiling tl = make_tiling(p.spatial, p.tune);
-    const int ntiles = tl.nta * tl.nth * tl.ntw;
+    const dev::Tiling tl = make_tiling(p, p.fi_frames > 0);
+    const int ntiles = tl.tiles;
     const int FT = p.fi_frames > 0 ? p.fi_frames : frame_tile_for(p.B);
     L.chunks = (p.B + FT - 1) / FT;
     L.blocks = (p.fi_frames > 0 ? ntiles : (ntiles + 3) / 4) * L.chunks;
@@ -2618,7 +2657,7 @@ ffdas_error_t launch_backward(ffdas_context &h, const DasProblem &p, const DasGe
                               const XView &xv, const void *gout, int64_t gs_b, void *gx,
                               float *gofs, float *gwt, float *gscale, void *gt, void *pws) {
     const dev::Geo g = make_geo(a, p);
-    const dev::Tiling tl = make_tiling(p.spatial, p.tune);
+    const dev::Tiling tl = make_tiling(p, p.fi_frames > 0);
     hipStream_t st = h.stream;
     hipError_t e = hipSuccess;
 
