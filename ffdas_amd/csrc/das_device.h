@@ -258,33 +258,33 @@ struct Tiling {
     int A, H, W;        // spatial view (outer dims folded into A)
     int ta, th, tw;     // wave tile, ta*th*tw == 64
     int nta, nth, ntw;  // tile counts
-    int tiles;          // tiles a launch covers (flat: of the orientation with most)
+    int tiles;          // tiles a launch covers (flat: of the shape with most)
     int xcd;            // order of the blocks over the XCDs (xcd_order)
-    int flat;           // a volume whose tiles the kernel orients (oriented): the per mille that a
-                        // tile 2 thick costs more, and 4 thick, as p2 + 4096 * p4; 0: fixed tiles
+    float flat;         // a volume whose tiles the kernel shapes (oriented): the cost of a tap
+                        // beside its window, in samples of window; 0: fixed tiles
     int steep;          // oriented: the axis the tiles are thin along (0 A, 1 H, 2 W)
 };
 
-// The tile of a volume whose steep axis has n voxels and the other two u and v: thin along the
-// steep axis, unless the voxels that the tiles cover beyond the grid, and compute for nothing,
-// cost more than the thickness.  Returns t | u << 8 | v << 16 of the tile; *tiles gets their count.
-__host__ __device__ inline int flat_tile(int n, int u, int v, int flat, int64_t *tiles) {
-    const int cand[6] = {1 | 8 << 8 | 8 << 16,  1 | 4 << 8 | 16 << 16, 1 | 16 << 8 | 4 << 16,
-                         2 | 8 << 8 | 4 << 16,  2 | 4 << 8 | 8 << 16,  4 | 4 << 8 | 4 << 16};
-    int best = 0;
-    int64_t cost = 0;
-    for (int c = 0; c < 6; c++) {
-        const int t = cand[c] & 255, tu = (cand[c] >> 8) & 255, tv = cand[c] >> 16;
-        const int64_t count = (int64_t)((n + t - 1) / t) * ((u + tu - 1) / tu) * ((v + tv - 1) / tv);
-        const int extra = c == 0 ? 0 : c < 3 ? 5 : c < 5 ? flat & 4095 : flat >> 12;
-        const int64_t k = count * (1000 + extra);
-        if (c == 0 || k < cost) {
-            best = cand[c];
-            cost = k;
-            *tiles = count;
-        }
+// Tiles of a volume whose steep axis has n voxels and the other two u and v, as log2 of the edges
+// ln | lu << 4 | lv << 8, and their count.
+constexpr int kFlatTiles = 6;
+__host__ __device__ inline int flat_shape(int c) {
+    constexpr int shape[kFlatTiles] = {0x330, 0x420, 0x240, 0x231, 0x321, 0x222};
+    return shape[c];
+}
+__host__ __device__ inline int64_t flat_count(int shape, int n, int u, int v) {
+    const int ln = shape & 15, lu = (shape >> 4) & 15, lv = shape >> 8;
+    return (int64_t)((n + (1 << ln) - 1) >> ln) * ((u + (1 << lu) - 1) >> lu) *
+           ((v + (1 << lv) - 1) >> lv);
+}
+// Shapes with more tiles than a sixteenth above the fewest compute too many voxels beyond the grid.
+__host__ __device__ inline int64_t flat_limit(int n, int u, int v) {
+    int64_t least = flat_count(flat_shape(0), n, u, v);
+    for (int c = 1; c < kFlatTiles; c++) {
+        const int64_t k = flat_count(flat_shape(c), n, u, v);
+        least = k < least ? k : least;
     }
-    return best;
+    return least + least / 16;
 }
 
 // Workgroups are dispatched to the eight XCDs in turn (linear block id mod 8).  With xcd
@@ -403,35 +403,67 @@ __device__ __forceinline__ void store_out(const AccT<ACC64> (&acc)[FT][CPLX ? 2 
     }
 }
 
-// A volume's tiles are thin along the axis whose step changes the receive distance most (depth,
-// first in the (z, y, x) grids of the examples, last in column-major callers'): the lanes of a
-// wave then read the narrowest window of each row.  Taken at the middle of the grid from the
-// middle channel; the sums do not depend on it.
+// The shape of a volume's tiles: the one whose taps cost least, a tap costing tl.flat and the window
+// of samples that the lanes of a wave read of a row, which is what the steps along the three axes
+// change the delay by, taken as the mean over 16 pairs of a channel and a voxel, one a lane (within
+// 6 per cent of the mean over all; 64 pairs are 64 cache lines a load, 15 us of a 530 us image).  The
+// axis of the largest step (depth, first in the (z, y, x) grids of the examples, last in
+// column-major callers') is walked last.  Every wave finds the same; the sums do not depend on it.
 __device__ __forceinline__ Tiling oriented(Tiling tl, const Geo &g) {
     tl.steep = 0;
-    if (!tl.flat) return tl;
-    const float *s = g.srcpos + 3 * (g.C / 2);
-    const auto r = [&](int a, int h, int w) {
-        const float *p = g.dstpos + 3 * (int64_t)((a * tl.H + h) * tl.W + w);
-        const float dx = p[0] - s[0], dy = p[1] - s[1], dz = p[2] - s[2];
-        return __builtin_sqrtf(dx * dx + dy * dy + dz * dz);
-    };
-    const int a = (tl.A - 1) / 2, h = (tl.H - 1) / 2, w = (tl.W - 1) / 2;   // each axis has a step
-    const float r0 = r(a, h, w);
-    const float da = __builtin_fabsf(r(a + 1, h, w) - r0), dh = __builtin_fabsf(r(a, h + 1, w) - r0),
-                dw = __builtin_fabsf(r(a, h, w + 1) - r0);
-    tl.steep = __builtin_amdgcn_readfirstlane(dw > da && dw >= dh ? 2 : dh > da ? 1 : 0);
-    int64_t count;
-    if (tl.steep == 0) {
-        const int c = flat_tile(tl.A, tl.H, tl.W, tl.flat, &count);
-        tl.ta = c & 255; tl.th = (c >> 8) & 255; tl.tw = c >> 16;
-    } else if (tl.steep == 1) {
-        const int c = flat_tile(tl.H, tl.A, tl.W, tl.flat, &count);
-        tl.th = c & 255; tl.ta = (c >> 8) & 255; tl.tw = c >> 16;
-    } else {
-        const int c = flat_tile(tl.W, tl.A, tl.H, tl.flat, &count);
-        tl.tw = c & 255; tl.ta = (c >> 8) & 255; tl.th = c >> 16;
+    if (tl.flat == 0.0f) return tl;
+    const int lane = threadIdx.x & 63;
+    float da = 0.0f, dh = 0.0f, dw = 0.0f;
+    if (lane < 16) {
+        const float *s = g.srcpos + 3 * (int)((int64_t)(2 * ((5 * lane + 5) & 15) + 1) * g.C >> 5);
+        const int a = (int)((int64_t)(2 * ((13 * lane + 3) & 15) + 1) * (tl.A - 1) >> 5),
+                  h = (int)((int64_t)(2 * (lane & 3) + 1) * (tl.H - 1) >> 3),
+                  w = (int)((int64_t)(2 * (lane >> 2) + 1) * (tl.W - 1) >> 3);   // each has a next
+        const auto tau = [&](int64_t n) {
+            const float *p = g.dstpos + 3 * n;
+            const float dx = p[0] - s[0], dy = p[1] - s[1], dz = p[2] - s[2];
+            // neighbours compound different transmits where the problem is sparse
+            return __builtin_sqrtf(dx * dx + dy * dy + dz * dz) + (g.sparse ? 0.0f : g.offsets[n]);
+        };
+        const int64_t n = ((int64_t)a * tl.H + h) * tl.W + w;
+        const float t0 = tau(n);
+        da = __builtin_fabsf(tau(n + (int64_t)tl.H * tl.W) - t0);
+        dh = __builtin_fabsf(tau(n + tl.W) - t0);
+        dw = __builtin_fabsf(tau(n + 1) - t0);
     }
+    const auto sum = [](float v) {
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+        return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+    };
+    da = sum(da);
+    dh = sum(dh);
+    dw = sum(dw);
+    tl.steep = dw > da && dw >= dh ? 2 : dh > da ? 1 : 0;
+    const int size = tl.steep == 0 ? tl.A : tl.steep == 1 ? tl.H : tl.W;
+    const int u = tl.steep == 0 ? tl.H : tl.A, v = tl.steep == 2 ? tl.H : tl.W;
+    const float ds = tl.steep == 0 ? da : tl.steep == 1 ? dh : dw;
+    const float du = tl.steep == 0 ? dh : da, dv = tl.steep == 2 ? dh : dw;
+    const int64_t limit = flat_limit(size, u, v);
+    int best = -1;
+    float cost = 0.0f;
+    for (int c = 0; c < kFlatTiles; c++) {
+        const int shape = flat_shape(c);
+        const int64_t count = flat_count(shape, size, u, v);
+        if (count > limit) continue;
+        const float window = (float)((1 << (shape & 15)) - 1) * ds +
+                             (float)((1 << ((shape >> 4) & 15)) - 1) * du +
+                             (float)((1 << (shape >> 8)) - 1) * dv;
+        const float k = (float)count * (16.0f * tl.flat + window);
+        if (best < 0 || k < cost) {
+            best = shape;
+            cost = k;
+        }
+    }
+    const int e0 = 1 << (best & 15), e1 = 1 << ((best >> 4) & 15), e2 = 1 << (best >> 8);
+    tl.ta = tl.steep == 0 ? e0 : e1;
+    tl.th = tl.steep == 1 ? e0 : tl.steep == 0 ? e1 : e2;
+    tl.tw = tl.steep == 2 ? e0 : e2;
     tl.nta = (tl.A + tl.ta - 1) / tl.ta;
     tl.nth = (tl.H + tl.th - 1) / tl.th;
     tl.ntw = (tl.W + tl.tw - 1) / tl.tw;

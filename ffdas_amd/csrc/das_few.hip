@@ -76,7 +76,9 @@ __global__ __launch_bounds__(1024) void das_fwd_few_kernel(Geo g, Tiling tl,
         tile = b - chunk * gridDim.x;
     }
     bool valid;
-    int n = voxel_of(oriented(tl, g), tile, lane, valid);
+    const Tiling ot = oriented(tl, g);
+    if (tile >= ot.nta * ot.nth * ot.ntw) return;            // the whole workgroup
+    int n = voxel_of(ot, tile, lane, valid);
     if (!valid) n = 0;          // computed, never stored: keeps every lane at the barrier
     const SplitPt yp = split_point(g.dstpos[3 * n], g.dstpos[3 * n + 1], g.dstpos[3 * n + 2]);
     const uint32_t last = (uint32_t)(g.S - 1);

@@ -398,7 +398,9 @@ __device__ __forceinline__ void fwd_fi_tile(const Geo &g, const Tiling &tl, cons
     const int own = w0 / G, wave = w0 - own * G;       // the workgroup's tile, its wave of G
     const int tile = block * ((int)(blockDim.x >> 6) / G) + own;
     bool valid;
-    int n = voxel_of(oriented(tl, g), tile, lane, valid);
+    const Tiling ot = oriented(tl, g);
+    if (tile - own >= ot.nta * ot.nth * ot.ntw) return;      // the workgroup has no tile
+    int n = voxel_of(ot, tile, lane, valid);
     if (!valid) n = 0;          // computed, never stored: keeps every lane at the barrier
     const FrameInnerRows<ST, FT, CW, PL> xr(xv, chunk, g.C, g.T, g.S);
     A acc[FT][CW];
@@ -1840,12 +1842,17 @@ bool xcd_groups() {
     return on;
 }
 
-// flat: the kernel orients a volume's tiles (dev::oriented).  Tiles 1, 2 and 4 voxels thick: one
-// frame of a 128^3 volume 11.7, 11.7 and 13.3 ms; sparse compounding of 64^3 voxels of 1024 channels
-// 12.4, 13.8 and 17.0 ms (with two small probes), the same whichever axis is depth (tiles thin
-// along the wrong one: 29 ms); eight dense frames a few per cent.  Sparse volumes that do not give
-// every CU a tile keep the cubes and the eighths (24^3 voxels 158 us, flat 164, in chunks 172; from
-// there on it is the other way round, 30^3 voxels 312 and 265).
+// flat: the kernel shapes a volume's tiles (dev::oriented), thin along depth where a step there
+// changes the delay much more than one across.  Cubes against the shape it finds, 1024 channels,
+// 64^3 voxels, four transmits: eight frames in FP16 1941 and 1715 us, in FP32 4870 and 3920, complex
+// 12.6 and 9.0 ms; one frame of 128^3 voxels, 16 transmits, 13.3 and 11.3 ms; sparse compounding
+// (with two small probes) 17.0 and 12.4 ms, the same whichever axis is depth (tiles thin along the
+// wrong one: 29 ms).  Where depth steps are half the lateral ones it keeps cubes, which are then
+// the better (50 x 40 x 40, complex: 1203 us, tiles 1 thick 1657).  The cost of a tap beside its
+// window (Tiling::flat) is what those times give: large for few frames, whose taps are few bytes,
+// small where the lines it fetches are what it waits for.  Sparse volumes that do not give every CU a tile keep the
+// cubes and the eighths (24^3 voxels 158 us, flat 164, in chunks 172; from there on it is the other
+// way round, 30^3 voxels 312 and 265).
 dev::Tiling make_tiling(const DasProblem &p, bool flat) {
     std::vector<int64_t> d;
     for (int64_t v : p.spatial)
@@ -1868,16 +1875,20 @@ dev::Tiling make_tiling(const DasProblem &p, bool flat) {
     t.nth = (t.H + t.th - 1) / t.th;
     t.ntw = (t.W + t.tw - 1) / t.tw;
     t.tiles = t.nta * t.nth * t.ntw;
-    if (flat && d.size() >= 3 && !(p.sparse && t.tiles < 256)) {
-        const int p2 = p.sparse ? 110 : 20, p4 = p.sparse ? 370 : p.fi_frames > 0 ? 50 : 130;
-        t.flat = p2 + 4096 * p4;
-        int64_t c[3];
-        dev::flat_tile(t.A, t.H, t.W, t.flat, &c[0]);
-        dev::flat_tile(t.H, t.A, t.W, t.flat, &c[1]);
-        dev::flat_tile(t.W, t.A, t.H, t.flat, &c[2]);
-        t.tiles = (int)std::max({c[0], c[1], c[2]});
+    if (flat && d.size() >= 3 && p.C > 0 && p.K > 0 && !(p.sparse && t.tiles < 256)) {
+        t.flat = p.sparse ? 70.0f : p.fi_frames > 0 ? 32.0f : 300.0f;
+        const int size[3][3] = {{t.A, t.H, t.W}, {t.H, t.A, t.W}, {t.W, t.A, t.H}};
+        int64_t most = 0;
+        for (const auto &n : size) {
+            const int64_t limit = dev::flat_limit(n[0], n[1], n[2]);
+            for (int c = 0; c < dev::kFlatTiles; c++) {
+                const int64_t k = dev::flat_count(dev::flat_shape(c), n[0], n[1], n[2]);
+                if (k <= limit) most = std::max(most, k);
+            }
+        }
+        t.tiles = (int)most;
     }
-    const bool chunks = p.sparse && (t.flat || t.tiles >= 512);
+    const bool chunks = p.sparse && (t.flat > 0.0f || t.tiles >= 512);
     t.xcd = !xcd_groups() ? 0 : chunks ? kXcdSparse : 1;
     return t;
 }
