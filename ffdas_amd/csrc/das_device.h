@@ -251,6 +251,25 @@ __device__ __forceinline__ void phase(float rev_h, float rev_l, const Tap &tp, f
     }
 }
 
+// The same for one term h + l of a delay, rounded once: the phase of a tap is a product of two of
+// these, and with what rounding u to FP32 drops put back (first order) the product is as good as
+// the sine and cosine of the whole.
+__device__ __forceinline__ void phase_term(float rev_h, float rev_l, float h, float l, float &s, float &c) {
+#pragma clang fp contract(off)
+    const float p = rev_h * h;
+    const float pe = __builtin_fmaf(rev_h, h, -p);
+    const float a = p - __builtin_rintf(p);                         // exact
+    const float b = pe + __builtin_fmaf(rev_l, h, (rev_h + rev_l) * l);
+    float u = a + b;
+    const float bp = u - a;
+    const float e = ((a - (u - bp)) + (b - bp)) * 6.283185307179586f;   // the rest, in radians
+    u -= __builtin_rintf(u);                                        // exact
+    float sn, cs;
+    sincos_rev_poly(u, sn, cs);
+    s = __builtin_fmaf(cs, e, sn);
+    c = __builtin_fmaf(-sn, e, cs);
+}
+
 // ---------------------------------------------------------------------------------------
 // voxel tiling: a wave covers a compact (ta x th x tw) tile of the (A, H, W) voxel grid
 // ---------------------------------------------------------------------------------------

@@ -109,7 +109,7 @@ __global__ __launch_bounds__(1024) void das_fwd_few_kernel(Geo g, Tiling tl,
 
     for (int kc = 0; kc < g.K && g.S >= 2; kc += KC) {
         int64_t ofs[KC];            // scale * offset, 32.32
-        float wt[KC];
+        float wt[KC], wi[CPLX ? KC : 1];   // complex: the weight times e^{i wavenum scale offset}
         uint32_t rowoff[SPARSE ? KC : 1];
         bool plainly = true;
 #pragma unroll
@@ -117,6 +117,7 @@ __global__ __launch_bounds__(1024) void das_fwd_few_kernel(Geo g, Tiling tl,
             const int jj = kc + j;
             ofs[j] = (int64_t)kFixedNone << 32;
             wt[j] = 0.0f;
+            if constexpr (CPLX) wi[j] = 0.0f;
             if constexpr (SPARSE) rowoff[j] = 0;
             if (jj < g.K) {
                 const int64_t o = (int64_t)jj * g.N + n;
@@ -133,8 +134,16 @@ __global__ __launch_bounds__(1024) void das_fwd_few_kernel(Geo g, Tiling tl,
                 const bool good = __builtin_fabsf(h) < kFixedLimit &&
                                   (aw == 0.0f || (aw > 1e-27f && aw < 3e38f));
                 if (any && good) ofs[j] = to_fixed(h, l);
+                else wt[j] = 0.0f;                       // it meets zeros: no NaN from it
                 if (any && !good) plainly = false;
-                if constexpr (!CPLX) wt[j] *= 2.3283064365386963e-10f;    // 2^-32
+                if constexpr (!CPLX) {
+                    wt[j] *= 2.3283064365386963e-10f;    // 2^-32
+                } else {
+                    float sn, cs;
+                    phase_term(g.rev_h, g.rev_l, any && good ? h : 0.0f, l, sn, cs);
+                    wi[j] = wt[j] * sn;
+                    wt[j] *= cs;
+                }
             }
         }
         const bool fixed_slots = __builtin_amdgcn_ballot_w64(!plainly) == 0;
@@ -185,6 +194,8 @@ __global__ __launch_bounds__(1024) void das_fwd_few_kernel(Geo g, Tiling tl,
             }
             int64_t rf = to_fixed(rh, rl);
             if (!dok) rf = (int64_t)kFixedNone << 32;
+            float sr = 0.0f, cr = 1.0f;
+            if constexpr (CPLX) phase_term(g.rev_h, g.rev_l, rh, rl, sr, cr);
             __amdgpu_buffer_rsrc_t rows[FT];
 #pragma unroll
             for (int f = 0; f < FT; f++)
@@ -218,15 +229,11 @@ __global__ __launch_bounds__(1024) void das_fwd_few_kernel(Geo g, Tiling tl,
                         for (int f = 0; f < FT; f++)
                             add(f, q[u][f], wt[j], tf, 4294967296.0f, 0.0f, 0.0f);
                     } else {
-                        const uint32_t k = (uint32_t)(tau[u] >> 32);
-                        Tap tp;
-                        tp.kf = k < last ? (float)(int)k : 0.0f;
-                        tp.t = tf * 2.3283064365386963e-10f;
-                        float sn, cs;
-                        phase<true>(g.rev_h, g.rev_l, tp, sn, cs);
+                        // the slot's rotation times the channel's: no sine or cosine a tap
+                        const float sn = wt[j] * sr + wi[j] * cr, cs = wt[j] * cr - wi[j] * sr;
 #pragma unroll
                         for (int f = 0; f < FT; f++)
-                            add(f, q[u][f], 0.0f, 0.0f, tp.t, wt[j] * sn, wt[j] * cs);
+                            add(f, q[u][f], 0.0f, 0.0f, tf * 2.3283064365386963e-10f, sn, cs);
                     }
                 }
             };
