@@ -7,6 +7,7 @@
 #include <cstdint>
 #include <type_traits>
 
+#include "das_index.h"
 #include "internal.h"
 
 namespace ffdas {
@@ -178,36 +179,6 @@ __device__ __forceinline__ Tap make_tap(float ofs, const Radius &R, float scale)
 }
 
 // ---------------------------------------------------------------------------------------
-// delays in 32.32 fixed point
-// ---------------------------------------------------------------------------------------
-// tau = scale * ofs + scale * r is a sum of one term per (voxel, slot) and one per (voxel,
-// channel).  With both terms in 32.32 fixed point the sum of a tap is one 64-bit integer
-// addition whose high word is floor(tau) and whose low word is the fraction, where the
-// floating-point form needs about fifteen operations (TwoSum, scale, two floors) for each
-// tap.  The terms carry the compensated pairs to within 2^-31 of a sample, below the FP32
-// rounding of the fraction that follows either way.
-constexpr float kFixedLimit = 4194304.0f;      // |term| < 2^22: its low part fits 31 bits
-constexpr int kFixedNone = 0x40000000;         // high word of a term that selects no sample
-
-// h + l (|h| < 2^22, |l| <= ulp(h)) as 32.32 fixed point.
-__device__ __forceinline__ int64_t to_fixed(float h, float l) {
-#pragma clang fp contract(off)
-    const float f = __builtin_floorf(h);
-    const uint32_t lo = (uint32_t)((h - f) * 4294967296.0f);           // saturates at 2^32 - 1
-    const int li = (int)__builtin_rintf(l * 4294967296.0f);
-    return (((int64_t)(int)f << 32) | lo) + (int64_t)li;
-}
-
-// scale * (h + l) as a float pair; exact for scale == 1.
-__device__ __forceinline__ void scale_pair(float scale, float &h, float &l) {
-#pragma clang fp contract(off)
-    const float sh = scale * h;
-    const float sl = __builtin_fmaf(scale, h, -sh);
-    l = __builtin_fmaf(scale, l, sl);
-    h = sh;
-}
-
-// ---------------------------------------------------------------------------------------
 // phase rotation e^{i wavenum tau}
 // ---------------------------------------------------------------------------------------
 // sin/cos of 2*pi*u for |u| <= 0.5 by quadrant reduction and Taylor polynomials on
@@ -268,93 +239,6 @@ __device__ __forceinline__ void phase_term(float rev_h, float rev_l, float h, fl
     sincos_rev_poly(u, sn, cs);
     s = __builtin_fmaf(cs, e, sn);
     c = __builtin_fmaf(-sn, e, cs);
-}
-
-// ---------------------------------------------------------------------------------------
-// voxel tiling: a wave covers a compact (ta x th x tw) tile of the (A, H, W) voxel grid
-// ---------------------------------------------------------------------------------------
-struct Tiling {
-    int A, H, W;        // spatial view (outer dims folded into A)
-    int ta, th, tw;     // wave tile, ta*th*tw == 64
-    int nta, nth, ntw;  // tile counts
-    int tiles;          // tiles a launch covers (flat: of the shape with most)
-    int xcd;            // order of the blocks over the XCDs (xcd_order)
-    float flat;         // a volume whose tiles the kernel shapes (oriented): the cost of a tap
-                        // beside its window, in samples of window; 0: fixed tiles
-    int steep;          // oriented: the axis the tiles are thin along (0 A, 1 H, 2 W)
-};
-
-// Tiles of a volume whose steep axis has n voxels and the other two u and v, as log2 of the edges
-// ln | lu << 4 | lv << 8, and their count.
-constexpr int kFlatTiles = 6;
-__host__ __device__ inline int flat_shape(int c) {
-    constexpr int shape[kFlatTiles] = {0x330, 0x420, 0x240, 0x231, 0x321, 0x222};
-    return shape[c];
-}
-__host__ __device__ inline int64_t flat_count(int shape, int n, int u, int v) {
-    const int ln = shape & 15, lu = (shape >> 4) & 15, lv = shape >> 8;
-    return (int64_t)((n + (1 << ln) - 1) >> ln) * ((u + (1 << lu) - 1) >> lu) *
-           ((v + (1 << lv) - 1) >> lv);
-}
-// Shapes with more tiles than a sixteenth above the fewest compute too many voxels beyond the grid.
-__host__ __device__ inline int64_t flat_limit(int n, int u, int v) {
-    int64_t least = flat_count(flat_shape(0), n, u, v);
-    for (int c = 1; c < kFlatTiles; c++) {
-        const int64_t k = flat_count(flat_shape(c), n, u, v);
-        least = k < least ? k : least;
-    }
-    return least + least / 16;
-}
-
-// Workgroups are dispatched to the eight XCDs in turn (linear block id mod 8).  With xcd
-// set, linear id b is read as block (b mod 8) * (nb / 8) + b / 8 of the grid's order, so the
-// blocks of one XCD form a contiguous range of tiles and share that XCD's L2.  A bijection
-// on the complete rounds of 8; the last nb mod 8 blocks keep their ids.
-__device__ __forceinline__ int xcd_block(int b, int nb) {
-    const int full = nb & ~7;
-    if (b >= full) return b;
-    return (b & 7) * (full >> 3) + (b >> 3);
-}
-
-// The same in chunks of q tiles: each XCD still works on neighbouring tiles, but regions whose
-// tiles cost less (channels outside their cones are passed over) are shared out over all of
-// them.  The chunk an XCD takes moves on by one each round of 8, so that a period in the grid
-// does not give one XCD the cheap tiles every time.  A bijection on the complete rounds.
-__device__ __forceinline__ int xcd_chunk(int b, int nb, int q) {
-    const int round = b / (8 * q), i = b - round * 8 * q;
-    if ((round + 1) * 8 * q > nb) return b;
-    return round * 8 * q + ((i + round) & 7) * q + (i >> 3);
-}
-
-// The order of Tiling::xcd: 0 the hardware's, 1 contiguous ranges, more: chunks of so many blocks.
-__device__ __forceinline__ int xcd_order(int xcd, int b, int nb) {
-    return xcd == 0 ? b : xcd == 1 ? xcd_block(b, nb) : xcd_chunk(b, nb, xcd);
-}
-
-__device__ __forceinline__ int voxel_of(const Tiling &tl, int tile, int lane, bool &valid) {
-    const int ntiles = tl.nta * tl.nth * tl.ntw;
-    valid = tile < ntiles;
-    // tiles in the order (w, h, a); where w or h is the steep axis, it comes last
-    int ia, ih, iw;
-    if (tl.steep == 2) {
-        ih = tile % tl.nth;
-        const int rest = tile / tl.nth;
-        ia = rest % tl.nta;
-        iw = rest / tl.nta;
-    } else {
-        iw = tile % tl.ntw;
-        const int rest = tile / tl.ntw;
-        const int nin = tl.steep == 1 ? tl.nta : tl.nth;
-        const int in = rest % nin, out = rest / nin;
-        ih = tl.steep == 1 ? out : in;
-        ia = tl.steep == 1 ? in : out;
-    }
-    const int lw = lane % tl.tw;
-    const int lh = (lane / tl.tw) % tl.th;
-    const int la = lane / (tl.tw * tl.th);
-    const int w = iw * tl.tw + lw, h = ih * tl.th + lh, a = ia * tl.ta + la;
-    valid = valid && w < tl.W && h < tl.H && a < tl.A;
-    return (a * tl.H + h) * tl.W + w;
 }
 
 // Axial voxel order for the channel-row scatter: the spatial grid is viewed as (D0, R) with
@@ -422,12 +306,9 @@ __device__ __forceinline__ void store_out(const AccT<ACC64> (&acc)[FT][CPLX ? 2 
     }
 }
 
-// The shape of a volume's tiles: the one whose taps cost least, a tap costing tl.flat and the window
-// of samples that the lanes of a wave read of a row, which is what the steps along the three axes
-// change the delay by, taken as the mean over 16 pairs of a channel and a voxel, one a lane (within
-// 6 per cent of the mean over all; 64 pairs are 64 cache lines a load, 15 us of a 530 us image).  The
-// axis of the largest step (depth, first in the (z, y, x) grids of the examples, last in
-// column-major callers') is walked last.  Every wave finds the same; the sums do not depend on it.
+// The shape of a volume's tiles (shaped), from the mean steps of the delay over 16 pairs of a channel
+// and a voxel, one a lane (within 6 per cent of the mean over all; 64 pairs are 64 cache lines a
+// load, 15 us of a 530 us image).  Every wave finds the same; the sums do not depend on it.
 __device__ __forceinline__ Tiling oriented(Tiling tl, const Geo &g) {
     tl.steep = 0;
     if (tl.flat == 0.0f) return tl;
@@ -455,38 +336,7 @@ __device__ __forceinline__ Tiling oriented(Tiling tl, const Geo &g) {
         for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
         return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
     };
-    da = sum(da);
-    dh = sum(dh);
-    dw = sum(dw);
-    tl.steep = dw > da && dw >= dh ? 2 : dh > da ? 1 : 0;
-    const int size = tl.steep == 0 ? tl.A : tl.steep == 1 ? tl.H : tl.W;
-    const int u = tl.steep == 0 ? tl.H : tl.A, v = tl.steep == 2 ? tl.H : tl.W;
-    const float ds = tl.steep == 0 ? da : tl.steep == 1 ? dh : dw;
-    const float du = tl.steep == 0 ? dh : da, dv = tl.steep == 2 ? dh : dw;
-    const int64_t limit = flat_limit(size, u, v);
-    int best = -1;
-    float cost = 0.0f;
-    for (int c = 0; c < kFlatTiles; c++) {
-        const int shape = flat_shape(c);
-        const int64_t count = flat_count(shape, size, u, v);
-        if (count > limit) continue;
-        const float window = (float)((1 << (shape & 15)) - 1) * ds +
-                             (float)((1 << ((shape >> 4) & 15)) - 1) * du +
-                             (float)((1 << (shape >> 8)) - 1) * dv;
-        const float k = (float)count * (16.0f * tl.flat + window);
-        if (best < 0 || k < cost) {
-            best = shape;
-            cost = k;
-        }
-    }
-    const int e0 = 1 << (best & 15), e1 = 1 << ((best >> 4) & 15), e2 = 1 << (best >> 8);
-    tl.ta = tl.steep == 0 ? e0 : e1;
-    tl.th = tl.steep == 1 ? e0 : tl.steep == 0 ? e1 : e2;
-    tl.tw = tl.steep == 2 ? e0 : e2;
-    tl.nta = (tl.A + tl.ta - 1) / tl.ta;
-    tl.nth = (tl.H + tl.th - 1) / tl.th;
-    tl.ntw = (tl.W + tl.tw - 1) / tl.tw;
-    return tl;
+    return shaped(tl, sum(da), sum(dh), sum(dw));
 }
 
 }  // namespace dev

@@ -505,7 +505,7 @@ __device__ __forceinline__ void das_fwd_body_iq(const Geo &g, const FrameInnerRo
                     const uint32_t k = (uint32_t)(tau[u] >> 32);
                     uint32_t off = k * (uint32_t)Rows::RB;
                     if constexpr (SPARSE) off += row[j];
-                    xr.fetch_at(rows, k < last ? off : kNoRows, q[u], SPARSE ? 0 : (kc + j) * (int)step);
+                    xr.fetch_at(rows, k < last ? off : kNoRows, q[u], SPARSE ? 0 : slot_offset(kc + j, g.K, (int)step));
                 }
                 // keep the group's loads ahead of their first use
                 __builtin_amdgcn_sched_barrier(0);
@@ -2040,16 +2040,7 @@ dev::Tiling make_tiling(const DasProblem &p, bool flat) {
     t.tiles = t.nta * t.nth * t.ntw;
     if (flat && d.size() >= 3 && p.C > 0 && p.K > 0 && !(p.sparse && t.tiles < 256)) {
         t.flat = p.sparse ? 70.0f : p.fi_frames > 0 ? 32.0f : 300.0f;
-        const int size[3][3] = {{t.A, t.H, t.W}, {t.H, t.A, t.W}, {t.W, t.A, t.H}};
-        int64_t most = 0;
-        for (const auto &n : size) {
-            const int64_t limit = dev::flat_limit(n[0], n[1], n[2]);
-            for (int c = 0; c < dev::kFlatTiles; c++) {
-                const int64_t k = dev::flat_count(dev::flat_shape(c), n[0], n[1], n[2]);
-                if (k <= limit) most = std::max(most, k);
-            }
-        }
-        t.tiles = (int)most;
+        t.tiles = (int)dev::flat_most(t.A, t.H, t.W);
     }
     const bool chunks = p.sparse && (t.flat > 0.0f || t.tiles >= 512);
     t.xcd = !xcd_groups() ? 0 : chunks ? kXcdSparse : 1;

@@ -1,0 +1,91 @@
+// Host UndefinedBehaviorSanitizer run of the delay-and-sum kernels' own index arithmetic
+// (ffdas_amd/csrc/das_index.h).  Exit status 0 and no sanitizer report is the pass condition.
+#include <cmath>
+#include <cstdio>
+#include <cstdlib>
+#include <vector>
+
+#include "das_index.h"
+
+using namespace ffdas::dev;
+
+#define CHECK(c)                                                       \
+    do {                                                               \
+        if (!(c)) {                                                    \
+            std::printf("%s:%d: %s\n", __FILE__, __LINE__, #c);        \
+            std::exit(1);                                              \
+        }                                                              \
+    } while (0)
+
+// Every scalar offset of a round of slots stays inside the channel's block of K transmits.
+static long slots() {
+    long n = 0;
+    for (int KC : {8, 16})
+        for (int TB : {1, 2, 4})
+            for (int K = 1; K <= 40; K++)
+                for (int kc = 0; kc < K; kc += KC)
+                    for (int j0 = 0; j0 < KC && kc + j0 < K; j0 += TB)
+                        for (int u = 0; u < TB; u++) {
+                            const int step = 1 << 20, j = kc + j0 + u;
+                            const int at = slot_offset(j, K, step);
+                            CHECK(at >= 0 && at <= (K - 1) * step);
+                            CHECK(j >= K || at == j * step);
+                            n++;
+                        }
+    return n;
+}
+
+// Every voxel is in exactly one tile of the shape the kernels choose, within the tiles launched.
+static long tiles() {
+    long n = 0;
+    const int grids[][3] = {{2, 2, 2}, {9, 5, 7}, {3, 17, 2}, {2, 3, 33}, {33, 3, 2}, {5, 16, 33},
+                            {33, 30, 29}, {64, 20, 17}, {17, 1, 5}};
+    const float steps[] = {0.0f, 0.4f, 3.0f, 40.0f, NAN};
+    for (const auto &s : grids)
+        for (float flat : {32.0f, 70.0f, 300.0f})
+            for (float da : steps)
+                for (float dh : steps)
+                    for (float dw : steps) {
+                        Tiling t{};
+                        t.A = s[0]; t.H = s[1]; t.W = s[2];
+                        t.flat = flat;
+                        t = shaped(t, da, dh, dw);
+                        const int count = t.nta * t.nth * t.ntw;
+                        CHECK(t.ta * t.th * t.tw == 64);
+                        CHECK(count <= flat_most(t.A, t.H, t.W));
+                        std::vector<int> seen((size_t)t.A * t.H * t.W, 0);
+                        for (int b = 0; b < count + 3; b++)
+                            for (int lane = 0; lane < 64; lane++) {
+                                bool valid;
+                                const int v = voxel_of(t, b, lane, valid);
+                                if (!valid) continue;
+                                CHECK(v >= 0 && v < (int)seen.size());
+                                seen[v]++;
+                            }
+                        for (int v : seen) CHECK(v == 1);
+                        n++;
+                    }
+    return n;
+}
+
+// The orders of the blocks over the XCDs are bijections, partial last rounds included.
+static long orders() {
+    long n = 0;
+    for (int nb = 1; nb < 1200; nb += 1 + nb / 40)
+        for (int xcd : {0, 1, 8, 64}) {
+            std::vector<int> seen(nb, 0);
+            for (int b = 0; b < nb; b++) {
+                const int to = xcd_order(xcd, b, nb);
+                CHECK(to >= 0 && to < nb);
+                seen[to]++;
+            }
+            for (int v : seen) CHECK(v == 1);
+            n++;
+        }
+    return n;
+}
+
+int main() {
+    std::printf("slots %ld, tiles %ld, orders %ld: index arithmetic clean\n", slots(), tiles(), orders());
+    return 0;
+}
