@@ -456,6 +456,15 @@ __global__ __launch_bounds__(256) void interp_point_order_kernel(
     best[e] = INT_MAX;
 }
 
+// Orders the LDS accesses of a wave's lanes among one another: what they wrote before is read after,
+// and what they read before is overwritten after.  The hardware keeps them in order; this keeps the
+// compiler from moving them.
+__device__ __forceinline__ void wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // 2^(lgr + lgp) lanes per cell: 2^lgr share out the runs of its box, 2^lgp the points of a run.
 // The points inside a cell's box are few and come to the lanes at different times, so they are
 // put on a queue of the wave, and the tests, most of the work, run with a queued point in
@@ -547,9 +556,12 @@ __global__ __launch_bounds__(256) void interp_locate_cells_kernel(
                                                       __builtin_amdgcn_mbcnt_lo((unsigned)hits, 0))] =
                     int2{base, at};
             waiting += __popcll(hits);
+            wave_order();
             if (waiting >= 64) {
                 waiting -= 64;
-                test(q[waiting + lane]);
+                const int2 c = q[waiting + lane];
+                wave_order();
+                test(c);
             }
         }
         if (__ballot(live) == 0) break;

@@ -45,6 +45,24 @@ def test_cells_match_point_scan(dev, monkeypatch, shape, n, mode):
         assert (cells != 7.5).float().mean() > 0.2
 
 
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 127, 128, 129, 4097, 50000])
+def test_queue_fills_and_drains(dev, monkeypatch, n):
+    """Two cells in turn: the lanes of a wave queue none, some or all of their points a step, across
+    the queue's own length."""
+    import torch
+    import ffdas_amd
+    rng = np.random.default_rng(n)
+    z, y, x = np.meshgrid([0., 1.], [0., 1.], [0., 1., 2.], indexing="ij")
+    g = np.stack([x, y, z + 0.3 * x], -1).astype(np.float32)       # sheared: half the box is empty
+    q = rng.uniform([0, 0, 0], [2, 1, 1.6], (n, 3)).astype(np.float32)
+    q[::3, 0] = rng.uniform(0.4, 0.6, len(q[::3]))
+    t = lambda a: torch.from_numpy(a).to(dev)
+    v = t(rng.standard_normal(g.shape[:3]).astype(np.float32))
+    cells = ffdas_amd.interpolate(t(g), v, t(q), fill=7.5)
+    monkeypatch.setenv("FFDAS_INTERP_LOCATE", "point")
+    assert torch.equal(cells, ffdas_amd.interpolate(t(g), v, t(q), fill=7.5))
+
+
 @pytest.mark.parametrize("dtype", ["float32", "complex64", "float64", "complex128"])
 @pytest.mark.parametrize("frames", [1, 2, 3, 4, 5, 8, 9, 16, 17])
 @pytest.mark.parametrize("n", [64, 5001])          # rows of whole cache lines, and not
