@@ -11,8 +11,8 @@
 // or one vertex id (nearest).
 // Evaluation (per call, the per-frame part): x is first copied frame-inner (the frames of a
 // chunk, up to 16 for 4-byte data and 8 otherwise, contiguous per vertex; one frame is read as it
-// is), so one thread per query point fetches each of its vertices' chunk with one vector load;
-// its lookup is read once per chunk; out is packed.
+// is where the output does not overlap it), so one thread per query point fetches each of its
+// vertices' chunk with one vector load; its lookup is read once per chunk; out is packed.
 #include <hip/hip_runtime.h>
 
 #include <cstring>   // before rocPRIM, whose iterators use memset
@@ -906,21 +906,24 @@ int frames_per_chunk(int64_t B, size_t elem) {
     return f;
 }
 
-// bytes of the frame-inner copy (one frame is read in place)
-size_t frames_bytes(int64_t B, int64_t npts, size_t elem) {
+// Bytes of the frame-inner copy.  One frame is read where it is, unless the output overlaps it (a
+// call that warps a volume in place): every value of x is read before any output is written.
+size_t frames_bytes(int64_t B, int64_t npts, size_t elem, const void *x, const void *out, int64_t n) {
     const int f = frames_per_chunk(B, elem);
-    return f == 1 ? 0 : (size_t)((B + f - 1) / f) * f * npts * elem;
+    const uintptr_t a = reinterpret_cast<uintptr_t>(x), b = reinterpret_cast<uintptr_t>(out);
+    if (f == 1 && (a + (size_t)npts * elem <= b || b + (size_t)n * elem <= a)) return 0;
+    return (size_t)((B + f - 1) / f) * f * npts * elem;
 }
 
 template <typename R, int CW, int FPC>
 ffdas_error_t evaluate_f(ffdas_context &h, const ffdas_interpolation_plan &p, const void *x,
                          void *out, const int *idx, const float *w, int64_t n, int64_t B,
-                         const El<R, CW> &f, void *ws) {
+                         const El<R, CW> &f, void *ws) {   // ws: the frame-inner copy, or null
     using E = El<R, CW>;
     using F = Frames<R, CW, FPC>;
     const int64_t npts = p.nx * p.ny * p.nz, chunks = (B + FPC - 1) / FPC;
     const F *xfi = static_cast<const F *>(x);
-    if (FPC > 1) {
+    if (ws) {
         ProfScope ps(h.stream, "interp_frames");
         hipLaunchKernelGGL((interp_frames_kernel<R, CW, FPC>), dim3(grid1(npts), (unsigned)chunks),
                            dim3(256), 0, h.stream, static_cast<const E *>(x), static_cast<F *>(ws),
@@ -1136,7 +1139,8 @@ static ffdas_error_t interpolation_call(ffdas_handle_t handle, ffdas_interpolati
     const size_t wb = use_pre ? 0 : lookup_weights(plan->mode, num_querypos);
     void *ws = nullptr;
     handle->xcopy.valid = false;
-    FFDAS_TRY(handle->workspace(ib + wb + std::max(ls.total, frames_bytes(B, bs, elem)), &ws));
+    const size_t fb = frames_bytes(B, bs, elem, x, out, num_querypos);
+    FFDAS_TRY(handle->workspace(ib + wb + std::max(ls.total, fb), &ws));
     char *c = static_cast<char *>(ws);
     const int *idx = plan->pre_idx;
     const float *w = plan->pre_w;
@@ -1148,12 +1152,13 @@ static ffdas_error_t interpolation_call(ffdas_handle_t handle, ffdas_interpolati
         idx = tidx;
         w = tw;
     }
+    void *frames = fb ? rest : nullptr;
     ffdas_error_t err;
     switch (xd.dtype) {
-        case FFDAS_R_32F: err = evaluate<float, 1>(*handle, *plan, x, out, idx, w, num_querypos, B, fill_value, rest); break;
-        case FFDAS_C_32F: err = evaluate<float, 2>(*handle, *plan, x, out, idx, w, num_querypos, B, fill_value, rest); break;
-        case FFDAS_R_64F: err = evaluate<double, 1>(*handle, *plan, x, out, idx, w, num_querypos, B, fill_value, rest); break;
-        default: err = evaluate<double, 2>(*handle, *plan, x, out, idx, w, num_querypos, B, fill_value, rest); break;
+        case FFDAS_R_32F: err = evaluate<float, 1>(*handle, *plan, x, out, idx, w, num_querypos, B, fill_value, frames); break;
+        case FFDAS_C_32F: err = evaluate<float, 2>(*handle, *plan, x, out, idx, w, num_querypos, B, fill_value, frames); break;
+        case FFDAS_R_64F: err = evaluate<double, 1>(*handle, *plan, x, out, idx, w, num_querypos, B, fill_value, frames); break;
+        default: err = evaluate<double, 2>(*handle, *plan, x, out, idx, w, num_querypos, B, fill_value, frames); break;
     }
     return err;
 }

@@ -85,3 +85,29 @@ def test_frame_chunks_match_single_frames(dev, dtype, frames, n, mode):
     view = buf[1:].view(frames, n)
     plan(xt, q, fill=-3.0, out=view)
     assert torch.equal(view, ref) and buf[0] == 5.0
+
+
+@pytest.mark.parametrize("frames", [1, 2, 16])
+@pytest.mark.parametrize("mode", ["linear", "nearest"])
+@pytest.mark.parametrize("kept", [True, False])
+@pytest.mark.parametrize("shift", [0, 100])
+def test_output_over_the_input(dev, frames, mode, kept, shift):
+    """A volume warped in place, wholly or partly: every value is read before it is overwritten."""
+    import torch
+    import ffdas_amd
+    rng = np.random.default_rng(frames + shift)
+    nz, ny, nx = 40, 41, 42
+    z, y, x = np.meshgrid(np.arange(nz), np.arange(ny), np.arange(nx), indexing="ij")
+    g = np.stack([x, y, z], -1).astype(np.float32)
+    q = g[::-1, ::-1, ::-1].copy()                      # each point reads the far end of the volume
+    t = lambda a: torch.from_numpy(a).to(dev)
+    v = t(rng.standard_normal((frames, nz, ny, nx)).astype(np.float32))
+    plan, q = ffdas_amd.Interpolator(t(g), mode=mode), t(q)
+    if kept:
+        plan.preprocess(q)
+    ref = plan(v, q)
+    buf = torch.zeros(v.numel() + shift, dtype=v.dtype, device=dev)
+    xin, out = buf[:v.numel()].view(v.shape), buf[shift:].view(v.shape)
+    xin.copy_(v)
+    plan(xin, q, out=out)
+    assert torch.equal(out, ref)
