@@ -17,17 +17,28 @@ namespace dev {
 // addition whose high word is floor(tau) and whose low word is the fraction, where the
 // floating-point form needs about fifteen operations (TwoSum, scale, two floors) for each
 // tap.  The terms carry the compensated pairs to within 2^-31 of a sample, below the FP32
-// rounding of the fraction that follows either way.
+// rounding of the fraction that follows either way (a term
+// between -1 and 0, whose fraction has the places of a number near 1, to within 2^-24).
 constexpr float kFixedLimit = 4194304.0f;      // |term| < 2^22: its low part fits 31 bits
 constexpr int kFixedNone = 0x40000000;         // high word of a term that selects no sample
+
+// The fraction of h, which for h just below an integer is at most the largest float below 1 (h less
+// its floor rounds to 1 there, and 2^32 does not convert to 32 bits).
+__host__ __device__ __forceinline__ float fraction(float h) {
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_fractf(h);
+#else
+    return __builtin_fminf(h - __builtin_floorf(h), 0x1.fffffep-1f);
+#endif
+}
 
 // h + l (|h| < 2^22, |l| <= ulp(h)) as 32.32 fixed point.
 __host__ __device__ __forceinline__ int64_t to_fixed(float h, float l) {
 #pragma clang fp contract(off)
     const float f = __builtin_floorf(h);
-    const uint32_t lo = (uint32_t)((h - f) * 4294967296.0f);           // saturates at 2^32 - 1
+    const uint32_t lo = (uint32_t)(fraction(h) * 4294967296.0f);
     const int li = (int)__builtin_rintf(l * 4294967296.0f);
-    return (((int64_t)(int)f << 32) | lo) + (int64_t)li;
+    return (int64_t)((uint64_t)(uint32_t)(int)f << 32 | lo) + (int64_t)li;
 }
 
 // scale * (h + l) as a float pair; exact for scale == 1.

@@ -85,7 +85,33 @@ static long orders() {
     return n;
 }
 
+// Terms of every size and sign, h just below an integer among them, convert without leaving 32 bits
+// and hold h + l to 2^-31; between -1 and 0, where h has more places than its fraction, to 2^-24.
+static long terms() {
+    long n = 0;
+    std::vector<float> hs = {0.0f, -0.0f, 4194303.75f, -4194303.75f, -1e-38f, -1e-45f, 1e-45f};
+    for (int e = -40; e < 22; e++)
+        for (float m : {1.0f, 1.25f, 1.9999999f}) {
+            const float v = std::ldexp(m, e);
+            hs.push_back(v);
+            hs.push_back(-v);
+            hs.push_back(std::nextafter(std::floor(v), -INFINITY));
+            hs.push_back(-std::nextafter(std::floor(v), INFINITY));
+        }
+    for (float h : hs)
+        for (float part : {0.0f, 0.5f, -0.5f, 0.37f}) {
+            const float ulp = std::nextafter(std::fabs(h), INFINITY) - std::fabs(h);
+            const float l = part * ulp;
+            const int64_t v = to_fixed(h, l);
+            const double want = std::ldexp((double)h + (double)l, 32);
+            CHECK(std::fabs((double)v - want) <= (h < 0.0f && h > -1.0f ? 256.0 : 2.0));
+            n++;
+        }
+    return n;
+}
+
 int main() {
-    std::printf("slots %ld, tiles %ld, orders %ld: index arithmetic clean\n", slots(), tiles(), orders());
+    std::printf("slots %ld, tiles %ld, orders %ld, terms %ld: index arithmetic clean\n", slots(), tiles(),
+                orders(), terms());
     return 0;
 }
