@@ -13,9 +13,9 @@ namespace dev {
 // four FMA-class operations.  A wave issues the loads of TB taps before it uses the first,
 // and G waves share a voxel tile by channels, so that small images fill the chip too.
 //
-// Terms that fixed point does not hold (a delay beyond 2^22 samples, not finite, or a weight
-// whose product with 2^-32 is not exact) take the floating-point tap of the plain kernel; a
-// wave meets them together.
+// A finite offset beyond every sample is a slot that reads nothing.  Other terms that fixed point
+// does not hold (not finite, a radius beyond 2^22 samples, or a real weight whose product with 2^-32
+// is not exact) take the floating-point tap of the plain kernel; a wave meets them together.
 //
 // 128^3 voxels, 1024 channels, 16 transmits, FP32, cone of 30 degrees: 27.8 ms with the
 // floating-point tap at one wave per tile, 18.1 ms with the fixed-point tap, 16 ms with 16 slots
@@ -130,9 +130,10 @@ __global__ __launch_bounds__(1024) void das_fwd_few_kernel(Geo g, Tiling tl,
                     if (any) rowoff[j] = (uint32_t)sq * (uint32_t)xs_t * (uint32_t)Rows::ES;
                 }
                 scale_pair(g.scale, h, l);
+                any = any && !beyond_samples(h, g.S);
                 const float aw = __builtin_fabsf(wt[j]);
-                const bool good = __builtin_fabsf(h) < kFixedLimit &&
-                                  (aw == 0.0f || (aw > 1e-27f && aw < 3e38f));
+                const bool good = __builtin_fabsf(h) < kFixedLimit && aw < 3e38f &&
+                                  (CPLX || aw == 0.0f || aw > 1e-27f);
                 if (any && good) ofs[j] = to_fixed(h, l);
                 else wt[j] = 0.0f;                       // it meets zeros: no NaN from it
                 if (any && !good) plainly = false;

@@ -17,8 +17,8 @@ namespace dev {
 // addition whose high word is floor(tau) and whose low word is the fraction, where the
 // floating-point form needs about fifteen operations (TwoSum, scale, two floors) for each
 // tap.  The terms carry the compensated pairs to within 2^-31 of a sample, below the FP32
-// rounding of the fraction that follows either way (a term
-// between -1 and 0, whose fraction has the places of a number near 1, to within 2^-24).
+// rounding of the fraction that follows either way (a term between -1 and 0, whose fraction has
+// the places of a number near 1, to within 2^-24).
 constexpr float kFixedLimit = 4194304.0f;      // |term| < 2^22: its low part fits 31 bits
 constexpr int kFixedNone = 0x40000000;         // high word of a term that selects no sample
 
@@ -39,6 +39,13 @@ __host__ __device__ __forceinline__ int64_t to_fixed(float h, float l) {
     const uint32_t lo = (uint32_t)(fraction(h) * 4294967296.0f);
     const int li = (int)__builtin_rintf(l * 4294967296.0f);
     return (int64_t)((uint64_t)(uint32_t)(int)f << 32 | lo) + (int64_t)li;
+}
+
+// Whether a finite delay h of a slot, beyond the limit, selects no sample of S whatever radius
+// within the limit (0 <= r < 2^22) is added: the slot is passed over, as one without a transmit
+// is, and its wave keeps the fixed-point taps.  (An infinite delay makes its voxel NaN.)
+__host__ __device__ __forceinline__ bool beyond_samples(float h, int S) {
+    return __builtin_fabsf(h) < 3e38f && (h <= -kFixedLimit || (h >= kFixedLimit && S <= (int)kFixedLimit));
 }
 
 // scale * (h + l) as a float pair; exact for scale == 1.

@@ -110,8 +110,27 @@ static long terms() {
     return n;
 }
 
+// An offset that is passed over selects no sample with any radius, in exact arithmetic; one within
+// the limit or not finite is not passed over.
+static long beyond() {
+    long n = 0;
+    for (int S : {2, 83, 4096, 4194303, 4194304, 4194305, 1 << 29})
+        for (float h : {-INFINITY, -3e38f, -6e6f, -4194304.5f, -4194304.0f, -4194303.75f, -1.0f, 0.0f, 5e3f,
+                        4194303.75f, 4194304.0f, 5e6f, 1e9f, 3e38f, INFINITY, NAN}) {
+            const bool far = beyond_samples(h, S);
+            if (!std::isfinite(h) || std::fabs(h) < kFixedLimit) CHECK(!far);
+            else if (S <= 4194304 && std::fabs(h) < 3e38f) CHECK(far);
+            for (double r : {0.0, 0.25, 700.0, 4194303.0, 4194303.9999}) {
+                const double k = std::floor((double)h + r);
+                if (far) CHECK(!(k >= 0.0 && k < (double)(S - 1)));
+                n++;
+            }
+        }
+    return n;
+}
+
 int main() {
-    std::printf("slots %ld, tiles %ld, orders %ld, terms %ld: index arithmetic clean\n", slots(), tiles(),
-                orders(), terms());
+    std::printf("slots %ld, tiles %ld, orders %ld, terms %ld, offsets %ld: index arithmetic clean\n", slots(),
+                tiles(), orders(), terms(), beyond());
     return 0;
 }
