@@ -886,8 +886,13 @@ __global__ __launch_bounds__(512) void das_bwd_param_fi_kernel(
         chunk = b / gridDim.x;
         tile = b - chunk * gridDim.x;
     }
+    const Tiling ot = oriented(tl, g);
+    if (tile >= ot.nta * ot.nth * ot.ntw) {         // no tile: the launch covers the shape with most
+        if (scale_part) block_scale_store<ACC64>(0, scale_part);
+        return;
+    }
     bool valid;
-    int n = voxel_of(oriented(tl, g), tile, lane, valid);
+    int n = voxel_of(ot, tile, lane, valid);
     if (!valid) n = 0;          // computed, never stored: keeps every lane at the barriers
     const FrameInnerRows<ST, FT, CW, PL> xr(xv, chunk, g.C, g.T, g.S);
     float *go = gofs ? gofs + chunk * pstride : nullptr;
