@@ -115,6 +115,18 @@ __host__ __device__ __forceinline__ int64_t flat_most(int A, int H, int W) {
     return most;
 }
 
+// Whether the kernels shape a volume's tiles, or keep cubes of 4 x 4 x 4 voxels: a launch that leaves
+// CUs idle takes as long as one of its tiles does, and the cubes of a grid thinner than they are hold
+// fewer voxels.  Frame-inner rows, 17 x 3 x 65 voxels with depth last, 256 channels, 4 transmits:
+// forward 77 us in cubes, 132 shaped, parameter adjoint 90 and 134; turned round, from 0.71 to 1.7 of
+// the cubes' time.  Few frames, whose taps are bound by the VALU, are shaped always.  Sparse volumes need
+// 256 cubes (24^3 voxels 158 us, shaped 164; 30^3 voxels 312 and 265).
+__host__ __device__ __forceinline__ bool flat_volume(int A, int H, int W, bool sparse, bool frame_inner) {
+    const int64_t cubes = (int64_t)((A + 3) / 4) * ((H + 3) / 4) * ((W + 3) / 4);
+    if (sparse) return cubes >= 256;
+    return !frame_inner || cubes >= 512 || (A >= 4 && H >= 4 && W >= 4);
+}
+
 // The tiles of a volume whose delay changes by da, dh and dw a step along its axes: the shape whose
 // taps cost least, a tap costing tl.flat and the window of samples that the lanes of a wave read of
 // a row, which is what those steps span over a tile (da, dh, dw are sums over 16 pairs).  The axis

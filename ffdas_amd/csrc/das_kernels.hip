@@ -2021,9 +2021,8 @@ bool xcd_groups() {
 // wrong one: 29 ms).  Where depth steps are half the lateral ones it keeps cubes, which are then
 // the better (50 x 40 x 40, complex: 1203 us, tiles 1 thick 1657).  The cost of a tap beside its
 // window (Tiling::flat) is what those times give: large for few frames, whose taps are few bytes,
-// small where the lines it fetches are what it waits for.  Sparse volumes that do not give every CU a tile keep the
-// cubes and the eighths (24^3 voxels 158 us, flat 164, in chunks 172; from there on it is the other
-// way round, 30^3 voxels 312 and 265).
+// small where the lines it fetches are what it waits for.  Which volumes: dev::flat_volume; the
+// sparse ones that keep cubes keep the eighths too (24^3 voxels 164 us, in chunks 172).
 dev::Tiling make_tiling(const DasProblem &p, bool flat) {
     std::vector<int64_t> d;
     for (int64_t v : p.spatial)
@@ -2046,7 +2045,8 @@ dev::Tiling make_tiling(const DasProblem &p, bool flat) {
     t.nth = (t.H + t.th - 1) / t.th;
     t.ntw = (t.W + t.tw - 1) / t.tw;
     t.tiles = t.nta * t.nth * t.ntw;
-    if (flat && d.size() >= 3 && p.C > 0 && p.K > 0 && !(p.sparse && t.tiles < 256)) {
+    if (flat && d.size() >= 3 && p.C > 0 && p.K > 0 &&
+        dev::flat_volume(t.A, t.H, t.W, p.sparse, p.fi_frames > 0)) {
         t.flat = p.sparse ? 70.0f : p.fi_frames > 0 ? 32.0f : 300.0f;
         t.tiles = (int)dev::flat_most(t.A, t.H, t.W);
     }

@@ -68,6 +68,20 @@ static long tiles() {
     return n;
 }
 
+// Which volumes are shaped: dense ones from 4 voxels on along every axis, or with cubes for every CU;
+// with few frames all, sparse ones with 256 cubes.
+static long volumes() {
+    for (bool swap : {false, true})
+        for (int thin : {2, 3, 4, 5}) {
+            CHECK(flat_volume(17, swap ? thin : 65, swap ? 65 : thin, false, true) == (thin >= 4));
+            CHECK(flat_volume(thin, 16, 16, false, false));
+            CHECK(flat_volume(256, swap ? thin : 256, swap ? 256 : thin, false, true));
+            CHECK(!flat_volume(24, 24, swap ? 24 : thin, true, true));
+        }
+    CHECK(flat_volume(8, 8, 8, false, true) && flat_volume(30, 30, 30, true, true));
+    return 4;
+}
+
 // The orders of the blocks over the XCDs are bijections, partial last rounds included.
 static long orders() {
     long n = 0;
@@ -130,7 +144,7 @@ static long beyond() {
 }
 
 int main() {
-    std::printf("slots %ld, tiles %ld, orders %ld, terms %ld, offsets %ld: index arithmetic clean\n", slots(),
-                tiles(), orders(), terms(), beyond());
+    std::printf("slots %ld, tiles %ld, volumes %ld, orders %ld, terms %ld, offsets %ld: index arithmetic "
+                "clean\n", slots(), tiles(), volumes(), orders(), terms(), beyond());
     return 0;
 }
