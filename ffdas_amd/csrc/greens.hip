@@ -1,13 +1,15 @@
 // Frequency-domain Green's function summation (ffdas_greens):
 //   out[b, t, f] = sum_s x[b, s, f] e^{i k_f r_ts} / r_ts,   r_ts = |dst_t - src_s|.
-// One event (greens_kernel): one lane per target, its position and per-source distance in
-// registers; the source position and the x values of a (source, frequency chunk) are the same
-// for the whole wave, so they come through the scalar unit; each thread keeps FPT complex sums
-// on the VALU.  More events (greens_mfma_kernel): the sums on the MFMA, see there.  FP32
-// throughout (the input may be stored as FP16).
+// One event, and up to four at few frequencies and many targets (greens_kernel): one lane per
+// target, its position and per-source distance in registers; the source position and the x values
+// of a (source, frequency chunk, event) are the same for the whole wave, so they come through the
+// scalar unit; each thread keeps FPT frequencies x BT events of complex sums on the VALU.  More
+// events and frequencies (greens_mfma_kernel): the sums on the MFMA, see there.  FP32 throughout (the
+// input may be stored as FP16).
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
 #include <climits>
 
 #include "internal.h"
@@ -24,16 +26,17 @@ __device__ __forceinline__ float2 load_x<float2>(const float2 *p) { return *p; }
 template <>
 __device__ __forceinline__ float2 load_x<__half2>(const __half2 *p) { return __half22float2(*p); }
 
-template <typename XT>
+template <typename XT, int BT>
 __global__ __launch_bounds__(256) void greens_kernel(const float *__restrict__ src,
                                                      const float *__restrict__ wav,
                                                      const XT *__restrict__ x,
                                                      const float *__restrict__ dst,
                                                      float2 *__restrict__ out, int nsrc, int nfreq,
-                                                     int ndst) {
+                                                     int ndst, int B) {
     const int t = blockIdx.x * 256 + threadIdx.x;
     const int f0 = blockIdx.y * kGreensFPT;
-    const int nf = min(kGreensFPT, nfreq - f0);
+    const int b0 = blockIdx.z * BT;
+    const int nf = min(kGreensFPT, nfreq - f0), nb = min(BT, B - b0);
     const bool valid = t < ndst;
     float px = 0, py = 0, pz = 0;
     if (valid) {
@@ -44,9 +47,11 @@ __global__ __launch_bounds__(256) void greens_kernel(const float *__restrict__ s
     float k[kGreensFPT];
 #pragma unroll
     for (int f = 0; f < kGreensFPT; f++) k[f] = f < nf ? wav[f0 + f] : 0.0f;
-    float ar[kGreensFPT], ai[kGreensFPT];
+    float ar[kGreensFPT][BT], ai[kGreensFPT][BT];
 #pragma unroll
-    for (int f = 0; f < kGreensFPT; f++) ar[f] = ai[f] = 0.0f;
+    for (int f = 0; f < kGreensFPT; f++)
+#pragma unroll
+        for (int b = 0; b < BT; b++) ar[f][b] = ai[f][b] = 0.0f;
 
     for (int s = 0; s < nsrc; s++) {
         // r = rsq * rsqrt(rsq), as the reference (greens_kernels.cuh:59-61)
@@ -54,24 +59,33 @@ __global__ __launch_bounds__(256) void greens_kernel(const float *__restrict__ s
         const float rsq = dx * dx + dy * dy + dz * dz;
         const float rinv = rsqrtf(rsq);
         const float r = rsq * rinv;
-        const XT *xs = x + (int64_t)s * nfreq + f0;
+        const XT *xs = x + ((int64_t)b0 * nsrc + s) * nfreq + f0;
 #pragma unroll
         for (int f = 0; f < kGreensFPT; f++) {
             if (f < nf) {
                 float sn, cs;
                 __sincosf(k[f] * r, &sn, &cs);
                 const float gr = cs * rinv, gi = sn * rinv;
-                const float2 v = load_x<XT>(xs + f);
-                ar[f] += gr * v.x - gi * v.y;
-                ai[f] += gr * v.y + gi * v.x;
+#pragma unroll
+                for (int b = 0; b < BT; b++) {
+                    if (b < nb) {
+                        const float2 v = load_x<XT>(xs + (int64_t)b * nsrc * nfreq + f);
+                        ar[f][b] += gr * v.x - gi * v.y;
+                        ai[f][b] += gr * v.y + gi * v.x;
+                    }
+                }
             }
         }
     }
     if (!valid) return;
-    float2 *o = out + (int64_t)t * nfreq + f0;
 #pragma unroll
-    for (int f = 0; f < kGreensFPT; f++)
-        if (f < nf) o[f] = float2{ar[f], ai[f]};
+    for (int b = 0; b < BT; b++) {
+        if (b >= nb) break;
+        float2 *o = out + ((int64_t)(b0 + b) * ndst + t) * nfreq + f0;
+#pragma unroll
+        for (int f = 0; f < kGreensFPT; f++)
+            if (f < nf) o[f] = float2{ar[f][b], ai[f][b]};
+    }
 }
 
 // More events: the multiply-adds on the MFMA, as a real product.  A wave has a tile of 16
@@ -271,19 +285,45 @@ __global__ __launch_bounds__(256, NT == 1 ? 5 : 3) void greens_mfma_kernel(const
     }
 }
 
+// Whether the sums stay on the VALU.  One event always (one column pair of the 8-event tile would be
+// in use: 128 sources to 256 x 128 targets, 512 frequencies 0.84 ms, on the MFMA 1.5).  Two to four where the
+// last chunk of frequencies leaves the MFMA tile, which forms all eight, mostly empty and there are
+// targets enough to fill the chip with one wave per 64 (the MFMA kernel has four times the waves).
+// 128 sources to 2^20 targets, VALU and MFMA: one frequency, 2 events 162 and 741 us, 4 events 201 and
+// 745; four frequencies, 4 events 470 and 760; eight, 2 events 591 and 754, 4 events 960 and 756.  To 2^15
+// targets the MFMA is the faster from one frequency on (2 events 45 and 30 us; 512 frequencies 1.79 and 1.5 ms).
+// With few sources the writes weigh more, and so does a second chunk of frequencies: 16 sources to 2^19
+// targets, 3 events, 12 frequencies 144 and 118 us.
+bool on_valu(int B, int nsrc, int nfreq, int ndst) {
+    if (B == 1) return true;
+    if (B > 4) return false;
+    const int chunks = (nfreq + kGreensFPT - 1) / kGreensFPT;
+    const double waves = (double)((ndst + 255) / 256) * 4.0 * chunks;
+    // frequencies a chunk up to which the VALU is the faster where it fills the chip, and fewer
+    // waves in proportion
+    const bool many = nsrc >= 64;
+    const double full = B == 4 ? 4.0 : B == 3 ? 5.0 : many ? 7.0 : 6.0;
+    double most = full * std::min(waves / 4096.0, 1.0);
+    if (many && waves >= 2048.0) most = std::min(full, most + 0.5);
+    if (many && waves >= 8192.0 && B > 2) most += 1.0;
+    if (many && waves >= 16384.0 && (B == 3 || (B == 2 && nfreq <= 64))) most += 1.0;
+    if (B == 3 && chunks > 1) most -= 1.0;
+    return (double)nfreq / chunks <= most;
+}
+
 template <typename XT>
 ffdas_error_t launch(hipStream_t st, const float *src, const float *wav, const void *x,
                      const float *dst, void *out, int nsrc, int nfreq, int ndst, int B) {
-    if (B == 1) {
-        // one column pair of the 8-event tile would be in use: for the geometry above 0.84 ms
-        // on the VALU and 1.5 ms on the MFMA, which 2 events take too (on the VALU 1.79)
+    if (on_valu(B, nsrc, nfreq, ndst)) {
         const dim3 grid((unsigned)((ndst + 255) / 256),
                         (unsigned)((nfreq + kGreensFPT - 1) / kGreensFPT), 1);
         ProfScope ps(st, "greens");
-        hipLaunchKernelGGL((greens_kernel<XT>), grid, dim3(256), 0, st, src, wav,
-                           static_cast<const XT *>(x), dst, static_cast<float2 *>(out), nsrc,
-                           nfreq, ndst);
-        return hip_status(hipGetLastError(), FFDAS_ERROR_CUDA_LAUNCH_FAILED);
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, src, wav, static_cast<const XT *>(x), dst,
+                               static_cast<float2 *>(out), nsrc, nfreq, ndst, B);
+            return hip_status(hipGetLastError(), FFDAS_ERROR_CUDA_LAUNCH_FAILED);
+        };
+        return B == 1 ? go(greens_kernel<XT, 1>) : go(greens_kernel<XT, 4>);
     }
     const int events = B <= 8 ? 8 : 16;
     const dim3 g((unsigned)((ndst + 63) / 64), (unsigned)((nfreq + kGreensFPW - 1) / kGreensFPW),
