@@ -411,7 +411,8 @@ __global__ __launch_bounds__(256) void interp_locate_kernel(
 // Location by cells.  The query points are counted, scanned and ordered by bin, so that the
 // points of the bins (x0 .. x1, y, z) are one run, and every cell walks the runs of its quantised
 // bounding box (the union of its tetrahedra's boxes: every tetrahedron the reference would list
-// in a point's bin is met).  A point inside the cell's box, widened by 5 % of its extent plus
+// in a point's bin is met; what the lanes of a cell do not get through in a few dozen steps is left to a
+// second kernel, a wave for each piece).  A point inside the cell's box, widened by 5 % of its extent plus
 // 1e-5 of the coordinates' magnitude per axis (the FP32 weights of a tetrahedron that the 1e-12
 // volume test admits err far less than that), is tested against the six tetrahedra in order; one
 // that passes, and whose own quantised box holds the point's bin, lowers the point's best key
@@ -465,54 +466,70 @@ __device__ __forceinline__ void wave_order() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// 2^(lgr + lgp) lanes per cell: 2^lgr share out the runs of its box, 2^lgp the points of a run.
-// The points inside a cell's box are few and come to the lanes at different times, so they are
-// put on a queue of the wave, and the tests, most of the work, run with a queued point in
-// every lane (one lane testing its own point on the spot: 0.54 ms for the cells of a 256 x 64 x 64
-// sector and 128^3 points, 0.26 ms queued).
-__global__ __launch_bounds__(256) void interp_locate_cells_kernel(
-    Box b, const float4 *__restrict__ v, int64_t ncell, int nx, int ny, int lgr, int lgp,
-    const int *__restrict__ pstart, const float4 *__restrict__ pts, int *__restrict__ best) {
-    __shared__ int2 queue[4][128];           // (base vertex, point) by wave
-    const int lane = threadIdx.x & 63;
-    int2 *q = queue[threadIdx.x >> 6];
-    const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t cell = gid >> (lgr + lgp);
-    const int psub = (int)gid & ((1 << lgp) - 1), rsub = (int)(gid >> lgp) & ((1 << lgr) - 1);
-    int base = 0, rows = 0, ny1 = 1;
+// The bounding box of a cell's vertices, widened, and the bins it lies in.
+struct CellBox {
     float lo[3], hi[3];
-    int b0[3] = {kBins - 1, kBins - 1, kBins - 1}, b1[3] = {0, 0, 0};
+    int b0[3], b1[3];
+    __device__ __forceinline__ int rows() const { return (b1[1] - b0[1] + 1) * (b1[2] - b0[2] + 1); }
+    // the ordered points of the bins (b0 .. b1, y, z) of row r
+    __device__ __forceinline__ int2 run(int r, const int *__restrict__ pstart) const {
+        const int ny = b1[1] - b0[1] + 1, dz = r / ny;
+        const int row = kBins * (b0[1] + r - dz * ny + kBins * (b0[2] + dz));
+        return int2{pstart[row + b0[0]], pstart[row + b1[0] + 1]};
+    }
+    __device__ __forceinline__ bool holds(const float4 *__restrict__ p) const {
+        const float4 u = *p;                 // one load
+        return u.x >= lo[0] && u.x <= hi[0] && u.y >= lo[1] && u.y <= hi[1] && u.z >= lo[2] && u.z <= hi[2];
+    }
+};
+
+__device__ __forceinline__ CellBox cell_box(const Box &b, const float4 *__restrict__ v, int base, int nx,
+                                            int ny) {
+    CellBox c;
 #pragma unroll
     for (int a = 0; a < 3; a++) {
-        lo[a] = 3.4e38f;
-        hi[a] = -3.4e38f;
+        c.lo[a] = 3.4e38f;
+        c.hi[a] = -3.4e38f;
+        c.b0[a] = kBins - 1;
+        c.b1[a] = 0;
     }
-    if (cell < ncell) {
-        base = cell_base((unsigned)cell, nx, ny);
 #pragma unroll
-        for (int k = 0; k < 8; k++) {
-            const float4 u = v[corner(base, k, nx, ny)];
-            const float p[3] = {u.x, u.y, u.z};
-#pragma unroll
-            for (int a = 0; a < 3; a++) {
-                lo[a] = fminf(lo[a], p[a]);
-                hi[a] = fmaxf(hi[a], p[a]);
-                const int q1 = vertex_bin(p[a], b.mn[a], b.sc[a]);
-                b0[a] = min(b0[a], q1);
-                b1[a] = max(b1[a], q1);
-            }
-        }
+    for (int k = 0; k < 8; k++) {
+        const float4 u = v[corner(base, k, nx, ny)];
+        const float p[3] = {u.x, u.y, u.z};
 #pragma unroll
         for (int a = 0; a < 3; a++) {
-            const float m = 0.05f * (hi[a] - lo[a]) + 1e-5f * (fabsf(lo[a]) + fabsf(hi[a])) + 1e-30f;
-            lo[a] -= m;
-            hi[a] += m;
+            c.lo[a] = fminf(c.lo[a], p[a]);
+            c.hi[a] = fmaxf(c.hi[a], p[a]);
+            const int q1 = vertex_bin(p[a], b.mn[a], b.sc[a]);
+            c.b0[a] = min(c.b0[a], q1);
+            c.b1[a] = max(c.b1[a], q1);
         }
-        ny1 = b1[1] - b0[1] + 1;
-        rows = ny1 * (b1[2] - b0[2] + 1);
     }
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        const float m = 0.05f * (c.hi[a] - c.lo[a]) + 1e-5f * (fabsf(c.lo[a]) + fabsf(c.hi[a])) + 1e-30f;
+        c.lo[a] -= m;
+        c.hi[a] += m;
+    }
+    return c;
+}
+
+// The points inside a cell's box are few and come to the lanes at different times, so they are put
+// on a queue of the wave, and the tests, most of the work, run with a queued point in every lane
+// (one lane testing its own point on the spot: 0.54 ms for the cells of a 256 x 64 x 64 sector and
+// 128^3 points, 0.26 ms queued).
+struct PointQueue {
+    Box b;
+    const float4 *__restrict__ v;
+    int nx, ny;
+    const float4 *__restrict__ pts;
+    int *__restrict__ best;
+    int2 *q;                 // 128 of (base vertex, point)
+    int waiting;             // queued points, uniform
+
     // a queued point against the six tetrahedra of its cell
-    auto test = [&](int2 c) {
+    __device__ __forceinline__ void test(int2 c) const {
         const float4 u = pts[c.y];
         const float p[3] = {u.x, u.y, u.z};
         // an outdated best only costs a test: the minimum is taken atomically
@@ -530,43 +547,170 @@ __global__ __launch_bounds__(256) void interp_locate_cells_kernel(
             atomicMin(best + c.y, key);
             break;
         }
-    };
-    int r = rsub, e = 0, pe = 0, waiting = 0;     // waiting: queued points, uniform
-    for (;;) {
-        // a step takes a point of the run, or goes to the next run
-        bool hit = false;
-        int at = 0;
-        if (e < pe) {
-            const float4 u = pts[e];
-            hit = u.x >= lo[0] && u.x <= hi[0] && u.y >= lo[1] && u.y <= hi[1] &&
-                  u.z >= lo[2] && u.z <= hi[2];
-            at = e;
-            e += 1 << lgp;
-        } else if (r < rows) {
-            const int dz = r / ny1, row = kBins * (b0[1] + r - dz * ny1 + kBins * (b0[2] + dz));
-            e = pstart[row + b0[0]] + psub;
-            pe = pstart[row + b1[0] + 1];
-            r += 1 << lgr;
-        }
-        const bool live = e < pe || r < rows;
-        const uint64_t hits = __ballot(hit);
-        if (hits) {
-            if (hit)
-                q[waiting + __builtin_amdgcn_mbcnt_hi((unsigned)(hits >> 32),
-                                                      __builtin_amdgcn_mbcnt_lo((unsigned)hits, 0))] =
-                    int2{base, at};
-            waiting += __popcll(hits);
-            wave_order();
-            if (waiting >= 64) {
-                waiting -= 64;
-                const int2 c = q[waiting + lane];
-                wave_order();
-                test(c);
-            }
-        }
-        if (__ballot(live) == 0) break;
     }
-    if (lane < waiting) test(q[lane]);
+    // the lanes with a hit queue theirs (all lanes call)
+    __device__ __forceinline__ void offer(bool hit, int base, int at) {
+        const uint64_t hits = __ballot(hit);
+        if (!hits) return;
+        if (hit)
+            q[waiting + __builtin_amdgcn_mbcnt_hi((unsigned)(hits >> 32),
+                                                  __builtin_amdgcn_mbcnt_lo((unsigned)hits, 0))] =
+                int2{base, at};
+        waiting += __popcll(hits);
+        wave_order();
+        if (waiting >= 64) {
+            waiting -= 64;
+            const int2 c = q[waiting + (threadIdx.x & 63)];
+            wave_order();
+            test(c);
+        }
+    }
+    __device__ __forceinline__ void finish() {
+        if ((int)(threadIdx.x & 63) < waiting) test(q[threadIdx.x & 63]);
+    }
+};
+
+// Work that the lanes of a cell leave to whole waves: runs of points and ranges of rows.  Points in
+// a small part of the grid (a zoomed raster) and cells far larger than the rest would otherwise be
+// walked by the few lanes that an average cell has.  An entry is (base vertex, first, end, step): rows
+// first, first + step, .. before end, at most 64; or, with step 0, the ordered points first .. end.
+// The entries are in kLists lists, a cache line for each one's count: 16384 waves that add to one count
+// from all XCDs take a millisecond.
+constexpr int kLists = 16, kCountStep = 16;        // kCountStep * 8 bytes apart
+struct Leftover {
+    unsigned long long *count;      // of list l at l * kCountStep
+    int4 *work;                     // from l * cap
+    int cap, slice;                 // entries of a list, points of one entry
+    // room for n entries in this workgroup's list, or none (what was reserved then is empty entries)
+    __device__ __forceinline__ int4 *reserve(int n) const {
+        const int list = blockIdx.x % kLists;
+        unsigned long long *c = count + list * kCountStep;
+        int4 *w = work + (int64_t)list * cap;
+        if (*(volatile unsigned long long *)c >= (unsigned long long)cap) return nullptr;
+        const unsigned long long at = atomicAdd(c, (unsigned long long)n);
+        if (at + n <= (unsigned long long)cap) return w + at;
+        for (unsigned long long k = at; k < (unsigned long long)cap; k++) w[k] = int4{0, 0, 0, 0};
+        return nullptr;
+    }
+};
+// Points and rows a lane walks before it leaves the rest.  256 x 64 x 64 sector, 180^3 points, the two
+// kernels: 16 steps 863 us, 24 716, 32 663, 48 608, 96 636; 128^3 points in a quarter of the box along each
+// axis 949, 941, 934, 935 (754 us walked by the lanes to the end), in the 64 x 16 x 20 vertices of a box
+// 281, 327, 366, 450 and 733 (1708 walked to the end).
+constexpr int kLaneSteps = 48;
+
+// The lanes of a wave leave what they have left of their runs (e .. pe) and rows (r .. rows).  Of the
+// 2^lgp lanes that share a run and the rows after it the first is nowhere ahead of the others: it
+// lists its own rest for all of them.  False where there is no room: they go on.
+__device__ __forceinline__ bool leave(const Leftover &rest, int base, int rows, int lgr, int lgp, int e, int pe,
+                                      int r) {
+    const int lane = threadIdx.x & 63;
+    const bool lists = (lane & ((1 << lgp) - 1)) == 0;
+    const int slices = lists && e < pe ? (pe - e - 1) / rest.slice + 1 : 0;
+    const int ranges = lists && r < rows ? ((rows - 1 - r) >> (lgr + 6)) + 1 : 0;
+    int upto = slices + ranges;                  // entries of this lane and those before
+    for (int o = 1; o < 64; o <<= 1) {
+        const int below = __shfl_up(upto, o);
+        if (lane >= o) upto += below;
+    }
+    const int n = __shfl(upto, 63);
+    unsigned long long to = 0;
+    if (lane == 0) to = (unsigned long long)rest.reserve(n);
+    to = __shfl(to, 0);
+    if (to == 0) return false;
+    int4 *w = (int4 *)to + (upto - slices - ranges);
+    for (int k = 0; k < slices; k++)
+        w[k] = int4{base, e + k * rest.slice, e + min(pe - e, (k + 1) * rest.slice), 0};
+    for (int k = 0; k < ranges; k++)
+        w[slices + k] = int4{base, r + (k << (lgr + 6)), min(rows, r + ((k + 1) << (lgr + 6))), 1 << lgr};
+    return true;
+}
+
+// 2^(lgr + lgp) lanes per cell: 2^lgr share out the rows of its box, 2^lgp the points of a run.
+__global__ __launch_bounds__(256, 7) void interp_locate_cells_kernel(
+    Box b, const float4 *__restrict__ v, int64_t ncell, int nx, int ny, int lgr, int lgp,
+    const int *__restrict__ pstart, const float4 *__restrict__ pts, int *__restrict__ best, Leftover rest) {
+    __shared__ int2 queue[4][128];
+    PointQueue q{b, v, nx, ny, pts, best, queue[threadIdx.x >> 6], 0};
+    const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t cell = gid >> (lgr + lgp);
+    const int psub = (int)gid & ((1 << lgp) - 1), rsub = (int)(gid >> lgp) & ((1 << lgr) - 1);
+    const int base = cell < ncell ? cell_base((unsigned)cell, nx, ny) : 0;
+    CellBox box{};
+    int rows = 0;
+    if (cell < ncell) {
+        box = cell_box(b, v, base, nx, ny);
+        rows = box.rows();
+    }
+    int r = rsub, e = 0, pe = 0;
+    for (bool left = false;;) {
+        bool live = true;
+        for (int k = left ? INT_MAX : kLaneSteps; k > 0 && live; k--) {
+            // a step takes a point of the run, or goes to the next run
+            bool hit = false;
+            int at = 0;
+            if (e < pe) {
+                hit = box.holds(pts + e);
+                at = e;
+                e += 1 << lgp;
+            } else if (r < rows) {
+                const int2 run = box.run(r, pstart);
+                e = run.x + psub;
+                pe = run.y;
+                r += 1 << lgr;
+            }
+            q.offer(hit, base, at);
+            live = __ballot(e < pe || r < rows) != 0;
+        }
+        if (!live || leave(rest, base, rows, lgr, lgp, e, pe, r)) break;
+        left = true;
+    }
+    q.finish();
+}
+
+// The leftover work, an entry a wave at a time.  All lanes take points: of a range of rows, the rows'
+// points one after the other.
+__global__ __launch_bounds__(256) void interp_locate_rest_kernel(
+    Box b, const float4 *__restrict__ v, int nx, int ny, const int *__restrict__ pstart,
+    const float4 *__restrict__ pts, int *__restrict__ best, Leftover rest) {
+    __shared__ int2 queue[4][128];
+    PointQueue q{b, v, nx, ny, pts, best, queue[threadIdx.x >> 6], 0};
+    const int lane = threadIdx.x & 63;
+    const int wave = blockIdx.x * 4 + (threadIdx.x >> 6), list = wave % kLists;
+    const unsigned long long listed = rest.count[list * kCountStep];
+    const int count = listed < (unsigned long long)rest.cap ? (int)listed : rest.cap;
+    for (int i = wave / kLists; i < count; i += gridDim.x * 4 / kLists) {
+        const int4 w = rest.work[(int64_t)list * rest.cap + i];
+        const int base = __builtin_amdgcn_readfirstlane(w.x), first = __builtin_amdgcn_readfirstlane(w.y),
+                  end = __builtin_amdgcn_readfirstlane(w.z), step = __builtin_amdgcn_readfirstlane(w.w);
+        if (first >= end) continue;
+        const CellBox box = cell_box(b, v, base, nx, ny);
+        if (step == 0) {
+            for (int e0 = first; e0 < end; e0 += 64) {
+                const int at = e0 + lane;
+                q.offer(at < end && box.holds(pts + min(at, end - 1)), base, at);
+            }
+            continue;
+        }
+        const int r = first + lane * step;
+        const int2 run = r < end ? box.run(r, pstart) : int2{0, 0};
+        int upto = run.y - run.x;                     // points of this lane's row and those before
+        for (int o = 1; o < 64; o <<= 1) {
+            const int below = __shfl_up(upto, o);
+            if (lane >= o) upto += below;
+        }
+        const int total = __shfl(upto, 63), shift = run.y - upto;
+        for (int k0 = 0; k0 < total; k0 += 64) {
+            const int k = k0 + lane;
+            int row = 0;                              // rows that end at or before point k
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1)
+                if (__shfl(upto, row + o - 1) <= k) row += o;
+            const int at = k + __shfl(shift, row & 63);
+            q.offer(k < total && box.holds(pts + (k < total ? at : 0)), base, at);
+        }
+    }
+    q.finish();
 }
 
 // The lookups of the ordered points.
@@ -818,15 +962,20 @@ ffdas_error_t build_lists(ffdas_context &h, ffdas_interpolation_plan &p) {
     return FFDAS_SUCCESS;
 }
 
-// By cells unless the point ids do not fit an int or FFDAS_INTERP_LOCATE is "point".
+// By cells unless the point ids, and the steps past the last, do not fit an int or
+// FFDAS_INTERP_LOCATE is "point".
 bool locate_by_cells(int64_t n) {
     const char *how = std::getenv("FFDAS_INTERP_LOCATE");
-    return n < INT_MAX && !(how && std::string(how) == "point");
+    return n < INT_MAX - (1 << 20) && !(how && std::string(how) == "point");
 }
 
 // Scratch of a location by cells, carved from one block.
 struct LocateScratch {
-    size_t pts = 0, best = 0, cnt = 0, start = 0, scan = 0, scan_bytes = 0, total = 0;
+    // the bins' counts, a last 0, and from the next multiple of 128 bytes the lists' counts
+    static constexpr int64_t list_counts() { return (kBins3 + 1 + 31) / 32 * 32; }
+    static constexpr int64_t counts() { return list_counts() + 2 * kLists * kCountStep; }
+    size_t pts = 0, best = 0, cnt = 0, start = 0, scan = 0, scan_bytes = 0, work = 0, total = 0;
+    int cap = 0;       // entries of a list of leftover work
     static ffdas_error_t plan(int64_t n, hipStream_t st, LocateScratch &s) {
         const size_t nb = (size_t)kBins3 + 1;
         int *none = nullptr;
@@ -836,9 +985,12 @@ struct LocateScratch {
         s.pts = 0;
         s.best = s.pts + up256((size_t)n * sizeof(float4));
         s.cnt = s.best + up256((size_t)n * sizeof(int));
-        s.start = s.cnt + up256(nb * sizeof(int));
+        s.start = s.cnt + up256(counts() * sizeof(int));
         s.scan = s.start + up256(nb * sizeof(int));
-        s.total = s.scan + up256(s.scan_bytes);
+        s.work = s.scan + up256(s.scan_bytes);
+        // at most 4096 slices of a run and 256 ranges of a cell's rows fit a list
+        s.cap = (int)std::min<int64_t>(std::max<int64_t>(n / 8, 1 << 18), 1 << 21) / kLists;
+        s.total = s.work + up256((size_t)s.cap * kLists * sizeof(int4));
         return FFDAS_SUCCESS;
     }
 };
@@ -865,18 +1017,24 @@ ffdas_error_t locate(ffdas_context &h, ffdas_interpolation_plan &p, const float 
     // of a run sharing it two points a lane.  Measured by lanes (runs x points): 9 points
     // (256 x 64 x 64 vertices, 128^3 points) 0.59 ms 1 x 1, 0.55 2 x 1, 0.61 2 x 4; 99 points
     // (128 x 32 x 32, 180^3) 2.84 ms 1 x 1, 0.98 4 x 4; 414 points (64 x 16 x 20, 180^3) 12.4 ms
-    // 1 x 1, 0.91 8 x 8; 0.2 points (400 x 90 x 90, 40^3) 0.44 ms 1 x 1, 0.53 4 x 1.
+    // 1 x 1, 0.91 8 x 8; 0.2 points (400 x 90 x 90, 40^3) 0.44 ms 1 x 1, 0.53 4 x 1.  A cell may
+    // have many waves (2 x 2 x 2 vertices, 128^3 points: 117 ms with 64 lanes a cell, 0.22 so), and what is
+    // far from the average is left over (64 x 16 x 20, 128^3 points in a sixteenth of the box along each axis:
+    // 52 ms walked by the lanes, 2 so).
     int lgr = 0, lgp = 0;
     if (p.ntet > 0) {
         const double bins = (double)p.list_total / (double)p.ntet, dens = (double)n / (double)kBins3;
         const auto lg = [](double v) { return v > 1.0 ? (int)(std::log2(v) + 0.5) : 0; };
-        const int all = std::min(lg(bins * dens / 6.0), 6);
-        lgp = std::min(all, lg(std::cbrt(bins) * dens / 2.0));
-        lgr = all - lgp;
+        const int all = lg(bins * dens / 6.0);
+        lgp = std::min({all, lg(std::cbrt(bins) * dens / 2.0), 6});      // the lanes of a run in one wave
+        lgr = std::min(all - lgp, 14);
+        while (lgr + lgp > 0 && ncell > (int64_t)1 << (30 - lgr - lgp)) (lgr > 0 ? lgr : lgp)--;
     }
+    const Leftover rest{(unsigned long long *)(cnt + ls.list_counts()), (int4 *)(c + ls.work), ls.cap,
+                        (int)std::max<int64_t>(n >> 12, 512)};
     ProfScope ps(st, "interp_locate");
     const Box b = box_of(p);
-    hipLaunchKernelGGL(interp_zero_i32_kernel, dim3(1024), dim3(256), 0, st, cnt, kBins3 + 1);
+    hipLaunchKernelGGL(interp_zero_i32_kernel, dim3(1024), dim3(256), 0, st, cnt, ls.counts());
     hipLaunchKernelGGL(interp_point_bin_kernel, dim3(grid1(n)), dim3(256), 0, st, b, qp, n, cnt, idx);
     size_t scan_bytes = ls.scan_bytes;
     if (rocprim::exclusive_scan(c + ls.scan, scan_bytes, cnt, start, 0, (size_t)kBins3 + 1,
@@ -884,9 +1042,12 @@ ffdas_error_t locate(ffdas_context &h, ffdas_interpolation_plan &p, const float 
         return FFDAS_ERROR_CUDA_LAUNCH_FAILED;
     hipLaunchKernelGGL(interp_point_order_kernel, dim3(grid1(n)), dim3(256), 0, st, b, qp, n, start,
                        cnt, pts, best);
-    if (ncell > 0)
+    if (ncell > 0) {
         hipLaunchKernelGGL(interp_locate_cells_kernel, dim3(grid1(ncell << (lgr + lgp))), dim3(256), 0,
-                           st, b, p.verts, ncell, nx, ny, lgr, lgp, start, pts, best);
+                           st, b, p.verts, ncell, nx, ny, lgr, lgp, start, pts, best, rest);
+        hipLaunchKernelGGL(interp_locate_rest_kernel, dim3(1024), dim3(256), 0, st, b, p.verts, nx, ny,
+                           start, pts, best, rest);
+    }
     hipLaunchKernelGGL(interp_found_kernel, dim3(grid1(n)), dim3(256), 0, st, p.verts, nx, ny,
                        start + kBins3, pts, best, p.mode, idx, w);
     return hip_status(hipGetLastError(), FFDAS_ERROR_CUDA_LAUNCH_FAILED);
