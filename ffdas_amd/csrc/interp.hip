@@ -35,6 +35,8 @@ struct ffdas_interpolation_plan {
     int64_t nx = 0, ny = 0, nz = 0;
     int mode = FFDAS_INTERP_LINEAR;
     float4 *verts = nullptr;           // nx * ny * nz, one 16-byte vector per vertex
+    unsigned char *flat = nullptr;     // behind them, by base vertex: the cell's flat tetrahedra (bits)
+    bool any_flat = false;
     float bmin[3] = {0, 0, 0}, scale[3] = {0, 0, 0};
     int64_t ntet = 0;
     long long list_total = 0;          // entries of the bin lists
@@ -122,11 +124,13 @@ __device__ __forceinline__ bool quantize(const Box &b, float x, float y, float z
     return true;
 }
 
-// What the plan needs on the host: the box and the number of entries the bin lists would have.
+// What the plan needs on the host: the box, the number of entries the bin lists would have and whether
+// any tetrahedron is flat (flat_tets).
 struct PlanHead {
     Box box;
-    unsigned long long total;
+    unsigned long long total;         // below 2^52; and kAnyFlat for each workgroup with flat cells
 };
+constexpr unsigned long long kAnyFlat = 1ull << 53;      // at most 1024 workgroups
 
 // The vertices into 16-byte vectors, and the minima and maxima of each block's part.
 __global__ __launch_bounds__(256) void interp_verts_kernel(const float *__restrict__ v, int64_t n,
@@ -221,21 +225,63 @@ __device__ __forceinline__ void tet_bins(const Box &b, const float4 *__restrict_
     }
 }
 
-// head->total += the bins of every tetrahedron's box
+// The tetrahedra of a cell whose FP32 weights may be off by more than a few per cent: |volume| below 1e-4
+// of the product of two of its edges and the reach of the bins' points (the cell's diagonal and a bin).
+// The numerators and the volume are good to 16 eps = 9.5e-7 of such products, so that a point whose
+// weights come out as 0 or more lies within 3 x 9.5e-7 / 1e-4 = 2.9 % of the box of any other tetrahedron.
+// The volumes as barycentric() forms them: below 1e-12 no point passes.  The sixth tetrahedron, whose
+// four corners are one face of the cell, is flat wherever that face is a plane out of the axes.
+__device__ __forceinline__ unsigned flat_tets(const Box &b, const float (&v)[8][3]) {
+#pragma clang fp contract(off)
+    float reach2 = 0.0f;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        float lo = v[0][a], hi = v[0][a];
+#pragma unroll
+        for (int k = 1; k < 8; k++) {
+            lo = fminf(lo, v[k][a]);
+            hi = fmaxf(hi, v[k][a]);
+        }
+        const float r = hi - lo + 1.0f / b.sc[a];
+        reach2 += r * r;
+    }
+    unsigned flat = 0;
+#pragma unroll
+    for (int t = 0; t < 6; t++) {
+        const float *v0 = v[kTet[t][0]], *v1 = v[kTet[t][1]], *v2 = v[kTet[t][2]], *v3 = v[kTet[t][3]];
+        const float a0 = v1[0] - v0[0], a1 = v1[1] - v0[1], a2 = v1[2] - v0[2];
+        const float b0 = v2[0] - v0[0], b1 = v2[1] - v0[1], b2 = v2[2] - v0[2];
+        const float c0 = v3[0] - v0[0], c1 = v3[1] - v0[1], c2 = v3[2] - v0[2];
+        const float bc0 = b1 * c2 - b2 * c1, bc1 = b2 * c0 - b0 * c2, bc2 = b0 * c1 - b1 * c0;
+        const float denom = fabsf(a0 * bc0 + a1 * bc1 + a2 * bc2);
+        const float na = a0 * a0 + a1 * a1 + a2 * a2, nb = b0 * b0 + b1 * b1 + b2 * b2,
+                    nc = c0 * c0 + c1 * c1 + c2 * c2;
+        const float pair = sqrtf(fmaxf(na, nb) * fmaxf(fminf(na, nb), nc));
+        if (!(denom < 1e-12f) && denom < 1e-4f * pair * sqrtf(reach2)) flat |= 1u << t;
+    }
+    return flat;
+}
+
+// head->total += the bins of every tetrahedron's box; flat = the cells' flat tetrahedra
 __global__ __launch_bounds__(256) void interp_total_kernel(const float4 *__restrict__ v,
                                                            int64_t ncell, int nx, int ny,
-                                                           PlanHead *__restrict__ head) {
+                                                           PlanHead *__restrict__ head,
+                                                           unsigned char *__restrict__ flat) {
     const Box b = head->box;
     unsigned long long sum = 0;
+    int any = 0;
     for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < ncell; c += (int64_t)gridDim.x * 256) {
         const int base = cell_base((unsigned)c, nx, ny);
         int bin[8][3];
+        float p[8][3];
 #pragma unroll
         for (int k = 0; k < 8; k++) {
             const float4 q = v[corner(base, k, nx, ny)];
-            bin[k][0] = vertex_bin(q.x, b.mn[0], b.sc[0]);
-            bin[k][1] = vertex_bin(q.y, b.mn[1], b.sc[1]);
-            bin[k][2] = vertex_bin(q.z, b.mn[2], b.sc[2]);
+            p[k][0] = q.x;
+            p[k][1] = q.y;
+            p[k][2] = q.z;
+#pragma unroll
+            for (int a = 0; a < 3; a++) bin[k][a] = vertex_bin(p[k][a], b.mn[a], b.sc[a]);
         }
 #pragma unroll
         for (int t = 0; t < 6; t++) {
@@ -248,12 +294,18 @@ __global__ __launch_bounds__(256) void interp_total_kernel(const float4 *__restr
             }
             sum += n;
         }
+        const unsigned f = flat_tets(b, p);
+        flat[base] = (unsigned char)f;
+        any |= (int)f;
     }
     for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+    any = __syncthreads_or(any);
     __shared__ unsigned long long red[4];
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = sum;
     __syncthreads();
-    if (threadIdx.x == 0) atomicAdd(&head->total, red[0] + red[1] + red[2] + red[3]);
+    // one write a workgroup: they meet in one line (for the flag an atomic a wave took 50 us, a store 160)
+    if (threadIdx.x == 0)
+        atomicAdd(&head->total, red[0] + red[1] + red[2] + red[3] + (any ? kAnyFlat : 0));
 }
 
 // The per-bin lists of the point-by-point location: every tetrahedron counted into, then
@@ -413,10 +465,10 @@ __global__ __launch_bounds__(256) void interp_locate_kernel(
 // bounding box (the union of its tetrahedra's boxes: every tetrahedron the reference would list
 // in a point's bin is met; what the lanes of a cell do not get through in a few dozen steps is left to a
 // second kernel, a wave for each piece).  A point inside the cell's box, widened by 5 % of its extent plus
-// 1e-5 of the coordinates' magnitude per axis (the FP32 weights of a tetrahedron that the 1e-12
-// volume test admits err far less than that), is tested against the six tetrahedra in order; one
-// that passes, and whose own quantised box holds the point's bin, lowers the point's best key
-// by an atomic minimum.  The lookups are written by a last pass over the points.  No lists of
+// 1e-5 of the coordinates' magnitude per axis, is tested against the six tetrahedra in order, any other
+// point of the runs near them against the flat ones, whose FP32 weights may err by more than that (flat_tets); one
+// that passes, and whose own quantised box holds the point's bin, lowers the point's best key by an
+// atomic minimum.  The lookups are written by a last pass over the points.  No lists of
 // tetrahedra are built: their atomics met at the apex of a sector, where thousands of small
 // cells share a bin (512 x 96 x 96 sector: count 7.9 and fill 8.7 ms of a plan, and 7.7 ms to
 // locate 256^3 points in them; now 0.3 ms and 3.6 ms).
@@ -477,8 +529,7 @@ struct CellBox {
         const int row = kBins * (b0[1] + r - dz * ny + kBins * (b0[2] + dz));
         return int2{pstart[row + b0[0]], pstart[row + b1[0] + 1]};
     }
-    __device__ __forceinline__ bool holds(const float4 *__restrict__ p) const {
-        const float4 u = *p;                 // one load
+    __device__ __forceinline__ bool holds(const float4 &u) const {
         return u.x >= lo[0] && u.x <= hi[0] && u.y >= lo[1] && u.y <= hi[1] && u.z >= lo[2] && u.z <= hi[2];
     }
 };
@@ -515,27 +566,80 @@ __device__ __forceinline__ CellBox cell_box(const Box &b, const float4 *__restri
     return c;
 }
 
+// Where a point outside a cell's box may pass the test of a flat tetrahedron.  Usually the sixth alone
+// is flat: its weight n / denom of corner 5 is at most 1, so that |q . (b x c)|, the distance from the
+// plane of corners 4, 5 and 7 times an area below `pair`, is at most |denom| < 1e-4 pair reach and the
+// rounding of n, 9.5e-7 pair reach (flat_tets).  That leaves few points (one call for a 256 x 64 x 64 sector
+// and 128^3 points: 758 us with all of them tested, 548 so, 529 with none).  Points below the box of
+// the grid, whose bin is 0 however far they are, are tested always.
+struct FlatPlane {
+    float n[3] = {0, 0, 0}, d = 0, tol = -1.0f;      // tol < 0: no flat tetrahedron
+    __device__ __forceinline__ bool holds(const Box &b, const float4 &u) const {
+        if (tol < 0.0f) return false;
+        const float r = fabsf(n[0] * u.x + n[1] * u.y + n[2] * u.z - d);
+        return !(r > tol) || u.x < b.mn[0] || u.y < b.mn[1] || u.z < b.mn[2];
+    }
+};
+
+__device__ __forceinline__ FlatPlane flat_plane(const Box &b, const float4 *__restrict__ v, unsigned flat,
+                                                const CellBox &c, int base, int nx, int ny) {
+    FlatPlane f;
+    if (flat == 0) return f;
+    f.tol = INFINITY;
+    if (flat != 0x20) return f;
+    const float4 v4 = v[corner(base, 4, nx, ny)], v5 = v[corner(base, 5, nx, ny)],
+                 v6 = v[corner(base, 6, nx, ny)], v7 = v[corner(base, 7, nx, ny)];
+    const float ax = v6.x - v4.x, ay = v6.y - v4.y, az = v6.z - v4.z;
+    const float bx = v5.x - v4.x, by = v5.y - v4.y, bz = v5.z - v4.z;
+    const float cx = v7.x - v4.x, cy = v7.y - v4.y, cz = v7.z - v4.z;
+    const float pair = fmaxf(fmaxf(ax * ax + ay * ay + az * az, bx * bx + by * by + bz * bz),
+                             cx * cx + cy * cy + cz * cz);      // above any product of two edges
+    const float s = 1.0f / pair;
+    f.n[0] = (by * cz - bz * cy) * s;
+    f.n[1] = (bz * cx - bx * cz) * s;
+    f.n[2] = (bx * cy - by * cx) * s;
+    f.d = f.n[0] * v4.x + f.n[1] * v4.y + f.n[2] * v4.z;
+    float reach = 0.0f, size = 0.0f;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        const float bin = 1.0f / b.sc[a];
+        reach += c.hi[a] - c.lo[a] + bin;
+        size += fabsf(c.lo[a]) + fabsf(c.hi[a]) + bin;
+    }
+    f.tol = 1.1e-4f * reach + 1e-6f * size;      // and the rounding of this sum itself
+    return f;
+}
+
 // The points inside a cell's box are few and come to the lanes at different times, so they are put
 // on a queue of the wave, and the tests, most of the work, run with a queued point in every lane
 // (one lane testing its own point on the spot: 0.54 ms for the cells of a 256 x 64 x 64 sector and
-// 128^3 points, 0.26 ms queued).
-struct PointQueue {
+// 128^3 points, 0.26 ms queued).  FLAT: the points of the bins outside the box are tested against the
+// cell's flat tetrahedra.
+constexpr int kFlatOnly = 1 << 30;       // base vertices are below 2^28
+template <bool FLAT> struct PointQueue {
     Box b;
     const float4 *__restrict__ v;
+    const unsigned char *__restrict__ flat;
     int nx, ny;
     const float4 *__restrict__ pts;
     int *__restrict__ best;
     int2 *q;                 // 128 of (base vertex, point)
     int waiting;             // queued points, uniform
 
-    // a queued point against the six tetrahedra of its cell
+    // a queued point against the six tetrahedra of its cell, or the flat ones
     __device__ __forceinline__ void test(int2 c) const {
         const float4 u = pts[c.y];
         const float p[3] = {u.x, u.y, u.z};
+        unsigned which = 0x3f;
+        if (FLAT && (c.x & kFlatOnly)) {
+            c.x &= ~kFlatOnly;
+            which = flat[c.x];
+        }
         // an outdated best only costs a test: the minimum is taken atomically
         const int known = best[c.y];
 #pragma unroll 1
         for (int key = c.x * 8; key < min(c.x * 8 + 6, known); key++) {
+            if (FLAT && !(which >> (key & 7) & 1)) continue;
             float w[4];
             if (!test_key(p, key, v, nx, ny, w)) continue;
             int tl[3], th[3], ib[3];
@@ -548,7 +652,7 @@ struct PointQueue {
             break;
         }
     }
-    // the lanes with a hit queue theirs (all lanes call)
+    // the lanes with a hit queue theirs (all lanes call); base: with kFlatOnly, for the flat ones
     __device__ __forceinline__ void offer(bool hit, int base, int at) {
         const uint64_t hits = __ballot(hit);
         if (!hits) return;
@@ -627,30 +731,36 @@ __device__ __forceinline__ bool leave(const Leftover &rest, int base, int rows, 
 }
 
 // 2^(lgr + lgp) lanes per cell: 2^lgr share out the rows of its box, 2^lgp the points of a run.
-__global__ __launch_bounds__(256, 7) void interp_locate_cells_kernel(
-    Box b, const float4 *__restrict__ v, int64_t ncell, int nx, int ny, int lgr, int lgp,
-    const int *__restrict__ pstart, const float4 *__restrict__ pts, int *__restrict__ best, Leftover rest) {
+template <bool FLAT>
+__global__ __launch_bounds__(256, FLAT ? 6 : 7) void interp_locate_cells_kernel(
+    Box b, const float4 *__restrict__ v, const unsigned char *__restrict__ flat, int64_t ncell, int nx,
+    int ny, int lgr, int lgp, const int *__restrict__ pstart, const float4 *__restrict__ pts,
+    int *__restrict__ best, Leftover rest) {
     __shared__ int2 queue[4][128];
-    PointQueue q{b, v, nx, ny, pts, best, queue[threadIdx.x >> 6], 0};
+    PointQueue<FLAT> q{b, v, flat, nx, ny, pts, best, queue[threadIdx.x >> 6], 0};
     const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int64_t cell = gid >> (lgr + lgp);
     const int psub = (int)gid & ((1 << lgp) - 1), rsub = (int)(gid >> lgp) & ((1 << lgr) - 1);
     const int base = cell < ncell ? cell_base((unsigned)cell, nx, ny) : 0;
     CellBox box{};
     int rows = 0;
+    FlatPlane plane;
     if (cell < ncell) {
         box = cell_box(b, v, base, nx, ny);
         rows = box.rows();
+        if (FLAT) plane = flat_plane(b, v, flat[base], box, base, nx, ny);
     }
     int r = rsub, e = 0, pe = 0;
     for (bool left = false;;) {
         bool live = true;
         for (int k = left ? INT_MAX : kLaneSteps; k > 0 && live; k--) {
             // a step takes a point of the run, or goes to the next run
-            bool hit = false;
+            bool hit = false, in = true;
             int at = 0;
             if (e < pe) {
-                hit = box.holds(pts + e);
+                const float4 u = pts[e];                 // one load
+                in = box.holds(u);
+                hit = in || (FLAT && plane.holds(b, u));
                 at = e;
                 e += 1 << lgp;
             } else if (r < rows) {
@@ -659,7 +769,7 @@ __global__ __launch_bounds__(256, 7) void interp_locate_cells_kernel(
                 pe = run.y;
                 r += 1 << lgr;
             }
-            q.offer(hit, base, at);
+            q.offer(hit, FLAT && !in ? base | kFlatOnly : base, at);
             live = __ballot(e < pe || r < rows) != 0;
         }
         if (!live || leave(rest, base, rows, lgr, lgp, e, pe, r)) break;
@@ -670,11 +780,12 @@ __global__ __launch_bounds__(256, 7) void interp_locate_cells_kernel(
 
 // The leftover work, an entry a wave at a time.  All lanes take points: of a range of rows, the rows'
 // points one after the other.
+template <bool FLAT>
 __global__ __launch_bounds__(256) void interp_locate_rest_kernel(
-    Box b, const float4 *__restrict__ v, int nx, int ny, const int *__restrict__ pstart,
-    const float4 *__restrict__ pts, int *__restrict__ best, Leftover rest) {
+    Box b, const float4 *__restrict__ v, const unsigned char *__restrict__ flat, int nx, int ny,
+    const int *__restrict__ pstart, const float4 *__restrict__ pts, int *__restrict__ best, Leftover rest) {
     __shared__ int2 queue[4][128];
-    PointQueue q{b, v, nx, ny, pts, best, queue[threadIdx.x >> 6], 0};
+    PointQueue<FLAT> q{b, v, flat, nx, ny, pts, best, queue[threadIdx.x >> 6], 0};
     const int lane = threadIdx.x & 63;
     const int wave = blockIdx.x * 4 + (threadIdx.x >> 6), list = wave % kLists;
     const unsigned long long listed = rest.count[list * kCountStep];
@@ -685,11 +796,15 @@ __global__ __launch_bounds__(256) void interp_locate_rest_kernel(
                   end = __builtin_amdgcn_readfirstlane(w.z), step = __builtin_amdgcn_readfirstlane(w.w);
         if (first >= end) continue;
         const CellBox box = cell_box(b, v, base, nx, ny);
+        FlatPlane plane;
+        if (FLAT) plane = flat_plane(b, v, flat[base], box, base, nx, ny);
+        const auto offer = [&](bool any, int at) {
+            const float4 u = pts[any ? at : 0];
+            const bool in = box.holds(u);
+            q.offer(any && (in || (FLAT && plane.holds(b, u))), FLAT && !in ? base | kFlatOnly : base, at);
+        };
         if (step == 0) {
-            for (int e0 = first; e0 < end; e0 += 64) {
-                const int at = e0 + lane;
-                q.offer(at < end && box.holds(pts + min(at, end - 1)), base, at);
-            }
+            for (int e0 = first; e0 < end; e0 += 64) offer(e0 + lane < end, e0 + lane);
             continue;
         }
         const int r = first + lane * step;
@@ -706,8 +821,7 @@ __global__ __launch_bounds__(256) void interp_locate_rest_kernel(
 #pragma unroll
             for (int o = 32; o > 0; o >>= 1)
                 if (__shfl(upto, row + o - 1) <= k) row += o;
-            const int at = k + __shfl(shift, row & 63);
-            q.offer(k < total && box.holds(pts + (k < total ? at : 0)), base, at);
+            offer(k < total, k + __shfl(shift, row & 63));
         }
     }
     q.finish();
@@ -896,6 +1010,7 @@ void free_plan_device(ffdas_interpolation_plan *p) {
                     (void *)p->pre_idx, (void *)p->pre_w})
         if (q) (void)hipFree(q);
     p->verts = nullptr;
+    p->flat = nullptr;
     p->bin_start = nullptr;
     p->bin_list = nullptr;
     p->pre_idx = nullptr;
@@ -1075,10 +1190,16 @@ ffdas_error_t locate(ffdas_context &h, ffdas_interpolation_plan &p, const float 
     hipLaunchKernelGGL(interp_point_order_kernel, dim3(grid1(n)), dim3(256), 0, st, b, qp, n, start,
                        cnt, pts, best);
     if (ncell > 0) {
-        hipLaunchKernelGGL(interp_locate_cells_kernel, dim3(grid1(ncell << (lgr + lgp))), dim3(256), 0,
-                           st, b, p.verts, ncell, nx, ny, lgr, lgp, start, pts, best, rest);
-        hipLaunchKernelGGL(interp_locate_rest_kernel, dim3(1024), dim3(256), 0, st, b, p.verts, nx, ny,
-                           start, pts, best, rest);
+        auto go = [&](auto cells, auto left) {
+            hipLaunchKernelGGL(cells, dim3(grid1(ncell << (lgr + lgp))), dim3(256), 0, st, b, p.verts, p.flat,
+                               ncell, nx, ny, lgr, lgp, start, pts, best, rest);
+            hipLaunchKernelGGL(left, dim3(1024), dim3(256), 0, st, b, p.verts, p.flat, nx, ny, start, pts,
+                               best, rest);
+        };
+        if (p.any_flat)
+            go(interp_locate_cells_kernel<true>, interp_locate_rest_kernel<true>);
+        else
+            go(interp_locate_cells_kernel<false>, interp_locate_rest_kernel<false>);
     }
     hipLaunchKernelGGL(interp_found_kernel, dim3(grid1(n)), dim3(256), 0, st, p.verts, nx, ny,
                        start + kBins3, pts, best, p.mode, idx, w);
@@ -1163,8 +1284,9 @@ ffdas_error_t evaluate(ffdas_context &h, const ffdas_interpolation_plan &p, cons
 ffdas_error_t build_plan(ffdas_context &h, ffdas_interpolation_plan &p, const float *gridpos) {
     const int64_t npts = p.nx * p.ny * p.nz;
     hipStream_t st = h.stream;
-    if (hipMalloc((void **)&p.verts, (size_t)npts * sizeof(float4)) != hipSuccess)
+    if (hipMalloc((void **)&p.verts, (size_t)npts * (sizeof(float4) + 1)) != hipSuccess)
         return FFDAS_ERROR_ALLOCATION_FAILED;
+    p.flat = reinterpret_cast<unsigned char *>(p.verts + npts);
     const int nblk = (int)std::min<int64_t>(1024, std::max<int64_t>(1, (npts + 255) / 256));
     void *ws = nullptr;
     const size_t head_bytes = up256(sizeof(PlanHead));
@@ -1177,7 +1299,7 @@ ffdas_error_t build_plan(ffdas_context &h, ffdas_interpolation_plan &p, const fl
     p.ntet = 6 * (p.nx - 1) * (p.ny - 1) * (p.nz - 1);
     if (p.ntet > 0)
         hipLaunchKernelGGL(interp_total_kernel, dim3(std::min(grid1(p.ntet / 6), 1024)), dim3(256), 0,
-                           st, p.verts, p.ntet / 6, (int)p.nx, (int)p.ny, head);
+                           st, p.verts, p.ntet / 6, (int)p.nx, (int)p.ny, head, p.flat);
     PlanHead hh{};
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(&hh, head, sizeof(hh), hipMemcpyDeviceToHost, st);
@@ -1187,6 +1309,8 @@ ffdas_error_t build_plan(ffdas_context &h, ffdas_interpolation_plan &p, const fl
         p.bmin[a] = hh.box.mn[a];
         p.scale[a] = hh.box.sc[a];
     }
+    p.any_flat = p.ntet > 0 && hh.total >= kAnyFlat;
+    hh.total &= kAnyFlat - 1;
     // entries of a point-by-point location's lists
     if (hh.total > (unsigned long long)INT_MAX || p.ntet > INT_MAX) return FFDAS_ERROR_DIMS_TOO_LARGE;
     p.list_total = (long long)hh.total;
