@@ -18,8 +18,8 @@ namespace dev {
 // is not exact) take the floating-point tap of the plain kernel; a wave meets them together.
 //
 // 128^3 voxels, 1024 channels, 16 transmits, FP32, cone of 30 degrees: 27.8 ms with the
-// floating-point tap at one wave per tile, 18.1 ms with the fixed-point tap, 16 ms with 16 slots
-// a round, 11.7 ms (2.9e12 units/s) with flat tiles and the XCDs sharing the grid in chunks.
+// floating-point tap at one wave per tile, 11.2 ms (3.1e12 units/s) with the fixed-point tap, 16
+// slots a round, flat tiles and the XCDs sharing the grid in chunks.
 constexpr int kXcdTiles = 64;
 
 template <Storage ST, int CW> struct FewRows {
@@ -296,10 +296,13 @@ template <bool CPLX, int FT> constexpr int tap_group() { return CPLX || FT > 1 ?
 
 // Waves per voxel tile of das_fwd_few_kernel: enough to put eight on each SIMD, at most 16 and
 // at most one per channel (128-element, 3-transmit image of 256 x 128: 147 us with one wave
-// per tile and the old tap, 21 us with 16).  Slots a lane holds at a time: 8, and 16 where
-// there are as many, which forms the radius half as often (128^3 volume, 16 transmits: 14.5 ms
-// with 8, 11.7 ms with 16; with 11 transmits, where the second half of a round of 16 would be
-// a remainder, 198 us with 8 and 213 us with 16 for 192 channels to 400 x 300).
+// per tile and the old tap, 21 us with 16).  Slots a lane holds at a time: 8, and 16, which forms the
+// radius half as often, where they leave no remainder or one below 4; a longer one costs more, since it
+// is not pipelined, than whole rounds of 8.  By 16 and by 8, 64^3 voxels and 256 channels, one frame:
+// 16 slots 554 and 587 us, 17 709 and 707, 20 794 and 760, 24 976 and 816, 31 1312 and 1122, 32 1049 and
+// 1084, 40 1494 and 1356, 48 1596 and 1632; 96^3 voxels and 1024 channels, 17 slots 7.98 and 8.21 ms, 24
+// 10.99 and 9.85; below 16 there are only rounds of 8 to fill (192 channels to 400 x 300, 11 slots: 213
+// and 198 us).
 template <Storage ST, bool CPLX, int FT>
 hipError_t launch_few_ft(hipStream_t st, const dev::Geo &g, const dev::Tiling &tl, const XView &xv,
                          void *out, int64_t os_b, double br, double bi) {
@@ -316,7 +319,7 @@ hipError_t launch_few_ft(hipStream_t st, const dev::Geo &g, const dev::Tiling &t
     };
     if (g.sparse) return go(dev::das_fwd_few_kernel<ST, CPLX, FT, 8, TB, true>);
     if constexpr (!CPLX && FT == 1)
-        if (g.K >= 16) return go(dev::das_fwd_few_kernel<ST, CPLX, FT, 16, TB, false>);
+        if (g.K >= 16 && g.K % 16 < 4) return go(dev::das_fwd_few_kernel<ST, CPLX, FT, 16, TB, false>);
     return go(dev::das_fwd_few_kernel<ST, CPLX, FT, 8, TB, false>);
 }
 
