@@ -272,24 +272,21 @@ __device__ __forceinline__ void sort_slots(int (&sq)[KC], float (&ofs)[KC], floa
     }
 }
 
-// Frame-inner forward with the loads of TB taps in flight together: each group of TB taps
+// Frame-inner forward of real data with the loads of TB taps in flight together: each group of TB taps
 // issues all its 16-byte loads before the first of them is used, so a wave keeps TB times
 // more gathers in flight than tap by tap.  A tap that reads nothing loads zeros (an offset
 // past the channel's block) with its weights zeroed, so it adds exactly zero and no branch
 // separates the loads from their use.
-template <Storage ST, bool ACC64, bool CPLX, bool PRECISE, int FT, int KC, int TB, bool PL>
-__device__ __forceinline__ void das_fwd_body_fi(const Geo &g, const FrameInnerRows<ST, FT, CPLX ? 2 : 1, PL> &xr,
+template <Storage ST, bool ACC64, bool PRECISE, int FT, int KC, int TB, bool PL>
+__device__ __forceinline__ void das_fwd_body_fi(const Geo &g, const FrameInnerRows<ST, FT, 1, PL> &xr,
                                                 int n, int m0, int mstep,
-                                                AccT<ACC64> (&acc)[FT][CPLX ? 2 : 1]) {
+                                                AccT<ACC64> (&acc)[FT][1]) {
     static_assert(KC % TB == 0, "taps per group must divide taps per round");
     using A = AccT<ACC64>;
-    using Rows = FrameInnerRows<ST, FT, CPLX ? 2 : 1, PL>;
-    constexpr int CW = CPLX ? 2 : 1;
+    using Rows = FrameInnerRows<ST, FT, 1, PL>;
     const SplitPt yp = split_point(g.dstpos[3 * n], g.dstpos[3 * n + 1], g.dstpos[3 * n + 2]);
 #pragma unroll
-    for (int f = 0; f < FT; f++)
-#pragma unroll
-        for (int c = 0; c < CW; c++) acc[f][c] = A(0);
+    for (int f = 0; f < FT; f++) acc[f][0] = A(0);
     if (g.S < 2) return;                       // no tap has two rows to read
 
     for (int kc = 0; kc < g.K; kc += KC) {
@@ -337,29 +334,14 @@ __device__ __forceinline__ void das_fwd_body_fi(const Geo &g, const FrameInnerRo
 #pragma unroll
                 for (int u = 0; u < TB; u++) {
                     const int j = j0 + u;
-                    A v[2][FT][CW];
+                    A v[2][FT][1];
                     xr.unpack(q[u], v);
-                    if constexpr (!CPLX) {
-                        const A c0 = (A)wt[j] * (A)tp[u].t;
-                        const A c = in[u] ? c0 : A(0);
-                        const A a = in[u] ? (A)wt[j] - c0 : A(0);
+                    const A c0 = (A)wt[j] * (A)tp[u].t;
+                    const A c = in[u] ? c0 : A(0);
+                    const A a = in[u] ? (A)wt[j] - c0 : A(0);
 #pragma unroll
-                        for (int f = 0; f < FT; f++)
-                            acc[f][0] = fmaA(c, v[1][f][0], fmaA(a, v[0][f][0], acc[f][0]));
-                    } else {
-                        float sn, cs;
-                        phase<PRECISE>(g.rev_h, g.rev_l, tp[u], sn, cs);
-                        const A wr = in[u] ? (A)(wt[j] * cs) : A(0);
-                        const A wi = in[u] ? (A)(wt[j] * sn) : A(0);
-                        const A t = in[u] ? (A)tp[u].t : A(0);
-#pragma unroll
-                        for (int f = 0; f < FT; f++) {
-                            const A lr = v[0][f][0] + t * (v[1][f][0] - v[0][f][0]);
-                            const A li = v[0][f][1] + t * (v[1][f][1] - v[0][f][1]);
-                            acc[f][0] += wr * lr - wi * li;
-                            acc[f][1] += wr * li + wi * lr;
-                        }
-                    }
+                    for (int f = 0; f < FT; f++)
+                        acc[f][0] = fmaA(c, v[1][f][0], fmaA(a, v[0][f][0], acc[f][0]));
                 }
             }
         }
@@ -573,7 +555,7 @@ __device__ __forceinline__ void fwd_fi_tile(const Geo &g, const Tiling &tl, cons
     else if constexpr (CPLX)
         das_fwd_body_iq<ST, FT, KC, TB, PL>(g, xr, n, wave, G, acc);
     else
-        das_fwd_body_fi<ST, ACC64, CPLX, PRECISE, FT, KC, TB, PL>(g, xr, n, wave, G, acc);
+        das_fwd_body_fi<ST, ACC64, PRECISE, FT, KC, TB, PL>(g, xr, n, wave, G, acc);
     if (G == 1) {
         if (valid) store_out<ACC64, CPLX, FT>(acc, outv, os_b, n, chunk * FT, g.B, beta_re, beta_im);
         return;
@@ -2692,7 +2674,7 @@ ffdas_error_t launch_forward(ffdas_context &h, const DasProblem &p, const DasGeo
         }
         return hip_status(e, FFDAS_ERROR_CUDA_LAUNCH_FAILED);
     }
-if (few_frames_ok(p, xv))
+    if (few)
         return hip_status(launch_forward_few(st, g, tl, p, xv, out, beta_re, beta_im),
                           FFDAS_ERROR_CUDA_LAUNCH_FAILED);
     if (!p.cplx) {
