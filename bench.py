@@ -268,8 +268,8 @@ def roofline(a, p, kt, U, tuned):
     L1/L2 and LDS serve them, so they do not bound against HBM.  onchip: the resource that
     binds the kernel, against its measured peak."""
     esz = p.x.element_size()
-    bytes_per_u = {"das_fwd_fi": 2 * esz, "das_fwd": 2 * esz, "das_bwd_param_fi": 2 * esz,
-                   "das_bwd_param": 2 * esz, "das_bwd_x": 2 * 4, "das_bwd_x_plain": 2 * 4}
+    bytes_per_u = {"das_fwd_fi": 2 * esz, "das_fwd": 2 * esz, "das_fwd_few": 2 * esz,
+                   "das_bwd_param_fi": 2 * esz, "das_bwd_param": 2 * esz, "das_bwd_x": 2 * 4, "das_bwd_x_plain": 2 * 4}
     dom = max((k for k in kt if k in bytes_per_u), key=kt.get)
     t = kt[dom] * 1e-3
     traffic = traffic_for(a.storage, dom)
@@ -603,14 +603,14 @@ def bench_interpolate(a):
     L.ffdas_profile_enable(0)
     eval_ms = kernel_ms("interp_eval")
     nq, npts = nq1 ** 3, nr * nt * nphi
-    located = float(torch.isfinite(interp(x[:1], q, fill=float("nan"))).float().mean())
+    located = float(torch.isfinite(interp(x, q, fill=float("nan"))[0]).float().mean())
     value = B * nq / (ms * 1e-3) / 1e9
     log(f"interpolate {B} x {nr}x{nt}x{nphi} -> {nq1}^3: {ms:.3f} ms/step ({value:.1f} G/s), "
         f"eval kernel {eval_ms:.3f} ms, plan {plan_ms:.1f} ms, locate {locate_ms:.3f} ms, "
         f"located {located:.3f}")
     # algorithmic bytes of one evaluation: every frame of x once, every output once, the
-    # lookup (4 ids + 4 weights per point) once per chunk of 16 frames (FP32 data)
-    nbytes = B * (nq + npts) * 4 + -(-B // 16) * nq * 32
+    # lookup (a key and 3 weights per point) once per chunk of 16 frames (FP32 data)
+    nbytes = B * (nq + npts) * 4 + -(-B // 16) * nq * 16
     roof = {"kernel": "interp_eval", "bound": "hbm", "ms": round(eval_ms, 4),
             "achieved": round(nbytes / (eval_ms * 1e-3) / 1e9, 1), "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "bytes_per_launch": nbytes,

@@ -312,7 +312,7 @@ hipError_t launch_few_ft(hipStream_t st, const dev::Geo &g, const dev::Tiling &t
     int G = 1;
     while (G < 16 && (int64_t)ntiles * grid.y * G < 8192 && 2 * G <= g.C) G *= 2;
     const size_t lds = G > 1 ? (size_t)G * FT * (CPLX ? 2 : 1) * 64 * sizeof(float) : 0;
-    ProfScope ps(st, "das_fwd");
+    ProfScope ps(st, "das_fwd_few");
     auto go = [&](auto kern) {
         kern<<<grid, 64 * G, lds, st>>>(g, tl, xv.ptr, xv.sb, xv.sc, xv.st, out, os_b, br, bi);
         return hipGetLastError();

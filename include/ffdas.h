@@ -398,7 +398,7 @@ FFDAS_API ffdas_error_t ffdas_greens(ffdas_handle_t handle, const float *srcpos,
 
 /* Opt-in kernel timing: while enabled, every kernel the library launches is bracketed by
  * hipEvents on its stream; ffdas_profile_query returns the summed duration [ms] and launch
- * count per kernel name ("das_fwd", "das_fwd_fi", "das_bwd_param", "das_bwd_param_fi",
+ * count per kernel name ("das_fwd", "das_fwd_few", "das_fwd_fi", "das_bwd_param", "das_bwd_param_fi",
  * "das_bwd_x", "das_bwd_x_plain", "das_fwd_fi_batched", "relayout_fi", "cast_rows",
  * "transpose_gout", "rank_gram", "rank_gram_reduce", "rank_jacobi", "rank_project",
  * "interp_locate", "interp_frames", "interp_eval", "greens").
