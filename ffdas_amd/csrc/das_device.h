@@ -92,6 +92,16 @@ __device__ __forceinline__ Radius radius_fast(const SplitPt &y, const SplitPt &p
     return R;
 }
 
+// |d| of R.dx, R.dy, R.dz in plain FP32.
+__device__ __forceinline__ Radius radius_plain(Radius R) {
+#pragma clang fp contract(off)
+    const float q = __builtin_fmaf(R.dx, R.dx, __builtin_fmaf(R.dy, R.dy, R.dz * R.dz));
+    R.rinv = __builtin_amdgcn_rsqf(q);
+    R.rh = q * R.rinv;
+    R.rl = 0.0f;
+    return R;
+}
+
 // The error-free transformations below (TwoSum, exact products via fmaf) rely on every
 // product and sum being rounded exactly where written, so floating-point contraction is
 // switched off inside these functions; intended fused operations are explicit fmaf calls.
@@ -100,24 +110,27 @@ __device__ __forceinline__ Radius radius_fast(const SplitPt &y, const SplitPt &p
 // the squared radius as an exact 32-bit integer plus an FP32 remainder, and one Newton
 // correction gives r = rh + rl with an error of a few 1e-8 samples over the whole range
 // of delays (instead of ~1e-4 for a single FP32 value near 2000 samples).
+//
+// BRANCH: how the wave leaves out points more than 32767 samples apart along an axis, which no
+// imaging geometry holds: it branches around the compensated form, or computes both and selects.
+// The same result.  The branch saves the clamps, but it ends a block of instructions, and where a
+// channel's step is long loads the wave waits for what it could have begun before (das_bwd_param_body).
+template <bool BRANCH = true>
 __device__ __forceinline__ Radius radius_precise(const SplitPt &y, const SplitPt &p) {
 #pragma clang fp contract(off)
     Radius R;
     const float dcx = y.cx - p.cx, dcy = y.cy - p.cy, dcz = y.cz - p.cz;   // exact integers
     const float dfx = y.fx - p.fx, dfy = y.fy - p.fy, dfz = y.fz - p.fz;   // |.| <= 1
     R.dx = dcx + dfx; R.dy = dcy + dfy; R.dz = dcz + dfz;
-    if (__builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(dcx), __builtin_fabsf(dcy)),
-                        __builtin_fabsf(dcz)) > 32767.0f) {
-        // far outside any imaging geometry: plain FP32
-        const float q = __builtin_fmaf(R.dx, R.dx, __builtin_fmaf(R.dy, R.dy, R.dz * R.dz));
-        R.rinv = __builtin_amdgcn_rsqf(q);
-        R.rh = q * R.rinv;
-        R.rl = 0.0f;
-        return R;
-    }
+    const float lim = 32767.0f;
+    const bool far = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(dcx), __builtin_fabsf(dcy)),
+                                     __builtin_fabsf(dcz)) > lim;
+    if (BRANCH && far) return radius_plain(R);
     // integer part of |d|^2, exact in 32 bits; 24-bit multiplications, which run at the full
     // rate (a 32-bit one takes four times as long)
-    const int ix = (int)dcx, iy = (int)dcy, iz = (int)dcz;
+    const int ix = (int)(BRANCH ? dcx : __builtin_amdgcn_fmed3f(dcx, -lim, lim));
+    const int iy = (int)(BRANCH ? dcy : __builtin_amdgcn_fmed3f(dcy, -lim, lim));
+    const int iz = (int)(BRANCH ? dcz : __builtin_amdgcn_fmed3f(dcz, -lim, lim));
     const uint32_t I = (uint32_t)__mul24(ix, ix) + (uint32_t)__mul24(iy, iy) +
                        (uint32_t)__mul24(iz, iz);
     // remainder 2*dc*df + df^2 per axis
@@ -136,7 +149,7 @@ __device__ __forceinline__ Radius radius_precise(const SplitPt &y, const SplitPt
     res = (res - pl) + (Il + F);
     R.rh = r0;
     R.rl = r2u < kRadiusSqMin ? 0.0f : res * (0.5f * R.rinv);
-    return R;
+    return !BRANCH && far ? radius_plain(R) : R;
 }
 
 struct Tap {
