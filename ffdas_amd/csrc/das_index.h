@@ -184,6 +184,31 @@ __host__ __device__ __forceinline__ int xcd_chunk(int b, int nb, int q) {
     return round * 8 * q + ((i + round) & 7) * q + (i >> 3);
 }
 
+// Whether sparse compounding takes chunks rather than contiguous ranges.  Shaped volumes do.  Images
+// do where their samples outgrow the caches that the XCDs share and a tap is long enough to wait for
+// them: chunks then keep the XCDs at one part of the samples, and ranges are the better while it is
+// the tiles' own rows that each L2 must hold.  record: bytes of all frames of a sample in a record
+// (0: rows in their natural order, or several problems in a launch, which go by the tiles alone);
+// samples: C * T * S; params: the parameter adjoint, which writes each slot besides, and passes over
+// the samples once in eight slots.  Chunks against ranges, 128 channels of 2000 samples:
+//   forward    256 x 256, FP32, 8 frames, 64 transmits (500 MiB), 8 slots     823 and 891 us
+//              500 x 260, FP16, 8 frames, 64 transmits (250 MiB), 8 slots     838 and 882
+//              256 x 256, FP32, 8 frames, 16 transmits (125 MiB), 8 slots     421 and 432
+//              256 x 256, FP32, 4 frames, 16 transmits (62 MiB), 8 slots      210 and 199
+//              256 x 256, BF16, 16 frames, 9 transmits (70 MiB), 2 slots      147 and 138
+//   adjoint    500 x 260, FP32, 16 frames, 64 transmits (1000 MiB), 8 slots   2.32 and 2.84 ms
+//              500 x 260, complex, 4 frames, 64 transmits (500 MiB), 8 slots  1.72 and 1.94
+//              256 x 256, FP32, 8 frames, 64 transmits (500 MiB), 16 slots    1.68 and 1.56
+//              256 x 256, FP16, 8 frames, 64 transmits (250 MiB), 8 slots     522 and 482 us
+//              256 x 256, FP16, 8 frames, 9 transmits (35 MiB), 1 slot        52 and 49
+inline bool sparse_chunks(bool shaped, int64_t tiles, int64_t record, int64_t samples, int K,
+                          bool params) {
+    if (shaped || tiles < 512) return shaped;
+    if (record == 0) return true;
+    const int64_t mib = (record * samples) >> 20;
+    return params ? mib >= 240 && (record >= 64 || (record >= 32 && K <= 8)) : mib >= 120;
+}
+
 // The order of Tiling::xcd: 0 the hardware's, 1 contiguous ranges, more: chunks of so many blocks.
 __host__ __device__ __forceinline__ int xcd_order(int xcd, int b, int nb) {
     return xcd == 0 ? b : xcd == 1 ? xcd_block(b, nb) : xcd_chunk(b, nb, xcd);

@@ -1990,7 +1990,7 @@ int frame_tile_for(int B) {
 // Sparse compounding takes chunks instead (xcd_chunk): what a tile fetches changes over the grid,
 // and with whole eighths the XCDs finished at different times (64^3 voxels of 1024 channels in
 // flat tiles: 18.7 ms in eighths, 14.2 round-robin, 13.0 in chunks of 8).  Images keep the eighths
-// below 512 tiles (8 frames, 9 transmits: 468 tiles 199 us and 211 in chunks, 648 tiles 235 and 221).
+// below 512 tiles, and above where dev::sparse_chunks says so.
 constexpr int kXcdSparse = 8;      // workgroups of a chunk
 
 bool xcd_groups() {
@@ -2011,7 +2011,8 @@ bool xcd_groups() {
 // window (Tiling::flat) is what those times give: large for few frames, whose taps are few bytes,
 // small where the lines it fetches are what it waits for.  Which volumes: dev::flat_volume; the
 // sparse ones that keep cubes keep the eighths too (24^3 voxels 164 us, in chunks 172).
-dev::Tiling make_tiling(const DasProblem &p, bool flat) {
+enum class Pass { Forward, Params, Batch };
+dev::Tiling make_tiling(const DasProblem &p, bool flat, Pass pass = Pass::Forward) {
     std::vector<int64_t> d;
     for (int64_t v : p.spatial)
         if (v > 1) d.push_back(v);
@@ -2038,7 +2039,11 @@ dev::Tiling make_tiling(const DasProblem &p, bool flat) {
         t.flat = p.sparse ? 70.0f : p.fi_frames > 0 ? 32.0f : 300.0f;
         t.tiles = (int)dev::flat_most(t.A, t.H, t.W);
     }
-    const bool chunks = p.sparse && (t.flat > 0.0f || t.tiles >= 512);
+    const int64_t record = p.fi_frames <= 0 || pass == Pass::Batch ? 0
+        : (int64_t)p.fi_frames * (int64_t)storage_bytes(p.k_storage) * (p.cplx ? 2 : 1);
+    const bool chunks = p.sparse && dev::sparse_chunks(t.flat > 0.0f, t.tiles, record,
+                                                       (int64_t)p.C * p.T * p.S, p.K,
+                                                       pass == Pass::Params);
     t.xcd = !xcd_groups() ? 0 : chunks ? kXcdSparse : 1;
     return t;
 }
@@ -2455,7 +2460,7 @@ hipError_t launch_fwd_batched_f(hipStream_t st, const std::vector<BatchMember> &
             int minC = 1 << 30;
             for (int i = 0; i < n; i++) {
                 const BatchMember &m = ms[off + i];
-                args.item[i].tl = make_tiling(m.p, true);
+                args.item[i].tl = make_tiling(m.p, true, Pass::Batch);
                 const dev::Tiling &tl = args.item[i].tl;
                 tiles += (int64_t)tl.tiles * ((m.p.B + F - 1) / F);
                 minC = std::min(minC, m.p.C);
@@ -2818,7 +2823,7 @@ ffdas_error_t launch_backward(ffdas_context &h, const DasProblem &p, const DasGe
                               const XView &xv, const void *gout, int64_t gs_b, void *gx,
                               float *gofs, float *gwt, float *gscale, void *gt, void *pws) {
     const dev::Geo g = make_geo(a, p);
-    const dev::Tiling tl = make_tiling(p, p.fi_frames > 0);
+    const dev::Tiling tl = make_tiling(p, p.fi_frames > 0, Pass::Params);
     hipStream_t st = h.stream;
     hipError_t e = hipSuccess;
 

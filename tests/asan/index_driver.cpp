@@ -99,6 +99,25 @@ static long orders() {
     return n;
 }
 
+// Sparse images go in chunks only where their samples outgrow the shared caches, in the parameter
+// adjoint only where a tap is long besides; few tiles never, shaped volumes always.
+static long shares() {
+    const int64_t few = 128 * 9 * 2000, many = 128 * 64 * 2000;
+    for (bool params : {false, true}) {
+        for (int64_t record : {16, 32, 64}) {
+            CHECK(!sparse_chunks(false, 1024, record, few / 2, 4, params));
+            CHECK(!sparse_chunks(false, 511, record, many, 4, params));
+            CHECK(sparse_chunks(true, 8, record, few, 4, params));
+        }
+        CHECK(sparse_chunks(false, 1024, 64, many, 16, params));
+        CHECK(sparse_chunks(false, 1024, 32, many, 8, params));
+        CHECK(sparse_chunks(false, 1024, 32, many, 9, params) == !params);
+        CHECK(sparse_chunks(false, 1024, 16, many, 8, params) == !params);
+        CHECK(sparse_chunks(false, 512, 0, few, 8, params));
+    }
+    return 2;
+}
+
 // Terms of every size and sign, h just below an integer among them, convert without leaving 32 bits
 // and hold h + l to 2^-31; between -1 and 0, where h has more places than its fraction, to 2^-24.
 static long terms() {
@@ -144,7 +163,8 @@ static long beyond() {
 }
 
 int main() {
-    std::printf("slots %ld, tiles %ld, volumes %ld, orders %ld, terms %ld, offsets %ld: index arithmetic "
-                "clean\n", slots(), tiles(), volumes(), orders(), terms(), beyond());
+    std::printf("slots %ld, tiles %ld, volumes %ld, orders %ld, shares %ld, terms %ld, offsets %ld: "
+                "index arithmetic clean\n", slots(), tiles(), volumes(), orders(), shares(), terms(),
+                beyond());
     return 0;
 }
