@@ -119,10 +119,16 @@ __host__ __device__ __forceinline__ int64_t flat_most(int A, int H, int W) {
 // CUs idle takes as long as one of its tiles does, and the cubes of a grid thinner than they are hold
 // fewer voxels.  Frame-inner rows, 17 x 3 x 65 voxels with depth last, 256 channels, 4 transmits:
 // forward 77 us in cubes, 132 shaped, parameter adjoint 90 and 134; turned round, from 0.71 to 1.7 of
-// the cubes' time.  Few frames, whose taps are bound by the VALU, are shaped always.  Sparse volumes need
+// the cubes' time.  Few frames, whose taps are bound by the VALU, are shaped whatever the grid.  Sparse volumes need
 // 256 cubes (24^3 voxels 158 us, shaped 164; 30^3 voxels 312 and 265).
-__host__ __device__ __forceinline__ bool flat_volume(int A, int H, int W, bool sparse, bool frame_inner) {
+// taps, channels times slots, have to be worth the look at the delays that shaping takes (4 us, and
+// 6 with more tiles than cubes fill): 40^3 voxels, 64 channels, one slot, 4 frames 37 us shaped and
+// 31 in cubes, one frame 37 and 26; at 512 taps from 0.81 to 1.03 of the cubes' time, at 1024 channels
+// and 8 slots 0.59 to 0.88.  Few frames gain later, 24^3 voxels 0.87 there and 1.09 at 256 x 4.
+__host__ __device__ __forceinline__ bool flat_volume(int A, int H, int W, bool sparse, bool frame_inner,
+                                                     int64_t taps = INT64_MAX) {
     const int64_t cubes = (int64_t)((A + 3) / 4) * ((H + 3) / 4) * ((W + 3) / 4);
+    if (taps < (sparse ? (frame_inner ? 128 : 256) : frame_inner ? 512 : 8192)) return false;
     if (sparse) return cubes >= 256;
     return !frame_inner || cubes >= 512 || (A >= 4 && H >= 4 && W >= 4);
 }

@@ -2035,7 +2035,7 @@ dev::Tiling make_tiling(const DasProblem &p, bool flat, Pass pass = Pass::Forwar
     t.ntw = (t.W + t.tw - 1) / t.tw;
     t.tiles = t.nta * t.nth * t.ntw;
     if (flat && d.size() >= 3 && p.C > 0 && p.K > 0 &&
-        dev::flat_volume(t.A, t.H, t.W, p.sparse, p.fi_frames > 0)) {
+        dev::flat_volume(t.A, t.H, t.W, p.sparse, p.fi_frames > 0, (int64_t)p.C * p.K)) {
         t.flat = p.sparse ? 70.0f : p.fi_frames > 0 ? 32.0f : 300.0f;
         t.tiles = (int)dev::flat_most(t.A, t.H, t.W);
     }

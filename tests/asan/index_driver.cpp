@@ -79,6 +79,13 @@ static long volumes() {
             CHECK(!flat_volume(24, 24, swap ? 24 : thin, true, true));
         }
     CHECK(flat_volume(8, 8, 8, false, true) && flat_volume(30, 30, 30, true, true));
+    // few taps are not worth the look
+    for (bool sparse : {false, true})
+        for (bool frame_inner : {false, true}) {
+            CHECK(!flat_volume(64, 64, 64, sparse, frame_inner, 64));
+            CHECK(flat_volume(64, 64, 64, sparse, frame_inner, 1024) == (sparse || frame_inner));
+            CHECK(flat_volume(64, 64, 64, sparse, frame_inner, 1024 * 8));
+        }
     return 4;
 }
 
