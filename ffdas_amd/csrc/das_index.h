@@ -124,11 +124,12 @@ __host__ __device__ __forceinline__ int64_t flat_most(int A, int H, int W) {
 // taps, channels times slots, have to be worth the look at the delays that shaping takes (4 us, and
 // 6 with more tiles than cubes fill): 40^3 voxels, 64 channels, one slot, 4 frames 37 us shaped and
 // 31 in cubes, one frame 37 and 26; at 512 taps from 0.81 to 1.03 of the cubes' time, at 1024 channels
-// and 8 slots 0.59 to 0.88.  Few frames gain later, 24^3 voxels 0.87 there and 1.09 at 256 x 4.
+// and 8 slots 0.59 to 0.88.  Few frames gain later, 24^3 voxels 0.87 there and 1.09 at 256 x 4;
+// sparse volumes sooner: 64^3 voxels, 64 channels, 2 slots, 2 complex frames 123 us and 188.
 __host__ __device__ __forceinline__ bool flat_volume(int A, int H, int W, bool sparse, bool frame_inner,
                                                      int64_t taps = INT64_MAX) {
     const int64_t cubes = (int64_t)((A + 3) / 4) * ((H + 3) / 4) * ((W + 3) / 4);
-    if (taps < (sparse ? (frame_inner ? 128 : 256) : frame_inner ? 512 : 8192)) return false;
+    if (taps < (sparse ? 64 : frame_inner ? 512 : 8192)) return false;
     if (sparse) return cubes >= 256;
     return !frame_inner || cubes >= 512 || (A >= 4 && H >= 4 && W >= 4);
 }
@@ -188,6 +189,37 @@ __host__ __device__ __forceinline__ int xcd_chunk(int b, int nb, int q) {
     const int round = b / (8 * q), i = b - round * 8 * q;
     if ((round + 1) * 8 * q > nb) return b;
     return round * 8 * q + ((i + round) & 7) * q + (i >> 3);
+}
+
+// Whether the forward of one to three frames goes to das_fwd_few_kernel: it shares a tile's channels
+// out over waves and its taps cost less, and pays for that a setup a tile and a term a channel.  tiles
+// are those of das_fwd_kernel, which has one wave a tile: below a thousand it cannot fill the chip.
+// Few against that kernel, from 1 slot up where it starts to pay:
+//   512 x 512, FP32, 1 frame, 64 channels          1 slot 1.23, 2: 1.08, 3: 0.98, 4: 0.78, 8: 0.45
+//   96^3, FP32, 2 frames, 64 channels              1.33, 1.08, 1.06, 0.95, 0.93
+//   1024 x 512, complex FP32, 1 frame, 256         1.27, 1.01, 0.96, 0.86, 0.78
+//   400 x 256, FP32, 1 frame, 16 channels          1.47, 1.29, 1.07, 1.01, 0.78; 256 channels below 1
+//   96^3, FP16, 2 frames, 64 channels              1.26, 1.11, 1.16, 1.14, 1.22 (16 slots 1.21)
+//   64^3, FP16, 2 frames, sparse, 64 channels      1.84, 2.00 and (4) 2.03, (8) 2.05; 1000 tiles 0.93 to 1.07
+//   64^3, FP32, 1 frame, sparse, 64 channels       1.61, 1.20 and (4) 0.90
+//   512 x 512, FP32, 2 frames, sparse, 64 channels 1.28, 1.21 and (4) 1.14, (8) 1.07
+inline bool few_pays(int64_t tiles, bool volume, int C, int K, int B, bool cplx, bool narrow,
+                     bool sparse) {
+    const bool words = !cplx && narrow;        // 16-bit samples, two loads a tap
+    const bool wide = tiles >= 3000;
+    if (tiles < 1000) return true;
+    if (words && B >= 2 && volume && (wide || C <= 32)) return false;
+    if (C <= 32) {                             // few channels to share out
+        if (sparse && (words || (volume ? !wide : tiles >= 1500))) return false;
+        return K >= (volume || tiles >= 1500 ? 4 : 2);
+    }
+    if (sparse && words) return tiles < 1500;
+    if (!wide) return true;
+    if (sparse && !volume && B >= 2) return false;
+    if (cplx) return K >= 2;
+    if (sparse) return K >= (B == 1 ? 3 : 2);
+    if (words && B >= 2) return K >= 4;
+    return K >= (B >= 2 && tiles >= 8000 ? 4 : 3);
 }
 
 // Whether sparse compounding takes chunks rather than contiguous ranges.  Shaped volumes do.  Images

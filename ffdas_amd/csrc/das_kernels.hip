@@ -2661,7 +2661,12 @@ ffdas_error_t launch_forward_batched(ffdas_context &h, const std::vector<BatchMe
 ffdas_error_t launch_forward(ffdas_context &h, const DasProblem &p, const DasGeomArgs &a,
                              const XView &xv, void *out, double beta_re, double beta_im) {
     const dev::Geo g = make_geo(a, p);
-    const bool few = p.fi_frames <= 0 && few_frames_ok(p, xv);
+    bool few = p.fi_frames <= 0 && few_frames_ok(p, xv);
+    if (few) {
+        const dev::Tiling plain = make_tiling(p, false);
+        few = dev::few_pays(plain.tiles, plain.ta > 1, p.C, p.K, p.B, p.cplx,
+                            storage_bytes(p.k_storage) == 2, p.sparse);
+    }
     const dev::Tiling tl = make_tiling(p, p.fi_frames > 0 || few);
     hipError_t e = hipSuccess;
     hipStream_t st = h.stream;

@@ -82,7 +82,7 @@ static long volumes() {
     // few taps are not worth the look
     for (bool sparse : {false, true})
         for (bool frame_inner : {false, true}) {
-            CHECK(!flat_volume(64, 64, 64, sparse, frame_inner, 64));
+            CHECK(!flat_volume(64, 64, 64, sparse, frame_inner, 63));
             CHECK(flat_volume(64, 64, 64, sparse, frame_inner, 1024) == (sparse || frame_inner));
             CHECK(flat_volume(64, 64, 64, sparse, frame_inner, 1024 * 8));
         }
@@ -122,6 +122,26 @@ static long shares() {
         CHECK(sparse_chunks(false, 1024, 16, many, 8, params) == !params);
         CHECK(sparse_chunks(false, 512, 0, few, 8, params));
     }
+    return 2;
+}
+
+// One to three frames stay with das_fwd_few_kernel where the tiles are few or the slots many.
+static long routes() {
+    for (bool volume : {false, true})
+        for (int B : {1, 2, 3})
+            for (bool cplx : {false, true})
+                for (bool narrow : {false, true})
+                    for (bool sparse : {false, true}) {
+                        const bool words = narrow && !cplx;
+                        const bool wide = words && B >= 2 && volume;
+                        CHECK(few_pays(999, volume, 16, 1, B, cplx, narrow, sparse));
+                        CHECK(few_pays(1499, volume, 64, 1, B, cplx, narrow, sparse));
+                        CHECK(few_pays(2999, volume, 64, 1, B, cplx, narrow, sparse) == !(sparse && words));
+                        CHECK(!few_pays(1000, volume, 32, 1, B, cplx, narrow, sparse));
+                        CHECK(!few_pays(3000, volume, 64, 1, B, cplx, narrow, sparse));
+                        CHECK(few_pays(100000, volume, 64, 4, B, cplx, narrow, sparse) ==
+                              !(wide || (sparse && (words || (!volume && B >= 2)))));
+                    }
     return 2;
 }
 
@@ -170,8 +190,8 @@ static long beyond() {
 }
 
 int main() {
-    std::printf("slots %ld, tiles %ld, volumes %ld, orders %ld, shares %ld, terms %ld, offsets %ld: "
-                "index arithmetic clean\n", slots(), tiles(), volumes(), orders(), shares(), terms(),
-                beyond());
+    std::printf("slots %ld, tiles %ld, volumes %ld, orders %ld, shares %ld, routes %ld, terms %ld, offsets %ld: "
+                "index arithmetic clean\n", slots(), tiles(), volumes(), orders(), shares(), routes(),
+                terms(), beyond());
     return 0;
 }
