@@ -294,6 +294,10 @@ __global__ __launch_bounds__(256, NT == 1 ? 5 : 3) void greens_mfma_kernel(const
 // targets the MFMA is the faster from one frequency on (2 events 45 and 30 us; 512 frequencies 1.79 and 1.5 ms).
 // With few sources the writes weigh more, and so does a second chunk of frequencies: 16 sources to 2^19
 // targets, 3 events, 12 frequencies 144 and 118 us.
+// Two events besides where the VALU kernel's workgroups, three a CU, fill the rounds they take: for a
+// quarter of the columns the MFMA tile then costs more.  11808 targets, 159 sources, 512 frequencies
+// (1504 workgroups, 0.98 of two rounds) 626 and 712 us, 32768 targets, 384 frequencies (four rounds) 1.16
+// and 1.42 ms; at 0.65 of the rounds (16000 targets, 256 frequencies) 510 and 481.
 bool on_valu(int B, int nsrc, int nfreq, int ndst) {
     if (B == 1) return true;
     if (B > 4) return false;
@@ -308,7 +312,10 @@ bool on_valu(int B, int nsrc, int nfreq, int ndst) {
     if (many && waves >= 8192.0 && B > 2) most += 1.0;
     if (many && waves >= 16384.0 && (B == 3 || (B == 2 && nfreq <= 64))) most += 1.0;
     if (B == 3 && chunks > 1) most -= 1.0;
-    return (double)nfreq / chunks <= most;
+    if ((double)nfreq / chunks <= most) return true;
+    const int64_t groups = (int64_t)((ndst + 255) / 256) * chunks, round = 768;
+    const int64_t rounds = (groups + round - 1) / round;
+    return B == 2 && many && (double)groups >= 0.87 * (double)(rounds * round);
 }
 
 template <typename XT>
